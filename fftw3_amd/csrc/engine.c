@@ -2140,6 +2140,18 @@ static int plan_split(ctx *c, const fk_problem *pb)
     return c->err ? -1 : 0;
 }
 
+/* divisors of a pass's line and table indices (fk_args.qm); 64-bit division
+   in the kernel where an index may not fit 31 bits */
+static void fill_magic(fk_args *a)
+{
+    memset(a->qm, 0, sizeof(a->qm));
+    if (a->nlines < (1LL << 31) && a->nb[0] > 0 && a->nb[1] > 0) {
+        fk_magic((unsigned long long)a->nb[0], &a->qm[0], &a->qs[0]);
+        fk_magic((unsigned long long)a->nb[1], &a->qm[1], &a->qs[1]);
+    }
+    if (a->tb > 0 && a->tN < (1LL << 31)) fk_magic((unsigned long long)a->tb, &a->qm[2], &a->qs[2]);
+}
+
 static fk_plan *build_plan(const fk_problem *pb0, hipStream_t st, const int *choice, int nchoice,
                            ctx *cout)
 {
@@ -2257,6 +2269,8 @@ static fk_plan *build_plan(const fk_problem *pb0, hipStream_t st, const int *cho
         }
     }
     if (c.err) goto fail;
+    for (i = 0; i < P->npass; ++i)
+        if (P->pass[i].type == FK_PASS_STOCKHAM) fill_magic(&P->pass[i].a);
 done_ok:
     for (i = 0; i < P->nscratch; ++i) {
         if (P->scratch_bytes[i]) {

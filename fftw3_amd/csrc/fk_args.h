@@ -37,7 +37,7 @@ enum {
 #define FK_SWAP_OUT  2u   /* swap re/im on store (backward transform) */
 #define FK_TW_OUT    4u   /* multiply output bin k of line with batch index
                              i0 by W_N^(k*i0) (four-step twiddle) */
-#define FK_SCALE     8u   /* multiply output by scale */
+#define FK_SCALE     8u   /* multiply output by scale (element-wise passes) */
 #define FK_REAL_UNIT 16u  /* R2C: real input stride is 1 / C2R: output stride 1 */
 #define FK_REAL_QUAD 32u  /* FP32 real input stride 1, lines 16-byte aligned: the
                              reordered loads of REDFT10 / RODFT10 read quads */
@@ -74,13 +74,27 @@ typedef struct {
        FK_IO_BLUE: chirp c_m (m < nvalid), then FFT_L(conj chirp)/L */
     const void *aux, *aux2;
     long long nvalid;         /* BLUE: logical length n; else unused */
-    double scale;
     unsigned flags;
     unsigned xcd_remap;       /* nonzero: spread tiles XCD-contiguously */
     unsigned rmode;           /* FK_RM_*: fused real-to-real kind */
     unsigned pad_;
     const void *rtw;          /* FK_RM_DCT2/3, FK_RM_DST2/3: exp(-i pi m / 4n), m < 2n */
+    /* division by multiplication, q / d = (2 q * qm >> 32) >> qs for q < 2^31:
+       0 and 1 divide by nb[0] and nb[1] (qm[0] = 0: nlines >= 2^31, 64-bit
+       division), 2 by tb (qm[2] = 0: tN >= 2^31) */
+    unsigned qm[3], qs[3];
 } fk_args;
+
+/* multiplier and shift of fk_args.qm / qs for a divisor 1 <= d < 2^31:
+   s = ceil(log2 d), m = ceil(2^(31+s) / d) < 2^32, so m d = 2^(31+s) + e with
+   0 <= e < d <= 2^s and floor(q m / 2^(31+s)) = floor(q / d) for q < 2^31 */
+static inline void fk_magic(unsigned long long d, unsigned *m, unsigned *s)
+{
+    unsigned k = 0;
+    while ((1ull << k) < d) ++k;
+    *m = (unsigned)(((1ull << (31 + k)) + d - 1) / d);
+    *s = k;
+}
 
 typedef struct {
     int prec;          /* 0 = double, 1 = float */

@@ -266,27 +266,54 @@ __device__ __forceinline__ cx<R> tw2(const fk_args &a, long long e)
 __device__ __forceinline__ cx<double> tw2d(const fk_args &a, long long e)
 {
     /* W_N^e from the two-level FP64 table, W_N^e = lo[e % b] * hi[e / b].
-       Four-step exponents are e = k*i0 < N; the reduction below only runs
-       for exponents outside [0, N). */
-    const long long N = a.tN, b = a.tb;
-    if (e < 0 || e >= N) {
-        e %= N;
-        if (e < 0) e += N;
+       The exponents are k*i0 of a four-step split, 0 <= e < N (output k < n1
+       of line i0 < n2, n1 n2 = N), and n1*p of the cross-row kernels. */
+    const long long b = a.tb;
+    if (a.qm[2]) {                             /* N < 2^31: 32-bit split */
+        const unsigned ue = (unsigned)e, q = __umulhi(2 * ue, a.qm[2]) >> a.qs[2];
+        const unsigned l = ue - q * (unsigned)b;
+        const double2 lo = reinterpret_cast<const double2 *>(a.tlo)[l];
+        const double2 hi = reinterpret_cast<const double2 *>(a.thi)[q];
+        return mk(lo.x * hi.x - lo.y * hi.y, lo.x * hi.y + lo.y * hi.x);
     }
-    long long il, ih;
-    if ((b & (b - 1)) == 0) {                  /* power-of-two split */
-        il = e & (b - 1);
-        ih = e >> __builtin_ctzll((unsigned long long)b);
-    } else if (N <= 0x7fffffffLL) {            /* 32-bit division */
-        const unsigned ue = (unsigned)e, ub = (unsigned)b, q = ue / ub;
-        ih = q;
-        il = ue - q * ub;
-    } else {
-        ih = e / b;
-        il = e - ih * b;
-    }
+    const long long ih = e / b, il = e - ih * b;
     const double *lo = a.tlo + 2 * il, *hi = a.thi + 2 * ih;
     return mk(lo[0] * hi[0] - lo[1] * hi[1], lo[0] * hi[1] + lo[1] * hi[0]);
+}
+
+/* batch indices of line q of a pass (0 <= q < nlines) */
+struct LineIx {
+    long long i0, i1, i2;
+};
+__device__ __forceinline__ LineIx line_ix(const fk_args &a, long long q)
+{
+    LineIx r;
+    if (a.qm[0]) {
+        const unsigned u = (unsigned)q;
+        const unsigned q1 = __umulhi(2 * u, a.qm[0]) >> a.qs[0];
+        const unsigned q2 = __umulhi(2 * q1, a.qm[1]) >> a.qs[1];
+        r.i0 = u - q1 * (unsigned)a.nb[0];
+        r.i1 = q1 - q2 * (unsigned)a.nb[1];
+        r.i2 = q2;
+    } else {
+        r.i0 = q % a.nb[0];
+        q /= a.nb[0];
+        r.i1 = q % a.nb[1];
+        r.i2 = q / a.nb[1];
+    }
+    return r;
+}
+
+/* input and output offset of a line, in elements of its array */
+__device__ __forceinline__ void line_off(const fk_args &a, const LineIx &x, long long &bin,
+                                         long long &bout)
+{
+    bin = x.i0 * a.ids[0];
+    bout = x.i0 * a.ods[0];
+    if (a.nb[1] != 1 || a.nb[2] != 1) {
+        bin += x.i1 * a.ids[1] + x.i2 * a.ids[2];
+        bout += x.i1 * a.ods[1] + x.i2 * a.ods[2];
+    }
 }
 
 } // namespace fk

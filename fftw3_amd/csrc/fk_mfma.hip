@@ -100,15 +100,14 @@ __global__ void __launch_bounds__(NT) k_mfma(fk_args a)
     if (tid < NL) {
         const long long line = tile * NL + tid;
         const bool act = line < a.nlines;
-        long long q = act ? line : 0;
-        const long long i0 = q % a.nb[0];
-        q /= a.nb[0];
-        const long long i1 = q % a.nb[1], i2 = q / a.nb[1];
+        const LineIx lx = line_ix(a, act ? line : 0);
+        long long bin, bout;
+        line_off(a, lx, bin, bout);
         /* offsets may be negative (negative strides): inactive lines are
            marked with the one value no offset takes */
-        lin[tid] = act ? i0 * a.ids[0] + i1 * a.ids[1] + i2 * a.ids[2] : NONE;
-        lout[tid] = act ? i0 * a.ods[0] + i1 * a.ods[1] + i2 * a.ods[2] : NONE;
-        li0[tid] = i0;
+        lin[tid] = act ? bin : NONE;
+        lout[tid] = act ? bout : NONE;
+        li0[tid] = lx.i0;
     }
     __syncthreads();
     const cx<float> *in = reinterpret_cast<const cx<float> *>(a.in);
@@ -215,7 +214,7 @@ __global__ void __launch_bounds__(NT) k_mfma(fk_args a)
     }
 
     /* store the tile with the output post-op */
-    const bool twout = a.flags & FK_TW_OUT, scl = a.flags & FK_SCALE;
+    const bool twout = a.flags & FK_TW_OUT;
     if (a.os == 1) {
         for (int e = tid; e < NL * L; e += NT) {
             const int lt = e / L, k = e % L;
@@ -223,7 +222,6 @@ __global__ void __launch_bounds__(NT) k_mfma(fk_args a)
             if (base == NONE) continue;
             cx<float> y = lds[idx(lt, k)];
             if (twout) y = mul(y, tw2<float>(a, (long long)k * li0[lt]));
-            if (scl) { y.x *= (float)a.scale; y.y *= (float)a.scale; }
             out[base + k] = swo ? swp(y) : y;
         }
     } else {
@@ -244,7 +242,6 @@ __global__ void __launch_bounds__(NT) k_mfma(fk_args a)
                 wcur = (it % 16 == 0) ? tw2d(a, (long long)k * i0) : mul(wcur, wstep);
                 y = mul(y, mk((float)wcur.x, (float)wcur.y));
             }
-            if (scl) { y.x *= (float)a.scale; y.y *= (float)a.scale; }
             out[base + (long long)k * a.os] = swo ? swp(y) : y;
         }
     }

@@ -110,15 +110,83 @@ struct SyncWave {
     }
 };
 
+/* What happens to a butterfly's registers after its loads (first stage) or
+   before its stores (last stage). */
+struct NoOp {
+    template <int N, typename R>
+    __device__ __forceinline__ void run(int, cx<R> *) const
+    {
+    }
+};
+
+/* Swap re and im of N values when the pass runs backward.  The empty asm
+   keeps the swap a branch that every wave takes or skips as a whole: as
+   selects it would cost the forward direction two instructions a value. */
+template <int N, typename R>
+__device__ __forceinline__ void swap_if(bool sw, cx<R> *v)
+{
+    if (sw) {
+        asm volatile("");
+        sfor<0, N>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            v[r] = swp(v[r]);
+        });
+    }
+}
+struct SwapOp {
+    bool sw;
+    template <int N, typename R>
+    __device__ __forceinline__ void run(int, cx<R> *v) const
+    {
+        swap_if<N>(sw, v);
+    }
+};
+
+/* Output post-op of the plain passes: four-step twiddle, then the swap.
+   The twiddle of output k = b + r*Ns (last stage, r = 0..N-1) of a line with
+   batch index i0 is W_N^(k*i0): looked up in the FP64 table every ANCH
+   outputs and stepped by W_N^(Ns*i0) in FP64 in between, so a thread gathers
+   2 table entries per ANCH outputs instead of 2 per output.  FP64 data
+   re-anchors every 4 (at most 3 products from a table value); FP32 data once
+   per butterfly (at most 15 FP64 products, ~1e-15, far below FP32 rounding). */
+template <int NS>
+struct PlainOut {
+    const fk_args &a;
+    bool tw, sw;
+    long long i0;
+    cx<double> step;
+    __device__ __forceinline__ PlainOut(const fk_args &a_, unsigned fl, long long i0_)
+        : a(a_), tw(fl & FK_TW_OUT), sw(fl & FK_SWAP_OUT), i0(i0_), step(mk(1.0, 0.0))
+    {
+        if (tw) step = tw2d(a, (long long)NS * i0);
+    }
+    template <int N, typename R>
+    __device__ __forceinline__ void run(int b, cx<R> *v) const
+    {
+        if (tw) {
+            constexpr int ANCH = sizeof(R) == 8 ? 4 : 16;
+            cx<double> cur = mk(1.0, 0.0);
+            sfor<0, N>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                if constexpr (r % ANCH == 0) cur = tw2d(a, (long long)(b + r * NS) * i0);
+                else cur = mul(cur, step);
+                v[r] = mul(v[r], mk((R)cur.x, (R)cur.y));
+            });
+        }
+        swap_if<N>(sw, v);
+    }
+};
+
 /*
  * One Stockham stage.  LoadF(j) -> cx<R> and StoreF(k, cx<R>) abstract the
  * data source and sink; IN_LDS/OUT_LDS say whether they touch LDS, which
- * decides the barriers.
+ * decides the barriers.  pre / fin run on a butterfly's registers after the
+ * loads / before the stores.
  */
 template <typename R, class RL, int S, int L, int TPL, bool IN_LDS, bool OUT_LDS,
-          class SY = SyncAll, class LoadF, class StoreF>
+          class SY = SyncAll, class LoadF, class StoreF, class PreF, class FinF>
 __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
-                                      LoadF &&ld, StoreF &&st)
+                                      LoadF &&ld, StoreF &&st, const PreF &pre, const FinF &fin)
 {
     constexpr int Rs = RL::r[S];
     constexpr int Ns = RL::ns(S);
@@ -150,8 +218,10 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
                     v[i][r] = mul(v[i][r], w[r - 1]);
                 });
             }
+            pre.template run<Rs>(b, v[i]);
             Dft<R, Rs, 1>::run(v[i]);
             const int base = (b - k) * Rs + k;
+            fin.template run<Rs>(base, v[i]);
             /* stage 0 (Ns = 1) writes Rs consecutive outputs from b*Rs */
             sfor<0, Rs>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
@@ -162,37 +232,40 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
     if constexpr (OUT_LDS) SY::sync();
 }
 
-/* Runs stages [S, RL::n) ; stage S loads with `first`, the last stage stores
-   with `last`, everything between goes through LDS. */
+/* Runs stages [S, RL::n) ; stage S loads with `first` (then `pre`), the last
+   stage stores with `last` (after `fin`), everything between goes through
+   LDS. */
 template <typename R, class RL, int S, int L, int TPL, bool FIRST_LDS,
-          bool LAST_LDS, class SY = SyncAll, class LdsF, class FirstF, class LastF>
+          bool LAST_LDS, class SY = SyncAll, class LdsF, class FirstF, class LastF,
+          class PreF = NoOp, class FinF = NoOp>
 __device__ __forceinline__ void run_stages(int u, const cx<R> *tw, LdsF &&lds,
-                                           FirstF &&first, LastF &&last)
+                                           FirstF &&first, LastF &&last,
+                                           const PreF &pre = PreF(), const FinF &fin = FinF())
 {
     constexpr int n = RL::n;
     auto lds_ld = [&](auto j) { return lds(j); };
     auto lds_st = [&](auto k, cx<R> v) { lds(k) = v; };
     if constexpr (S == 0 && n == 1) {
-        stage<R, RL, 0, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, first, last);
+        stage<R, RL, 0, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, first, last, pre, fin);
     } else if constexpr (S == 0) {
-        stage<R, RL, 0, L, TPL, FIRST_LDS, true, SY>(u, tw, first, lds_st);
-        run_stages<R, RL, 1, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, lds, first, last);
+        stage<R, RL, 0, L, TPL, FIRST_LDS, true, SY>(u, tw, first, lds_st, pre, NoOp());
+        run_stages<R, RL, 1, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, lds, first, last, NoOp(), fin);
     } else if constexpr (S == n - 1) {
-        stage<R, RL, S, L, TPL, true, LAST_LDS, SY>(u, tw, lds_ld, last);
+        stage<R, RL, S, L, TPL, true, LAST_LDS, SY>(u, tw, lds_ld, last, NoOp(), fin);
     } else {
-        stage<R, RL, S, L, TPL, true, true, SY>(u, tw, lds_ld, lds_st);
-        run_stages<R, RL, S + 1, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, lds, first, last);
+        stage<R, RL, S, L, TPL, true, true, SY>(u, tw, lds_ld, lds_st, NoOp(), NoOp());
+        run_stages<R, RL, S + 1, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, lds, first, last, NoOp(), fin);
     }
 }
 
 __device__ __forceinline__ long long remap_tile(unsigned xcd)
 {
-    long long w = blockIdx.x;
+    const unsigned w = blockIdx.x;
     if (!xcd) return w;
     /* workgroups are dispatched round-robin over 8 XCDs; give each XCD a
        contiguous run of tiles so neighbouring tiles share its L2 */
-    long long nwg = gridDim.x, per = nwg / 8, rem = nwg % 8;
-    long long x = w % 8, i = w / 8;
+    const unsigned nwg = gridDim.x, per = nwg / 8, rem = nwg % 8;
+    const unsigned x = w % 8, i = w / 8;
     return x * per + (x < rem ? x : rem) + i;
 }
 
@@ -218,53 +291,26 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
 
     const int tid = threadIdx.x;
     const bool real = (NT == NR) || tid < NR;
-    const int lt = !real ? 0 : (MODE == FK_ROW) ? tid / TPL : tid % NL;
+    /* row mapping with whole waves per line: the line, and all that follows
+       from it, is computed once per wave on the scalar unit */
+    constexpr bool UNI = MODE == FK_ROW && TPL % 64 == 0;
+    const int lt_ = !real ? 0 : (MODE == FK_ROW) ? tid / TPL : tid % NL;
+    const int lt = UNI ? __builtin_amdgcn_readfirstlane(lt_) : lt_;
     const int u = !real ? (tid - NR) % TPL : (MODE == FK_ROW) ? tid % TPL : tid / NL;
     const long long line = tile * NL + lt;
     const bool act = real && line < a.nlines;
 
-    long long i0 = 0, i1 = 0, i2 = 0;
-    {
-        long long q = act ? line : 0;
-        i0 = q % a.nb[0];
-        q /= a.nb[0];
-        i1 = q % a.nb[1];
-        i2 = q / a.nb[1];
-    }
-    const long long bin = i0 * a.ids[0] + i1 * a.ids[1] + i2 * a.ids[2];
-    const long long bout = i0 * a.ods[0] + i1 * a.ods[1] + i2 * a.ods[2];
+    /* inactive lanes take line 0 (in bounds) */
+    const LineIx lx = line_ix(a, act ? line : 0);
+    const long long i0 = lx.i0;
+    long long bin, bout;
+    line_off(a, lx, bin, bout);
     const cx<R> *tw = reinterpret_cast<const cx<R> *>(a.tw);
     const unsigned fl = a.flags;
     const bool swi = fl & FK_SWAP_IN, swo = fl & FK_SWAP_OUT;
-    /* output scale: multiplying by 1 when unscaled is exact and costs less
-       than selecting between scaled and unscaled values */
-    const R sc = (fl & FK_SCALE) ? (R)a.scale : (R)1;
-
     auto lds_at = [&](auto j) -> cx<R> & {
         if constexpr (NT == NR) return lds[G::idx(lt, j)];
         else return real ? lds[G::idx(lt, j)] : trash[tid & 63];
-    };
-
-    /* output post-op: twiddle, scale, swap.  The four-step twiddle of
-       output k = b + r*Ns (last stage, r = 0..R-1 stored in order) is
-       W_N^(k*i0): looked up from the FP64 table every ANCH outputs and
-       stepped by W_N^(Ns*i0) in FP64 in between, so a thread gathers 2
-       table entries per ANCH outputs instead of 2 per output.  FP64 data
-       re-anchors every 4 (at most 3 products from a table value); FP32
-       data once per butterfly (at most 15 FP64 products, ~1e-15, far below
-       FP32 rounding). */
-    constexpr int NS_LAST = RL::ns(RL::n - 1);
-    constexpr int ANCH = sizeof(R) == 8 ? 4 : 16;
-    cx<double> tw_cur = mk(1.0, 0.0), tw_step = mk(1.0, 0.0);
-    if (fl & FK_TW_OUT) tw_step = tw2d(a, (long long)NS_LAST * i0);
-    auto post = [&](int k, cx<R> v) -> cx<R> {
-        if (fl & FK_TW_OUT) {
-            if ((k / NS_LAST) % ANCH == 0) tw_cur = tw2d(a, (long long)k * i0);
-            else tw_cur = mul(tw_cur, tw_step);
-            v = mul(v, mk((R)tw_cur.x, (R)tw_cur.y));
-        }
-        v.x *= sc; v.y *= sc;
-        return swo ? swp(v) : v;
     };
 
     if constexpr (IO == FK_IO_PLAIN || IO == FK_IO_TOUT) {
@@ -275,23 +321,23 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         const long long is = a.is, os = a.os;
         const cx<R> *inu = reinterpret_cast<const cx<R> *>(a.in) + bin + u * is;
         cx<R> *out = reinterpret_cast<cx<R> *>(a.out);
-        auto gld = [&](int j) -> cx<R> {
-            cx<R> v = inu[(long long)(j - u) * is];
-            return swi ? swp(v) : v;
-        };
+        auto gld = [&](int j) -> cx<R> { return inu[(long long)(j - u) * is]; };
         if constexpr (IO == FK_IO_PLAIN) {
             cx<R> *outu = out + bout + u * os;
             auto gst = [&](int k, cx<R> v) {
-                if (act) outu[(long long)(k - u) * os] = post(k, v);
+                if (act) outu[(long long)(k - u) * os] = v;
             };
-            run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst);
+            const PlainOut<RL::ns(RL::n - 1)> fin(a, fl, i0);
+            run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst, SwapOp{swi},
+                                                           fin);
         } else {
             auto lst = [&](auto k, cx<R> v) { lds_at(k) = v; };
             /* output offsets may be negative (negative strides): inactive
                lines are marked with the one value no offset takes */
             constexpr long long NONE = -0x7fffffffffffffffLL - 1; /* INT64_MIN */
             if (u == 0 && real) lbase[lt] = act ? bout : NONE;
-            run_stages<R, RL, 0, L, TPL, false, true, SY>(u, tw, lds_at, gld, lst);
+            run_stages<R, RL, 0, L, TPL, false, true, SY>(u, tw, lds_at, gld, lst, SwapOp{swi},
+                                                          SwapOp{swo});
             /* the store below reads every line of the tile */
             if constexpr (!std::is_same<SY, SyncAll>::value) __syncthreads();
             /* lines-fastest store: consecutive threads write consecutive
@@ -299,11 +345,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             for (int e = tid; e < NL * L; e += NT) {
                 const int l2 = e % NL, k = e / NL;
                 const long long ob = lbase[l2];
-                if (ob != NONE) {
-                    cx<R> v = lds[G::idx(l2, k)];
-                    v.x *= sc; v.y *= sc;
-                    out[ob + k * a.os] = swo ? swp(v) : v;
-                }
+                if (ob != NONE) out[ob + k * a.os] = lds[G::idx(l2, k)];
             }
         }
     } else if constexpr (IO == FK_IO_R2C_FULL) {
@@ -315,10 +357,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             return act ? mk(inr[(long long)j * a.is], (R)0) : mk((R)0, (R)0);
         };
         auto gst = [&](int k, cx<R> v) {
-            if (act && 2 * k <= L) {
-                v.x *= sc; v.y *= sc;
-                out[bout + (long long)k * a.os] = v;
-            }
+            if (act && 2 * k <= L) out[bout + (long long)k * a.os] = v;
         };
         run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst);
     } else if constexpr (IO == FK_IO_C2R_FULL) {
@@ -340,10 +379,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             return swp(v);
         };
         auto gst = [&](int k, cx<R> v) {
-            if (!act) return;
-            R y = v.y;
-            y *= sc;
-            outr[(long long)k * a.os] = y;
+            if (act) outr[(long long)k * a.os] = v.y;
         };
         run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst);
     } else if constexpr (IO == FK_IO_DCT4) {
@@ -365,8 +401,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         auto gst = [&](int p, cx<R> v) {
             if (!act) return;
             const cx<R> c = mul(v, rt[4 * p]);
-            R ye = (R)2 * c.x, yo = (R)-2 * c.y;
-            ye *= sc; yo *= sc;
+            const R ye = (R)2 * c.x, yo = (R)-2 * c.y;
             outr[(2LL * p) * a.os] = ye;
             outr[(N2 - 1 - 2LL * p) * a.os] = sn ? -yo : yo;
         };
@@ -447,7 +482,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
            (n1 = the tile's line-group index, uniform over the workgroup) */
         cx<R> wp[XR ? NL : 1];
         if constexpr (XR) {
-            const long long n1 = tile % a.nb[1];
+            const long long n1 = line_ix(a, tile * NL).i1;
             sfor<0, NL>([&](auto pc) {
                 constexpr int pp = decltype(pc)::value;
                 wp[pp] = pp == 0 ? mk((R)1, (R)0) : tw2<R>(a, n1 * pp);
@@ -518,10 +553,8 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                     /* X[k] = E + W O; X[L-k] = conj(E - W O), written as the
                        form of bin L-k on its own (E' = conj E, O' = conj O,
                        W' = -conj W) so that both round as that form does */
-                    cx<R> X = mk(er + orr * wx - oi * wy, ei + orr * wy + oi * wx);
-                    cx<R> Y = mk(er + orr * (-wx) - (-oi) * wy, (-ei) + orr * wy + (-oi) * (-wx));
-                    X.x *= sc; X.y *= sc;
-                    Y.x *= sc; Y.y *= sc;
+                    const cx<R> X = mk(er + orr * wx - oi * wy, ei + orr * wy + oi * wx);
+                    const cx<R> Y = mk(er + orr * (-wx) - (-oi) * wy, (-ei) + orr * wy + (-oi) * (-wx));
                     if constexpr (XR) {
                         xs[2 * (g * GK + i)] = X;
                         xs[2 * (g * GK + i) + 1] = Y;
@@ -616,7 +649,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                which is line n2's half spectrum (its own output row) */
             constexpr long long NONE = -0x7fffffffffffffffLL - 1; /* INT64_MIN */
             if (u == 0 && real) lbase[lt] = act ? bin : NONE;
-            const long long n1 = tile % a.nb[1];
+            const long long n1 = line_ix(a, tile * NL).i1;
             cx<R> wp[NL];
             sfor<0, NL>([&](auto pc) {
                 constexpr int pp = decltype(pc)::value;
@@ -694,7 +727,6 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         }
         auto gst = [&](int k, cx<R> v) {
             /* v = swap(z_k) */
-            v.x *= sc; v.y *= sc;
             if (!act) return;
             if (rm == FK_RM_DCT3 || rm == FK_RM_DST3) {
                 /* y_2i = v_i (i < L), y_{2i+1} = v_{n-1-i}: v_m goes to 2m
@@ -738,8 +770,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         auto mid = [&](int j) -> cx<R> { return swp(mul(lds_at(j), Bt[j])); };
         auto gst = [&](int k, cx<R> v) {
             if (k < n && act) {
-                cx<R> y = mul(swp(v), chirp[k]);
-                y.x *= sc; y.y *= sc;
+                const cx<R> y = mul(swp(v), chirp[k]);
                 out[bout + k * a.os] = swo ? swp(y) : y;
             }
         };
@@ -788,11 +819,11 @@ stockham_pipe(fk_args a)
     using SY = typename std::conditional<wave_lines, SyncWave, SyncAll>::type;
     extern __shared__ unsigned char smem_raw[];
     cx<R> *lds = reinterpret_cast<cx<R> *>(smem_raw);
-    const int tid = threadIdx.x, lt = tid / TPL, u = tid % TPL;
+    const int tid = threadIdx.x, u = tid % TPL;
+    const int lt = TPL % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / TPL) : tid / TPL;
     const long long ntiles = (a.nlines + NL - 1) / NL, step = gridDim.x;
     const unsigned fl = a.flags;
     const bool swi = fl & FK_SWAP_IN, swo = fl & FK_SWAP_OUT;
-    const R sc = (fl & FK_SCALE) ? (R)a.scale : (R)1;
     const long long is = a.is, os = a.os;
     const cx<R> *tw = reinterpret_cast<const cx<R> *>(a.tw);
     const cx<R> *in = reinterpret_cast<const cx<R> *>(a.in);
@@ -803,12 +834,7 @@ stockham_pipe(fk_args a)
     auto line_of = [&](long long t, long long &bin, long long &bout) -> bool {
         const long long line = t * NL + lt;
         const bool act = line < a.nlines;
-        long long q = act ? line : 0;
-        const long long i0 = q % a.nb[0];
-        q /= a.nb[0];
-        const long long i1 = q % a.nb[1], i2 = q / a.nb[1];
-        bin = i0 * a.ids[0] + i1 * a.ids[1] + i2 * a.ids[2];
-        bout = i0 * a.ods[0] + i1 * a.ods[1] + i2 * a.ods[2];
+        line_off(a, line_ix(a, act ? line : 0), bin, bout);
         return act;
     };
     long long t = blockIdx.x;
@@ -819,21 +845,13 @@ stockham_pipe(fk_args a)
         const cx<R> *p = in + bin + u * is;
         sfor<0, R0>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
-            const cx<R> x = p[(long long)(r * NB0) * is];
-            v[r] = swi ? swp(x) : x;
+            v[r] = p[(long long)(r * NB0) * is];
         });
     };
     long long bin, bout;
     bool act = line_of(t, bin, bout);
     fetch(bin, cur);
     auto lds_at = [&](auto j) -> cx<R> & { return lds[G::idx(lt, j)]; };
-    /* output post-op of stockham<> without the four-step twiddle (the
-       planner runs passes that need it with stockham<>): scale, swap */
-    auto post = [&](cx<R> v) -> cx<R> {
-        v.x *= sc;
-        v.y *= sc;
-        return swo ? swp(v) : v;
-    };
     for (;;) {
         const long long tn = t + step;
         const bool more = tn < ntiles;
@@ -849,9 +867,12 @@ stockham_pipe(fk_args a)
             return cur[r];
         };
         auto gst = [&](auto k, cx<R> v) {
-            if (NL == 1 || act) outu[(long long)((int)k - u) * os] = post(v);
+            if (NL == 1 || act) outu[(long long)((int)k - u) * os] = v;
         };
-        run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, first, gst);
+        /* no four-step twiddle here: the planner runs passes that need it
+           with stockham<> */
+        run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, first, gst, SwapOp{swi},
+                                                       SwapOp{swo});
         if (!more) break;
         sfor<0, R0>([&](auto rc) {
             constexpr int r = decltype(rc)::value;
@@ -881,10 +902,10 @@ struct XsGeo {
     static constexpr int BPT = (NB + TPL - 1) / TPL;
 };
 
-template <typename R, class RL, int S, int L, int TPL, class PosF, class LastF>
+template <typename R, class RL, int S, int L, int TPL, class PosF, class LastF, class FinF>
 __device__ __forceinline__ void run_xs(int u, const cx<R> *__restrict__ tw, R *buf, PosF &&idx,
                                        cx<R> (&v)[XsGeo<RL, S, L, TPL>::BPT][XsGeo<RL, S, L, TPL>::Rs],
-                                       LastF &&last)
+                                       LastF &&last, const FinF &fin)
 {
     using X = XsGeo<RL, S, L, TPL>;
     constexpr int Rs = X::Rs, Ns = X::Ns, NB = X::NB, BPT = X::BPT;
@@ -901,6 +922,7 @@ __device__ __forceinline__ void run_xs(int u, const cx<R> *__restrict__ tw, R *b
                 });
             }
             Dft<R, Rs, 1>::run(v[i]);
+            if constexpr (S == RL::n - 1) fin.template run<Rs>(b, v[i]);
         }
     });
     auto each_out = [&](auto &&f) {
@@ -941,7 +963,7 @@ __device__ __forceinline__ void run_xs(int u, const cx<R> *__restrict__ tw, R *b
         __syncthreads();
         each_in([&](int j, cx<R> &x) { x.y = buf[idx(j)]; });
         __syncthreads();
-        run_xs<R, RL, S + 1, L, TPL>(u, tw, buf, idx, w, last);
+        run_xs<R, RL, S + 1, L, TPL>(u, tw, buf, idx, w, last, fin);
     }
 }
 
@@ -961,36 +983,19 @@ stockham_xs(fk_args a)
     const int u = MODE == FK_ROW ? tid % TPL : tid / NL;
     const long long line = tile * NL + lt;
     const bool act = line < a.nlines;
-    long long q = act ? line : 0;
-    const long long i0 = q % a.nb[0];
-    q /= a.nb[0];
-    const long long i1 = q % a.nb[1], i2 = q / a.nb[1];
-    const long long bin = i0 * a.ids[0] + i1 * a.ids[1] + i2 * a.ids[2];
-    const long long bout = i0 * a.ods[0] + i1 * a.ods[1] + i2 * a.ods[2];
+    const LineIx lx = line_ix(a, act ? line : 0);
+    long long bin, bout;
+    line_off(a, lx, bin, bout);
     const cx<R> *tw = reinterpret_cast<const cx<R> *>(a.tw);
     const cx<R> *in = reinterpret_cast<const cx<R> *>(a.in) + bin;
     cx<R> *out = reinterpret_cast<cx<R> *>(a.out);
     const unsigned fl = a.flags;
-    const bool swi = fl & FK_SWAP_IN, swo = fl & FK_SWAP_OUT;
-    /* output scale: multiplying by 1 when unscaled is exact and costs less
-       than selecting between scaled and unscaled values */
-    const R sc = (fl & FK_SCALE) ? (R)a.scale : (R)1;
+    const bool swi = fl & FK_SWAP_IN;
     R *buf = reinterpret_cast<R *>(smem_raw) + (MODE == FK_ROW ? lt * LP : lt);
     auto idx = [](int j) { return MODE == FK_ROW ? j + j / PAD : j * NL; };
-    /* output post-op as in stockham_body: four-step twiddle anchored in the
-       FP64 table every ANCH outputs of a butterfly, scale, swap */
-    constexpr int NS_LAST = RL::ns(RL::n - 1);
-    constexpr int ANCH = sizeof(R) == 8 ? 4 : 16;
-    cx<double> tw_cur = mk(1.0, 0.0), tw_step = mk(1.0, 0.0);
-    if (fl & FK_TW_OUT) tw_step = tw2d(a, (long long)NS_LAST * i0);
+    const PlainOut<RL::ns(RL::n - 1)> fin(a, fl, lx.i0);
     auto gst = [&](int k, cx<R> v) {
-        if (fl & FK_TW_OUT) {
-            if ((k / NS_LAST) % ANCH == 0) tw_cur = tw2d(a, (long long)k * i0);
-            else tw_cur = mul(tw_cur, tw_step);
-            v = mul(v, mk((R)tw_cur.x, (R)tw_cur.y));
-        }
-        v.x *= sc; v.y *= sc;
-        if (act) out[bout + k * a.os] = swo ? swp(v) : v;
+        if (act) out[bout + k * a.os] = v;
     };
     using X0 = XsGeo<RL, 0, L, TPL>;
     cx<R> v[X0::BPT][X0::Rs];
@@ -1005,7 +1010,7 @@ stockham_xs(fk_args a)
             });
         }
     });
-    run_xs<R, RL, 0, L, TPL>(u, tw, buf, idx, v, gst);
+    run_xs<R, RL, 0, L, TPL>(u, tw, buf, idx, v, gst, fin);
 }
 
 template <typename R, int NL, int MODE, int PAD, class RL, int TPL>

@@ -213,7 +213,6 @@ static void stockham_ops(const fk_pass *ps, ops *o)
            with the output, per element */
         ops_acc(&t, 2 * L, &CMUL);
     }
-    if (fl & FK_SCALE) t.mul += 2 * outs;
     ops_acc(o, lines, &t);
 }
 
