@@ -2152,6 +2152,42 @@ static void fill_magic(fk_args *a)
     if (a->tb > 0 && a->tN < (1LL << 31)) fk_magic((unsigned long long)a->tb, &a->qm[2], &a->qs[2]);
 }
 
+/* FP64 row passes of plain lines read and write non-temporally where that
+   measured faster (us, arrays rotated; one pass unless noted):
+     one pass, arrays of 16 MiB (together larger than the 32 MB of L2) and
+     more: 512 x 2048 9.0 -> 7.0, 512 x 8192 28.2 -> 25.3, 512 x 65536 377 ->
+     364, 4096 x 1024 28.6 -> 26.3, also where a second transform reads the
+     output back (512 x 8192 there and back 51.5 -> 51.5, 4096 63 -> 52); below
+     16 MiB no difference;
+     the pipelined kernels up to 512 MiB (4096 x 8192 206 -> 204; 4096 x 16384
+     388 -> 404 the other way);
+     the first pass of several: its input from 64 MiB on (512x512 x 16 57.6 ->
+     53.7, x 64 203 -> 182, x 128 410 -> 391; x 4 19.4 -> 19.9 the other way),
+     its output, which the next pass reads, from 1 GiB on, four times the
+     memory-side cache (512x512 x 256 775 -> 760; x 64 182 -> 208 the other
+     way).
+   FP32 rows and column passes measured the same or slower. */
+static void mark_streams(fk_plan *P)
+{
+    const long long MB = 1LL << 20;
+    int i;
+    for (i = 0; i < P->npass; ++i) {
+        fk_pass *p = P->pass + i;
+        long long n;
+        if (p->type != FK_PASS_STOCKHAM || p->k->mode != FK_ROW || p->k->io != FK_IO_PLAIN ||
+            p->k->prec != 0)
+            continue;
+        n = p->a.nlines * p->k->L * (long long)csz(0);
+        if (P->npass == 1) {
+            if (n >= 16 * MB && (!p->k->loop || n <= 512 * MB))
+                p->a.flags |= FK_NT_IN | FK_NT_OUT;
+        } else if (i == 0) {
+            if (n >= 64 * MB) p->a.flags |= FK_NT_IN;
+            if (n >= 1024 * MB) p->a.flags |= FK_NT_OUT;
+        }
+    }
+}
+
 static fk_plan *build_plan(const fk_problem *pb0, hipStream_t st, const int *choice, int nchoice,
                            ctx *cout)
 {
@@ -2271,6 +2307,7 @@ static fk_plan *build_plan(const fk_problem *pb0, hipStream_t st, const int *cho
     if (c.err) goto fail;
     for (i = 0; i < P->npass; ++i)
         if (P->pass[i].type == FK_PASS_STOCKHAM) fill_magic(&P->pass[i].a);
+    mark_streams(P);
 done_ok:
     for (i = 0; i < P->nscratch; ++i) {
         if (P->scratch_bytes[i]) {

@@ -42,6 +42,9 @@ enum {
 #define FK_REAL_QUAD 32u  /* FP32 real input stride 1, lines 16-byte aligned: the
                              reordered loads of REDFT10 / RODFT10 read quads */
 
+#define FK_NT_IN     64u  /* FP64 plain rows: non-temporal input reads */
+#define FK_NT_OUT    128u /* FP64 plain rows: non-temporal output writes */
+
 /* real-to-real kinds fused into the FK_IO_R2C_RR / FK_IO_C2R_RR kernels (rmode):
    the real line is read or written in the kind's order, with the kind's
    twiddle exp(-i pi m / 4n) from rtw */

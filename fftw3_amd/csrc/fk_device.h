@@ -42,6 +42,71 @@ __device__ __forceinline__ cx<R> mul(cx<R> a, cx<R> b)
 template <typename R>
 __device__ __forceinline__ cx<R> swp(cx<R> a) { return mk(a.y, a.x); }
 
+/* ---- access to the arrays a pass transforms ---- */
+
+template <int BYTES> struct RawT;
+template <> struct RawT<4> { typedef unsigned t; };
+template <> struct RawT<8> { typedef unsigned long long t; };
+template <> struct RawT<16> { typedef unsigned t __attribute__((ext_vector_type(4))); };
+
+/* How an access treats the caches: C_KEEP as usual; C_ONCE a load that leaves
+   nothing in the CU's L1 (agent scope, 8-byte values), so that the twiddle
+   tables stay there; C_NT non-temporal, which also leaves nothing in L2 and
+   the memory-side cache. */
+enum { C_KEEP = 0, C_ONCE = 1, C_NT = 2 };
+template <int A>
+using Acc = std::integral_constant<int, A>;
+
+template <int A, class T>
+__device__ __forceinline__ T ldg(Acc<A>, const T *p)
+{
+    typedef typename RawT<sizeof(T)>::t U;
+    if constexpr (A == C_NT)
+        return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const U *>(p)));
+    else if constexpr (A == C_ONCE && sizeof(T) == 8)
+        return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const U *>(p), __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT));
+    else
+        return *p;
+}
+template <int A, class T>
+__device__ __forceinline__ void stg(Acc<A>, T *p, T v)
+{
+    typedef typename RawT<sizeof(T)>::t U;
+    if constexpr (A == C_NT)
+        __builtin_nontemporal_store(__builtin_bit_cast(U, v), reinterpret_cast<U *>(p));
+    else
+        *p = v;
+}
+
+/* Calls f(Acc<A>) with A = C_NT when the (uniform) flag is set, else C_KEEP.
+   The empty asm keeps it one branch around the whole block. */
+template <class F>
+__device__ __forceinline__ void with_acc(bool nt, F &&f)
+{
+    if (nt) {
+        asm volatile("");
+        f(Acc<C_NT>{});
+    } else {
+        f(Acc<C_KEEP>{});
+    }
+}
+
+/* A data source or sink of a stage that chooses between forms of its
+   accesses once for all of a butterfly's elements: f is called with the
+   loop over the elements and calls it with the accessor of its choice. */
+template <class F>
+struct Hoisted {
+    F f;
+};
+template <class F>
+__device__ __forceinline__ Hoisted<F> hoisted(F f)
+{
+    return Hoisted<F>{f};
+}
+template <class T> struct is_hoisted : std::false_type {};
+template <class F> struct is_hoisted<Hoisted<F>> : std::true_type {};
+
 /* ---- compile-time trigonometry (Taylor series on an octant) ---- */
 
 constexpr double kPI = 3.14159265358979323846264338327950288;

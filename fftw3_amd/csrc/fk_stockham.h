@@ -179,8 +179,8 @@ struct PlainOut {
 
 /*
  * One Stockham stage.  LoadF(j) -> cx<R> and StoreF(k, cx<R>) abstract the
- * data source and sink; IN_LDS/OUT_LDS say whether they touch LDS, which
- * decides the barriers.  pre / fin run on a butterfly's registers after the
+ * data source and sink (or are Hoisted); IN_LDS/OUT_LDS say whether they
+ * touch LDS, which decides the barriers.  pre / fin run on a butterfly's registers after the
  * loads / before the stores.
  */
 template <typename R, class RL, int S, int L, int TPL, bool IN_LDS, bool OUT_LDS,
@@ -193,16 +193,22 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
     constexpr int NB = L / Rs;
     constexpr int BPT = (NB + TPL - 1) / TPL;
     cx<R> v[BPT][Rs];
-    sfor<0, BPT>([&](auto ic) {
-        constexpr int i = decltype(ic)::value;
-        const int b = u + i * TPL;
-        if ((NB % TPL == 0) || b < NB) {
-            sfor<0, Rs>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
-                v[i][r] = ld(At<r * NB>{b});
-            });
-        }
-    });
+    auto load = [&](auto &&get) {
+        sfor<0, BPT>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            const int b = u + i * TPL;
+            if ((NB % TPL == 0) || b < NB) {
+                sfor<0, Rs>([&](auto rc) {
+                    constexpr int r = decltype(rc)::value;
+                    v[i][r] = get(At<r * NB>{b});
+                });
+            }
+        });
+    };
+    typedef typename std::decay<LoadF>::type Ld;
+    typedef typename std::decay<StoreF>::type St;
+    if constexpr (is_hoisted<Ld>::value) ld.f(load);
+    else load(ld);
     if constexpr (IN_LDS && OUT_LDS) SY::sync();
     sfor<0, BPT>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
@@ -223,10 +229,14 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
             const int base = (b - k) * Rs + k;
             fin.template run<Rs>(base, v[i]);
             /* stage 0 (Ns = 1) writes Rs consecutive outputs from b*Rs */
-            sfor<0, Rs>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
-                st(At<r * Ns, (S == 0 ? Rs : 1)>{base}, v[i][r]);
-            });
+            auto store = [&](auto &&put) {
+                sfor<0, Rs>([&](auto rc) {
+                    constexpr int r = decltype(rc)::value;
+                    put(At<r * Ns, (S == 0 ? Rs : 1)>{base}, v[i][r]);
+                });
+            };
+            if constexpr (is_hoisted<St>::value) st.f(store);
+            else store(st);
         }
     });
     if constexpr (OUT_LDS) SY::sync();
@@ -308,6 +318,8 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
     const cx<R> *tw = reinterpret_cast<const cx<R> *>(a.tw);
     const unsigned fl = a.flags;
     const bool swi = fl & FK_SWAP_IN, swo = fl & FK_SWAP_OUT;
+    const bool nti = fl & FK_NT_IN, nto = fl & FK_NT_OUT;
+    constexpr bool NTP = sizeof(R) == 8 && MODE == FK_ROW && IO == FK_IO_PLAIN;
     auto lds_at = [&](auto j) -> cx<R> & {
         if constexpr (NT == NR) return lds[G::idx(lt, j)];
         else return real ? lds[G::idx(lt, j)] : trash[tid & 63];
@@ -321,12 +333,20 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         const long long is = a.is, os = a.os;
         const cx<R> *inu = reinterpret_cast<const cx<R> *>(a.in) + bin + u * is;
         cx<R> *out = reinterpret_cast<cx<R> *>(a.out);
-        auto gld = [&](int j) -> cx<R> { return inu[(long long)(j - u) * is]; };
+        auto gld = hoisted([&](auto &&load) {
+            with_acc(NTP && nti, [&](auto acc) {
+                load([&](int j) -> cx<R> { return ldg(acc, inu + (long long)(j - u) * is); });
+            });
+        });
         if constexpr (IO == FK_IO_PLAIN) {
             cx<R> *outu = out + bout + u * os;
-            auto gst = [&](int k, cx<R> v) {
-                if (act) outu[(long long)(k - u) * os] = v;
-            };
+            auto gst = hoisted([&](auto &&store) {
+                with_acc(NTP && nto, [&](auto acc) {
+                    store([&](int k, cx<R> v) {
+                        if (act) stg(acc, outu + (long long)(k - u) * os, v);
+                    });
+                });
+            });
             const PlainOut<RL::ns(RL::n - 1)> fin(a, fl, i0);
             run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst, SwapOp{swi},
                                                            fin);
@@ -406,7 +426,284 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             outr[(N2 - 1 - 2LL * p) * a.os] = sn ? -yo : yo;
         };
         run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst);
-    } else if constexpr (IO == FK_IO_R2C || IO == FK_IO_R2C_RR || IO == FK_IO_R2C_XR) {
+    } else if constexpr (IO == FK_IO_R2C || IO == FK_IO_R2C_XR) {
+        /* real line of 2L samples viewed as L complex z_j = x_2j + i x_2j+1;
+           after the L-point DFT Z, X[k] = E[k] + W_2L^k O[k] with
+           E = (Z[k] + conj Z[L-k])/2, O = (Z[k] - conj Z[L-k])/(2i),
+           k = 0..L (the role of rdft/ct-hc2c.c:197-210's HC2C_VIA_DFT).
+           What bounds it: the twiddle loads of its three stages and of the
+           post-pass outnumber the data loads and live in the CU's L1, which
+           the data streams through.  Data read past L1 (C_ONCE) leaves the
+           tables there: FP32 2048 x 65536 0.246 -> 0.205 ms. */
+        const R *inr = reinterpret_cast<const R *>(a.in) + bin;
+        cx<R> *out = reinterpret_cast<cx<R> *>(a.out);
+        const cx<R> *wk = reinterpret_cast<const cx<R> *>(a.aux);
+        const long long is = a.is, os = a.os;
+        auto gld = hoisted([&](auto &&load) {
+            if (fl & FK_REAL_UNIT) {
+                const cx<R> *inz = reinterpret_cast<const cx<R> *>(inr) + u;
+                load([&](int j) -> cx<R> { return ldg(Acc<C_ONCE>{}, inz + (j - u)); });
+            } else {
+                asm volatile("");
+                const R *inu = inr + 2 * u * is;
+                load([&](int j) -> cx<R> {
+                    const long long o = 2 * (j - u) * is;
+                    return mk(inu[o], inu[o + is]);
+                });
+            }
+        });
+        auto lst = [&](auto k, cx<R> v) { lds_at(k) = v; };
+        /* bin k <= L/2 gives bins k and L-k from the same Z[k], Z[L-k] and
+           one twiddle (W_2L^(L-k) = -conj W_2L^k); bins k = u + i*TPL in
+           groups of 8 (compile-time count): the group's twiddle loads are
+           in flight together */
+        constexpr int HK = L / 2;
+        constexpr int NK2 = (HK + 1 + TPL - 1) / TPL;
+        constexpr int GK = 8;
+        constexpr bool XR = IO == FK_IO_R2C_XR;
+        /* few bins per thread: their twiddles are loaded before the stages,
+           so the load latency hides behind the FFT instead of following it */
+        constexpr bool PRE = NK2 <= 20;
+        cx<R> wpre[PRE ? NK2 : 1];
+        if constexpr (PRE) {
+            sfor<0, NK2>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int k = u + i * TPL;
+                wpre[i] = wk[k <= HK ? k : HK];
+            });
+        }
+        run_stages<R, RL, 0, L, TPL, false, true, SY>(u, tw, lds_at, gld, lst);
+        /* bins k = u + i*TPL <= L/2 and L-k of the line: f(i, k, X[k], X[L-k]) */
+        auto bins = [&](auto &&f) {
+            sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
+                constexpr int g = decltype(gc)::value;
+                constexpr int cnt = (NK2 - g * GK) < GK ? (NK2 - g * GK) : GK;
+                cx<R> w[cnt];
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    if constexpr (PRE) w[i] = wpre[g * GK + i];
+                    else if (k <= HK) w[i] = wk[k];
+                });
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    if (k <= HK) {
+                        const cx<R> zk = lds_at(k);
+                        const cx<R> zc = lds_at(k == 0 ? 0 : L - k);
+                        const R er = (R)0.5 * (zk.x + zc.x), ei = (R)0.5 * (zk.y - zc.y);
+                        /* O = (Z[k] - conj Z[L-k]) / (2i) */
+                        const R orr = (R)0.5 * (zk.y + zc.y), oi = (R)-0.5 * (zk.x - zc.x);
+                        const R wx = w[i].x, wy = w[i].y;
+                        /* X[k] = E + W O; X[L-k] = conj(E - W O), written as
+                           the form of bin L-k on its own (E' = conj E,
+                           O' = conj O, W' = -conj W) so that both round as
+                           that form does */
+                        const cx<R> X = mk(er + orr * wx - oi * wy, ei + orr * wy + oi * wx);
+                        const cx<R> Y =
+                            mk(er + orr * (-wx) - (-oi) * wy, (-ei) + orr * wy + (-oi) * (-wx));
+                        f(std::integral_constant<int, g * GK + i>{}, k, X, Y);
+                    }
+                });
+            });
+        };
+        if constexpr (!XR) {
+            cx<R> *outk = out + bout + u * os, *outm = out + bout + (L - u) * os;
+            bins([&](auto ic, int k, cx<R> X, cx<R> Y) {
+                const long long d = (long long)(decltype(ic)::value * TPL) * os;
+                if (act) {
+                    outk[d] = X;
+                    if (2 * k != L) outm[-d] = Y;
+                }
+            });
+        } else {
+            /* twiddles of the first column stage, W_n0^(n1*p) (n1 = the
+               tile's line-group index, uniform over the workgroup) */
+            const LineIx tx = line_ix(a, tile * NL);
+            long long tin, tout;
+            line_off(a, tx, tin, tout);
+            cx<R> wp[NL];
+            sfor<0, NL>([&](auto pc) {
+                constexpr int pp = decltype(pc)::value;
+                wp[pp] = pp == 0 ? mk((R)1, (R)0) : tw2<R>(a, tx.i1 * pp);
+            });
+            /* the bins stay in registers until every bin of the line has
+               been formed, then replace Z in the line's LDS row */
+            cx<R> xs[2 * NK2];
+            bins([&](auto ic, int, cx<R> X, cx<R> Y) {
+                constexpr int i = decltype(ic)::value;
+                xs[2 * i] = X;
+                xs[2 * i + 1] = Y;
+            });
+            SY::sync();
+            sfor<0, NK2>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int k = u + i * TPL;
+                if (k <= HK) {
+                    lds_at(k) = xs[2 * i];
+                    if (2 * k != L) lds_at(L - k) = xs[2 * i + 1];
+                }
+            });
+            __syncthreads();
+            /* first stage of the column DFT over the tile's NL rows
+               n = n1 + m*n2 (n2 = the line's batch index i0, n1 = i1; the
+               planner sets nb[0] = NL, so a tile is one n1 and always whole):
+               for every bin k y_p = W_n0^(n1*p) sum_n2 X_n2[k] W_NL^(n2*p),
+               n0 = a.tN, stored to the tile's output line p */
+            cx<R> *outk = out + tout + tid * os;
+            for (int k = tid; k <= L; k += NT, outk += NT * os) {
+                cx<R> v[NL];
+                sfor<0, NL>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    v[q] = lds[G::idx(q, k)];
+                });
+                Dft<R, NL, 1>::run(v);
+                sfor<0, NL>([&](auto pc) {
+                    constexpr int pp = decltype(pc)::value;
+                    outk[pp * a.ods[0]] = pp == 0 ? v[0] : mul(v[pp], wp[pp]);
+                });
+            }
+        }
+    } else if constexpr (IO == FK_IO_C2R || IO == FK_IO_C2R_XR) {
+        /* half-length inverse: Z[k] = E[k] + i O[k],
+           E[k] = X[k] + conj X[L-k], O[k] = (X[k] - conj X[L-k]) W_2L^-k,
+           z = DFT^-1_L(Z) (unnormalized), y_2m = Re z_m, y_2m+1 = Im z_m.
+           Im X[0] and Im X[L] are ignored, as the r2cb codelets do. */
+        const cx<R> *in = reinterpret_cast<const cx<R> *>(a.in);
+        R *outr = reinterpret_cast<R *>(a.out) + bout;
+        const cx<R> *wk = reinterpret_cast<const cx<R> *>(a.aux);
+        const long long is = a.is, os = a.os;
+        /* bins X[k], X[L-k] (k <= L/2) are read together and give Z[k] and
+           Z[L-k] with one twiddle (W_2L^(L-k) = -conj W_2L^k); they are
+           written to LDS before the stages, which read Z as it is */
+        constexpr int HK = L / 2;
+        constexpr int NK2 = (HK + 1 + TPL - 1) / TPL;
+        constexpr int GK = 8;
+        /* swapped Z (the backward DFT runs as the forward one on swapped
+           data): e = X[k] + conj X[L-k], d = X[k] - conj X[L-k],
+           o = d conj(W_2L^k); Z[k] = e + i o and, by the symmetry above,
+           Z[L-k] = conj e + i conj o */
+        auto zpair = [&](int k, cx<R> xk, cx<R> xc, cx<R> w, cx<R> &z0, cx<R> &z1) {
+            if (k == 0) {
+                xk.y = 0;
+                xc.y = 0;
+            }
+            const cx<R> e = mk(xk.x + xc.x, xk.y - xc.y);
+            const cx<R> d = mk(xk.x - xc.x, xk.y + xc.y);
+            const cx<R> o = mk(d.x * w.x + d.y * w.y, d.y * w.x - d.x * w.y);
+            z0 = mk(e.y + o.x, e.x - o.y);
+            z1 = mk(o.x - e.y, e.x + o.y);
+        };
+        if constexpr (IO == FK_IO_C2R_XR) {
+            /* last stage of the inverse column DFT over the tile's NL input
+               rows (row p = the line's batch index i0, n1 = i1; the planner
+               sets nb[0] = NL, so a tile is one n1 and always whole): for
+               every bin k u_n2 = sum_p W_NL^(-n2*p) W_n0^(-n1*p) Y_p[k],
+               n0 = a.tN, which is line n2's half spectrum (its own output
+               row); the inverse DFT as the forward one on swapped data.
+               Bin L/2 is thread 0's as well: its loads are issued with the
+               others', so that no wave waits for memory twice. */
+            const LineIx tx = line_ix(a, tile * NL);
+            long long tin, tout;
+            line_off(a, tx, tin, tout);
+            cx<R> wp[NL];
+            sfor<0, NL>([&](auto pc) {
+                constexpr int pp = decltype(pc)::value;
+                const cx<R> t = pp == 0 ? mk((R)1, (R)0) : tw2<R>(a, tx.i1 * pp);
+                wp[pp] = mk(t.x, -t.y);
+            });
+            auto coldft = [&](cx<R> *v) {
+                sfor<0, NL>([&](auto pc) {
+                    constexpr int pp = decltype(pc)::value;
+                    v[pp] = swp(pp == 0 ? v[0] : mul(v[pp], wp[pp]));
+                });
+                Dft<R, NL, 1>::run(v);
+            };
+            auto put = [&](int k, cx<R> w, cx<R> *v, cx<R> *vm) {
+                sfor<0, NL>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    cx<R> z0, z1;
+                    zpair(k, swp(v[q]), swp(vm[q]), w, z0, z1);
+                    lds[G::idx(q, k)] = z0;
+                    if (k != 0 && 2 * k != L) lds[G::idx(q, L - k)] = z1;
+                });
+            };
+            const cx<R> *ink = in + tin + tid * is, *inm = in + tin + (L - tid) * is;
+            auto fetch = [&](const cx<R> *p, cx<R> *v) {
+                sfor<0, NL>([&](auto pc) {
+                    constexpr int pp = decltype(pc)::value;
+                    v[pp] = ldg(Acc<C_ONCE>{}, p + pp * a.ids[0]);
+                });
+            };
+            cx<R> vh[NL];
+            if (tid == 0) fetch(in + tin + HK * is, vh);
+            for (int k = tid; k < HK; k += NT, ink += NT * is, inm -= NT * is) {
+                cx<R> v[NL], vm[NL];
+                fetch(ink, v);
+                fetch(inm, vm);
+                const cx<R> w = wk[k];
+                coldft(v);
+                coldft(vm);
+                put(k, w, v, vm);
+            }
+            if (tid == 0) {
+                coldft(vh);
+                put(HK, wk[HK], vh, vh);
+            }
+            __syncthreads();
+        } else {
+            /* loads in groups of 8 (compile-time count) so that each group
+               is in flight at once, then its LDS stores */
+            const cx<R> *ink = in + bin + u * is, *inm = in + bin + (L - u) * is;
+            sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
+                constexpr int g = decltype(gc)::value;
+                constexpr int cnt = (NK2 - g * GK) < GK ? (NK2 - g * GK) : GK;
+                cx<R> xa[cnt], xb[cnt], w[cnt];
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    const long long d = (long long)((g * GK + i) * TPL) * is;
+                    if (k <= HK) {
+                        xa[i] = ldg(Acc<C_ONCE>{}, ink + d);
+                        xb[i] = ldg(Acc<C_ONCE>{}, inm - d);
+                        w[i] = wk[k];
+                    }
+                });
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    if (k <= HK) {
+                        cx<R> z0, z1;
+                        zpair(k, xa[i], xb[i], w[i], z0, z1);
+                        lds_at(k) = z0;
+                        if (k != 0 && 2 * k != L) lds_at(L - k) = z1;
+                    }
+                });
+            });
+            SY::sync();
+        }
+        auto gst = hoisted([&](auto &&store) {
+            /* v = swap(z_k) */
+            if (fl & FK_REAL_UNIT) {
+                cx<R> *outz = reinterpret_cast<cx<R> *>(outr) + u;
+                store([&](int k, cx<R> v) {
+                    if (act) outz[k - u] = mk(v.y, v.x);
+                });
+            } else {
+                asm volatile("");
+                R *outu = outr + 2 * u * os;
+                store([&](int k, cx<R> v) {
+                    const long long o = 2 * (k - u) * os;
+                    if (act) {
+                        outu[o] = v.y;
+                        outu[o + os] = v.x;
+                    }
+                });
+            }
+        });
+        auto zld = [&](auto j) -> cx<R> { return lds_at(j); };
+        run_stages<R, RL, 0, L, TPL, true, false, SY>(u, tw, lds_at, zld, gst);
+    } else if constexpr (IO == FK_IO_R2C_RR) {
         /* real line of 2L samples viewed as L complex z_j = x_2j + i x_2j+1;
            after the L-point DFT Z, X[k] = E[k] + W_2L^k O[k] with
            E = (Z[k] + conj Z[L-k])/2, O = (Z[k] - conj Z[L-k])/(2i),
@@ -596,7 +893,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                 });
             }
         }
-    } else if constexpr (IO == FK_IO_C2R || IO == FK_IO_C2R_RR || IO == FK_IO_C2R_XR) {
+    } else if constexpr (IO == FK_IO_C2R_RR) {
         /* half-length inverse: Z[k] = E[k] + i O[k],
            E[k] = X[k] + conj X[L-k], O[k] = (X[k] - conj X[L-k]) W_2L^-k,
            z = DFT^-1_L(Z) (unnormalized), y_2m = Re z_m, y_2m+1 = Im z_m.
@@ -843,9 +1140,11 @@ stockham_pipe(fk_args a)
     /* stage-0 inputs of the thread's butterfly */
     auto fetch = [&](long long bin, cx<R> *v) {
         const cx<R> *p = in + bin + u * is;
-        sfor<0, R0>([&](auto rc) {
-            constexpr int r = decltype(rc)::value;
-            v[r] = p[(long long)(r * NB0) * is];
+        with_acc(sizeof(R) == 8 && (fl & FK_NT_IN), [&](auto acc) {
+            sfor<0, R0>([&](auto rc) {
+                constexpr int r = decltype(rc)::value;
+                v[r] = ldg(acc, p + (long long)(r * NB0) * is);
+            });
         });
     };
     long long bin, bout;
@@ -866,9 +1165,13 @@ stockham_pipe(fk_args a)
             constexpr int r = AtOff<typename std::decay<decltype(j)>::type>::v / NB0;
             return cur[r];
         };
-        auto gst = [&](auto k, cx<R> v) {
-            if (NL == 1 || act) outu[(long long)((int)k - u) * os] = v;
-        };
+        auto gst = hoisted([&](auto &&store) {
+            with_acc(sizeof(R) == 8 && (fl & FK_NT_OUT), [&](auto acc) {
+                store([&](int k, cx<R> v) {
+                    if (NL == 1 || act) stg(acc, outu + (long long)(k - u) * os, v);
+                });
+            });
+        });
         /* no four-step twiddle here: the planner runs passes that need it
            with stockham<> */
         run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, first, gst, SwapOp{swi},
