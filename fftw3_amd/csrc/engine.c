@@ -105,7 +105,7 @@ void fk_free(void *p)
 /* ------------------------------------------------------------------ */
 /* cached device tables (freed by fk_cleanup)                          */
 
-enum { T_STAGE, T_TW2, T_LINE, T_CHIRP, T_BLUEB };
+enum { T_STAGE, T_TW2, T_LINE, T_CHIRP, T_BLUEB, T_DCT, T_DCT4 };
 
 typedef struct tbl {
     int type, prec, nrad;
@@ -200,6 +200,35 @@ static const void *line_table(int prec, long long n, long long count, hipStream_
     t = tbl_new(T_LINE, prec, n, count, 0, 0, csz(prec) * (size_t)count);
     if (!t) return 0;
     if (fkm_gen_line_tw(t->dev, prec, n, count, st)) return 0;
+    return t->dev;
+}
+
+/* twiddles of the fused REDFT10 / REDFT01 kernels (and their sine kinds) of
+   length n: for k <= n/4 the pair exp(-i pi k / 2n), exp(-i pi 5k / 2n) =
+   exp(-i pi k / 2n) W_n^k, next to each other */
+static const void *dct_table(int prec, long long n, hipStream_t st)
+{
+    const long long cnt = n / 4 + 1;
+    tbl *t = tbl_find(T_DCT, prec, n, 0, 0, 0);
+    if (t) return t->dev;
+    t = tbl_new(T_DCT, prec, n, 0, 0, 0, 2 * csz(prec) * (size_t)cnt);
+    if (!t) return 0;
+    if (fkm_gen_affine_tw(t->dev, prec, 0, 2, 4 * n, 1, 0, cnt, st)) return 0;
+    if (fkm_gen_affine_tw(t->dev, prec, 1, 2, 4 * n, 5, 0, cnt, st)) return 0;
+    return t->dev;
+}
+
+/* twiddles of the fused REDFT11 / RODFT11 kernels of length n = 2L: L input
+   twiddles exp(-i pi (4m+1) / 4n), then L output twiddles exp(-i pi p / n) */
+static const void *dct4_table(int prec, long long n, hipStream_t st)
+{
+    const long long L = n / 2;
+    tbl *t = tbl_find(T_DCT4, prec, n, 0, 0, 0);
+    if (t) return t->dev;
+    t = tbl_new(T_DCT4, prec, n, 0, 0, 0, 2 * csz(prec) * (size_t)L);
+    if (!t) return 0;
+    if (fkm_gen_affine_tw(t->dev, prec, 0, 1, 8 * n, 4, 1, L, st)) return 0;
+    if (fkm_gen_affine_tw(t->dev, prec, L, 1, 2 * n, 1, 0, L, st)) return 0;
     return t->dev;
 }
 
@@ -1820,23 +1849,35 @@ static int plan_r2r_1d(ctx *c, int kind, long long n, long long is, long long os
                        ((uintptr_t)(io == FK_IO_R2C_RR ? iptr : optr) % (2 * rs)) == 0;
             const void *wk = line_table(prec, 2 * L, L + 1, c->st);
             for (i = 0; i < nb; ++i) unit &= ((io == FK_IO_R2C_RR ? b[i].is : b[i].os) % 2) == 0;
-            const int twid = rm == FK_RM_DCT2 || rm == FK_RM_DST2 || rm == FK_RM_DCT3 ||
-                             rm == FK_RM_DST3 || rm == FK_RM_DCT4 || rm == FK_RM_DST4;
-            if (twid) wt = line_table(prec, 8 * n, 2 * n, c->st);
+            const int dct2 = rm == FK_RM_DCT2 || rm == FK_RM_DST2;
+            const int dct3 = rm == FK_RM_DCT3 || rm == FK_RM_DST3;
+            const int twid = dct2 || dct3 || rm == FK_RM_DCT4 || rm == FK_RM_DST4;
+            if (rm == FK_RM_DCT4 || rm == FK_RM_DST4) wt = dct4_table(prec, n, c->st);
+            else if (twid) wt = dct_table(prec, n, c->st);
             if (!wk || (twid && !wt)) {
                 c->err = 1;
                 set_err("twiddle table allocation failed");
                 return -1;
             }
             if (unit) fl |= FK_REAL_UNIT;
-            if (prec == 1 && k->mode == FK_ROW && (rm == FK_RM_DCT2 || rm == FK_RM_DST2) && is == 1 &&
-                ((uintptr_t)iptr % 16) == 0) {
+            /* REDFT11 / RODFT11 on unit-stride lines whole pairs apart (and
+               the arrays bound at execute aligned to pairs, launch_pass) */
+            if (io == FK_IO_DCT4 && is == 1 && os == 1) {
+                int pairs = 1;
+                for (i = 0; i < nb; ++i) pairs &= b[i].is % 2 == 0 && b[i].os % 2 == 0;
+                if (pairs) fl |= FK_REAL_UNIT;
+            }
+            /* unit-stride lines a whole number of quads apart: REDFT10 /
+               RODFT10 read, REDFT01 / RODFT01 write four reals at a time
+               when the array bound at execute is 16-byte aligned
+               (launch_pass) */
+            if (k->mode == FK_ROW && ((dct2 && is == 1) || (dct3 && os == 1))) {
                 int quad = 1;
-                for (i = 0; i < nb; ++i) quad &= (b[i].is % 4) == 0;
-                if (quad) {
-                    fl |= FK_REAL_QUAD;
-                    need_align(c, ib, 16);
-                }
+                for (i = 0; i < nb; ++i) quad &= ((dct2 ? b[i].is : b[i].os) % 4) == 0;
+                if (quad) fl |= FK_REAL_QUAD;
+                /* the requirement on the input that FP32 plans made on
+                   aligned arrays have always had */
+                if (quad && dct2 && prec == 1 && ((uintptr_t)iptr % 16) == 0) need_align(c, ib, 16);
             }
             emit_stockham(c, k, is, os, nb, b, ib, 0, ob, 0, fl, rs, rs);
             for (; before < (size_t)P->npass; ++before) {
@@ -2152,7 +2193,7 @@ static void fill_magic(fk_args *a)
     if (a->tb > 0 && a->tN < (1LL << 31)) fk_magic((unsigned long long)a->tb, &a->qm[2], &a->qs[2]);
 }
 
-/* FP64 row passes of plain lines read and write non-temporally where that
+/* Row passes that bypass the caches.  FP64 passes of plain lines read and write non-temporally where that
    measured faster (us, arrays rotated; one pass unless noted):
      one pass, arrays of 16 MiB (together larger than the 32 MB of L2) and
      more: 512 x 2048 9.0 -> 7.0, 512 x 8192 28.2 -> 25.3, 512 x 65536 377 ->
@@ -2166,7 +2207,10 @@ static void fill_magic(fk_args *a)
      its output, which the next pass reads, from 1 GiB on, four times the
      memory-side cache (512x512 x 256 775 -> 760; x 64 182 -> 208 the other
      way).
-   FP32 rows and column passes measured the same or slower. */
+   FP32 rows and column passes measured the same or slower.
+   The quad loads of REDFT10 / RODFT10 rows, first pass and from 64 MiB on:
+   FP32 2048^2 x 16 288 -> 239, FP32 2048 x 32768 138 -> 118, FP64 512^2 x 64
+   126 -> 120; not FP64 alone (1024 x 32768 107 -> 116). */
 static void mark_streams(fk_plan *P)
 {
     const long long MB = 1LL << 20;
@@ -2174,10 +2218,14 @@ static void mark_streams(fk_plan *P)
     for (i = 0; i < P->npass; ++i) {
         fk_pass *p = P->pass + i;
         long long n;
-        if (p->type != FK_PASS_STOCKHAM || p->k->mode != FK_ROW || p->k->io != FK_IO_PLAIN ||
-            p->k->prec != 0)
+        if (p->type != FK_PASS_STOCKHAM || p->k->mode != FK_ROW) continue;
+        n = p->a.nlines * p->k->L * (long long)csz(p->k->prec);
+        if (p->k->io == FK_IO_R2C_RR) {
+            if (i == 0 && n >= 64 * MB && (p->k->prec == 1 || P->npass > 1))
+                p->a.flags |= FK_NT_IN;
             continue;
-        n = p->a.nlines * p->k->L * (long long)csz(0);
+        }
+        if (p->k->io != FK_IO_PLAIN || p->k->prec != 0) continue;
         if (P->npass == 1) {
             if (n >= 16 * MB && (!p->k->loop || n <= 512 * MB))
                 p->a.flags |= FK_NT_IN | FK_NT_OUT;
@@ -2643,6 +2691,11 @@ static int launch_pass(const fk_pass *ps, void *const *buf, hipStream_t st, int 
         void *args[1];
         a.in = (const char *)buf[ps->ibuf] + ps->ioff;
         a.out = (char *)buf[ps->obuf] + ps->ooff;
+        if ((a.flags & FK_REAL_QUAD) &&
+            ((uintptr_t)(ps->k->io == FK_IO_R2C_RR ? a.in : (const void *)a.out) % 16))
+            a.flags &= ~FK_REAL_QUAD;
+        if (ps->k->io == FK_IO_DCT4 && (((uintptr_t)a.in | (uintptr_t)a.out) % (2 * rsz(prec))))
+            a.flags &= ~FK_REAL_UNIT;
         args[0] = &a;
         return (int)hipLaunchKernel(ps->k->fn, (dim3){ps->grid, 1, 1}, (dim3){ps->block, 1, 1},
                                     args, ps->lds, st);

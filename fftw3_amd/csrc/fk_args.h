@@ -39,15 +39,15 @@ enum {
                              i0 by W_N^(k*i0) (four-step twiddle) */
 #define FK_SCALE     8u   /* multiply output by scale (element-wise passes) */
 #define FK_REAL_UNIT 16u  /* R2C: real input stride is 1 / C2R: output stride 1 */
-#define FK_REAL_QUAD 32u  /* FP32 real input stride 1, lines 16-byte aligned: the
-                             reordered loads of REDFT10 / RODFT10 read quads */
+#define FK_REAL_QUAD 32u  /* unit-stride real lines, 16-byte aligned: REDFT10 / RODFT10
+                             read, REDFT01 / RODFT01 write four reals at a time */
 
-#define FK_NT_IN     64u  /* FP64 plain rows: non-temporal input reads */
-#define FK_NT_OUT    128u /* FP64 plain rows: non-temporal output writes */
+#define FK_NT_IN     64u  /* FP64 plain rows, REDFT10 / RODFT10 rows: non-temporal reads */
+#define FK_NT_OUT    128u /* FP64 plain rows: non-temporal writes */
 
 /* real-to-real kinds fused into the FK_IO_R2C_RR / FK_IO_C2R_RR kernels (rmode):
    the real line is read or written in the kind's order, with the kind's
-   twiddle exp(-i pi m / 4n) from rtw */
+   twiddles from rtw */
 enum { FK_RM_NONE = 0,
        FK_RM_HC = 1,      /* R2C: halfcomplex output (R2HC) */
        FK_RM_DHT = 2,     /* R2C: Hartley output */
@@ -81,7 +81,9 @@ typedef struct {
     unsigned xcd_remap;       /* nonzero: spread tiles XCD-contiguously */
     unsigned rmode;           /* FK_RM_*: fused real-to-real kind */
     unsigned pad_;
-    const void *rtw;          /* FK_RM_DCT2/3, FK_RM_DST2/3: exp(-i pi m / 4n), m < 2n */
+    const void *rtw;          /* FK_RM_DCT2/3, FK_RM_DST2/3: pairs exp(-i pi k / 2n),
+                                 exp(-i pi 5k / 2n), k <= n/4; FK_RM_DCT4, FK_RM_DST4:
+                                 exp(-i pi (4m+1) / 4n), m < n/2, then exp(-i pi p / n) */
     /* division by multiplication, q / d = (2 q * qm >> 32) >> qs for q < 2^31:
        0 and 1 divide by nb[0] and nb[1] (qm[0] = 0: nlines >= 2^31, 64-bit
        division), 2 by tb (qm[2] = 0: tN >= 2^31) */

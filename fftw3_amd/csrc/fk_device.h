@@ -104,6 +104,19 @@ __device__ __forceinline__ Hoisted<F> hoisted(F f)
 {
     return Hoisted<F>{f};
 }
+/* A data source or sink that takes all of a thread's elements of the stage
+   at once: f(v), v[butterfly of the thread][element]. */
+template <class F>
+struct Whole {
+    F f;
+};
+template <class F>
+__device__ __forceinline__ Whole<F> whole(F f)
+{
+    return Whole<F>{f};
+}
+template <class T> struct is_whole : std::false_type {};
+template <class F> struct is_whole<Whole<F>> : std::true_type {};
 template <class T> struct is_hoisted : std::false_type {};
 template <class F> struct is_hoisted<Hoisted<F>> : std::true_type {};
 

@@ -60,6 +60,31 @@ struct At {
     __device__ __forceinline__ constexpr operator int() const { return b + OFF; }
 };
 
+template <class T>
+struct AtOff;
+template <int OFF, int ALIGN>
+struct AtOff<At<OFF, ALIGN>> {
+    static constexpr int v = OFF;
+};
+
+/* Butterfly I of a thread in a stage of NB butterflies over TPL threads:
+   u + I*TPL, or mirrored (needs NB a multiple of 2*TPL): the second half of
+   the thread's butterflies are the images b -> NB-1-b of the first, so that
+   a thread holds elements j and L-1-j of its line together. */
+template <int NB, int TPL, bool MIR>
+struct Bfly {
+    static constexpr int BPT = (NB + TPL - 1) / TPL;
+    static_assert(!MIR || NB % (2 * TPL) == 0, "mirrored mapping");
+    template <int I>
+    __device__ __forceinline__ static int at(int u)
+    {
+        if constexpr (MIR && I >= BPT / 2) return NB - 1 - u - (I - BPT / 2) * TPL;
+        else return u + I * TPL;
+    }
+    /* the index of the image of butterfly I */
+    static constexpr int image(int I) { return I < BPT / 2 ? I + BPT / 2 : I - BPT / 2; }
+};
+
 /* XL = 1 adds one scratch line for threads beyond TPL*NL (a persistent
    workgroup running a geometry smaller than itself). */
 template <typename R, int L, int TPL, int NL, int MODE, int PAD, int XL = 0>
@@ -183,20 +208,21 @@ struct PlainOut {
  * touch LDS, which decides the barriers.  pre / fin run on a butterfly's registers after the
  * loads / before the stores.
  */
-template <typename R, class RL, int S, int L, int TPL, bool IN_LDS, bool OUT_LDS,
-          class SY = SyncAll, class LoadF, class StoreF, class PreF, class FinF>
+template <typename R, class RL, int S, int L, int TPL, bool IN_LDS, bool OUT_LDS, bool MIR,
+          class SY, class LoadF, class StoreF, class PreF, class FinF>
 __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
                                       LoadF &&ld, StoreF &&st, const PreF &pre, const FinF &fin)
 {
     constexpr int Rs = RL::r[S];
     constexpr int Ns = RL::ns(S);
     constexpr int NB = L / Rs;
-    constexpr int BPT = (NB + TPL - 1) / TPL;
+    using BF = Bfly<NB, TPL, MIR>;
+    constexpr int BPT = BF::BPT;
     cx<R> v[BPT][Rs];
     auto load = [&](auto &&get) {
         sfor<0, BPT>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            const int b = u + i * TPL;
+            const int b = BF::template at<i>(u);
             if ((NB % TPL == 0) || b < NB) {
                 sfor<0, Rs>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
@@ -207,12 +233,13 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
     };
     typedef typename std::decay<LoadF>::type Ld;
     typedef typename std::decay<StoreF>::type St;
-    if constexpr (is_hoisted<Ld>::value) ld.f(load);
+    if constexpr (is_whole<Ld>::value) ld.f(v);
+    else if constexpr (is_hoisted<Ld>::value) ld.f(load);
     else load(ld);
     if constexpr (IN_LDS && OUT_LDS) SY::sync();
     sfor<0, BPT>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        const int b = u + i * TPL;
+        const int b = BF::template at<i>(u);
         if ((NB % TPL == 0) || b < NB) {
             /* the last stage has Ns = NB, so b < Ns there: its outputs are
                b + r*Ns, a compile-time offset from the thread's index */
@@ -236,18 +263,19 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
                 });
             };
             if constexpr (is_hoisted<St>::value) st.f(store);
-            else store(st);
+            else if constexpr (!is_whole<St>::value) store(st);
         }
     });
+    if constexpr (is_whole<St>::value) st.f(v);
     if constexpr (OUT_LDS) SY::sync();
 }
 
 /* Runs stages [S, RL::n) ; stage S loads with `first` (then `pre`), the last
    stage stores with `last` (after `fin`), everything between goes through
-   LDS. */
+   LDS.  M0 / ML: mirrored mapping of the first / last stage. */
 template <typename R, class RL, int S, int L, int TPL, bool FIRST_LDS,
-          bool LAST_LDS, class SY = SyncAll, class LdsF, class FirstF, class LastF,
-          class PreF = NoOp, class FinF = NoOp>
+          bool LAST_LDS, class SY = SyncAll, bool M0 = false, bool ML = false, class LdsF,
+          class FirstF, class LastF, class PreF = NoOp, class FinF = NoOp>
 __device__ __forceinline__ void run_stages(int u, const cx<R> *tw, LdsF &&lds,
                                            FirstF &&first, LastF &&last,
                                            const PreF &pre = PreF(), const FinF &fin = FinF())
@@ -256,17 +284,29 @@ __device__ __forceinline__ void run_stages(int u, const cx<R> *tw, LdsF &&lds,
     auto lds_ld = [&](auto j) { return lds(j); };
     auto lds_st = [&](auto k, cx<R> v) { lds(k) = v; };
     if constexpr (S == 0 && n == 1) {
-        stage<R, RL, 0, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, first, last, pre, fin);
+        static_assert(!M0 && !ML, "one-stage kernels are not mirrored");
+        stage<R, RL, 0, L, TPL, FIRST_LDS, LAST_LDS, false, SY>(u, tw, first, last, pre, fin);
     } else if constexpr (S == 0) {
-        stage<R, RL, 0, L, TPL, FIRST_LDS, true, SY>(u, tw, first, lds_st, pre, NoOp());
-        run_stages<R, RL, 1, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, lds, first, last, NoOp(), fin);
+        stage<R, RL, 0, L, TPL, FIRST_LDS, true, M0, SY>(u, tw, first, lds_st, pre, NoOp());
+        run_stages<R, RL, 1, L, TPL, FIRST_LDS, LAST_LDS, SY, M0, ML>(u, tw, lds, first, last, NoOp(),
+                                                                     fin);
     } else if constexpr (S == n - 1) {
-        stage<R, RL, S, L, TPL, true, LAST_LDS, SY>(u, tw, lds_ld, last, NoOp(), fin);
+        stage<R, RL, S, L, TPL, true, LAST_LDS, ML, SY>(u, tw, lds_ld, last, NoOp(), fin);
     } else {
-        stage<R, RL, S, L, TPL, true, true, SY>(u, tw, lds_ld, lds_st, NoOp(), NoOp());
-        run_stages<R, RL, S + 1, L, TPL, FIRST_LDS, LAST_LDS, SY>(u, tw, lds, first, last, NoOp(), fin);
+        stage<R, RL, S, L, TPL, true, true, false, SY>(u, tw, lds_ld, lds_st, NoOp(), NoOp());
+        run_stages<R, RL, S + 1, L, TPL, FIRST_LDS, LAST_LDS, SY, M0, ML>(u, tw, lds, first, last,
+                                                                         NoOp(), fin);
     }
 }
+
+/* whether the first / last stage of a kernel can run mirrored with whole
+   element pairs: an even radix and a multiple of 2*TPL butterflies */
+template <class RL, int TPL>
+struct MirOk {
+    static constexpr int L = RL::L(), R0 = RL::r[0], RN = RL::r[RL::n - 1];
+    static constexpr bool first = RL::n > 1 && R0 % 2 == 0 && (L / R0) % (2 * TPL) == 0;
+    static constexpr bool last = RL::n > 1 && RN % 2 == 0 && (L / RN) % (2 * TPL) == 0;
+};
 
 __device__ __forceinline__ long long remap_tile(unsigned xcd)
 {
@@ -405,27 +445,96 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
     } else if constexpr (IO == FK_IO_DCT4) {
         /* REDFT11 of n = 2L reals: z_m = (x_2m + i x_{n-1-2m}) exp(-i pi (4m+1) / 4n),
            Z = L-point DFT, c_p = Z_p exp(-i pi p / n), y_2p = 2 Re c_p,
-           y_{n-1-2p} = -2 Im c_p.  RODFT11_k(x) = (-1)^k REDFT11_k(x reversed). */
+           y_{n-1-2p} = -2 Im c_p.  RODFT11_k(x) = (-1)^k REDFT11_k(x reversed).
+           rtw holds the L input twiddles, then the L output twiddles.  The
+           sine kind's z_m is the cosine kind's with re and im swapped.  With
+           the mirrored mapping a thread has elements m and L-1-m, samples 2m,
+           2m+1 and n-2-2m, n-1-2m of the line on both sides: pairs of
+           neighbours (FK_REAL_UNIT: unit strides, pairs aligned). */
         const R *inr = reinterpret_cast<const R *>(a.in) + bin;
         R *outr = reinterpret_cast<R *>(a.out) + bout;
-        const cx<R> *rt = reinterpret_cast<const cx<R> *>(a.rtw);
+        const cx<R> *t0 = reinterpret_cast<const cx<R> *>(a.rtw), *t1 = t0 + L;
         const bool sn = a.rmode == FK_RM_DST4;
+        const long long is = a.is, os = a.os;
         constexpr long long N2 = 2LL * L;
-        auto gld = [&](int m) -> cx<R> {
-            if (!act) return mk((R)0, (R)0);
-            const long long q0 = 2LL * m, q1 = N2 - 1 - 2LL * m;
-            const R xa = inr[(sn ? N2 - 1 - q0 : q0) * a.is];
-            const R xb = inr[(sn ? N2 - 1 - q1 : q1) * a.is];
-            return mul(mk(xa, xb), rt[4 * m + 1]);
-        };
-        auto gst = [&](int p, cx<R> v) {
-            if (!act) return;
-            const cx<R> c = mul(v, rt[4 * p]);
-            const R ye = (R)2 * c.x, yo = (R)-2 * c.y;
-            outr[(2LL * p) * a.os] = ye;
-            outr[(N2 - 1 - 2LL * p) * a.os] = sn ? -yo : yo;
-        };
-        run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst);
+        constexpr int R0 = RL::r[0], NB0 = L / R0, RN = RL::r[RL::n - 1], NBN = L / RN;
+        constexpr bool M0 = MirOk<RL, TPL>::first, ML = MirOk<RL, TPL>::last;
+        using BF0 = Bfly<NB0, TPL, M0>;
+        using BFN = Bfly<NBN, TPL, ML>;
+        struct alignas(2 * sizeof(R)) P2 { R x, y; };
+        auto first = whole([&](auto &v) {
+            sfor<0, BF0::BPT>([&](auto ic) {
+                constexpr int i = decltype(ic)::value, im = M0 ? BF0::image(i) : i;
+                const int b = BF0::template at<i>(u);
+                if ((NB0 % TPL == 0) || b < NB0) {
+                    if (M0 && (fl & FK_REAL_UNIT)) {
+                        asm volatile("");
+                        const P2 *p = reinterpret_cast<const P2 *>(inr) + b;
+                        sfor<0, R0>([&](auto rc) {
+                            constexpr int r = decltype(rc)::value;
+                            const P2 x = ldg(Acc<C_ONCE>{}, p + r * NB0);
+                            v[i][r].x = x.x;
+                            v[im][R0 - 1 - r].y = x.y;
+                        });
+                    } else {
+                        const R *p = inr + 2 * b * is, *q = inr + (N2 - 1 - 2 * b) * is;
+                        sfor<0, R0>([&](auto rc) {
+                            constexpr int r = decltype(rc)::value;
+                            const long long o = (2LL * r * NB0) * is;
+                            v[i][r].x = p[o];
+                            v[i][r].y = q[-o];
+                        });
+                    }
+                }
+            });
+            sfor<0, BF0::BPT>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int b = BF0::template at<i>(u);
+                if ((NB0 % TPL == 0) || b < NB0) {
+                    swap_if<R0>(sn, v[i]);
+                    sfor<0, R0>([&](auto rc) {
+                        constexpr int r = decltype(rc)::value;
+                        v[i][r] = mul(v[i][r], t0[b + r * NB0]);
+                    });
+                }
+            });
+        });
+        auto last = whole([&](auto &v) {
+            sfor<0, BFN::BPT>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int b = BFN::template at<i>(u);
+                if ((NBN % TPL == 0) || b < NBN)
+                    sfor<0, RN>([&](auto rc) {
+                        constexpr int r = decltype(rc)::value;
+                        const cx<R> c = mul(v[i][r], t1[b + r * NBN]);
+                        const R yo = (R)-2 * c.y;
+                        v[i][r] = mk((R)2 * c.x, sn ? -yo : yo);
+                    });
+            });
+            sfor<0, BFN::BPT>([&](auto ic) {
+                constexpr int i = decltype(ic)::value, im = ML ? BFN::image(i) : i;
+                const int b = BFN::template at<i>(u);
+                if (act && ((NBN % TPL == 0) || b < NBN)) {
+                    if (ML && (fl & FK_REAL_UNIT)) {
+                        asm volatile("");
+                        P2 *p = reinterpret_cast<P2 *>(outr) + b;
+                        sfor<0, RN>([&](auto rc) {
+                            constexpr int r = decltype(rc)::value;
+                            p[r * NBN] = P2{v[i][r].x, v[im][RN - 1 - r].y};
+                        });
+                    } else {
+                        R *p = outr + 2 * b * os, *q = outr + (N2 - 1 - 2 * b) * os;
+                        sfor<0, RN>([&](auto rc) {
+                            constexpr int r = decltype(rc)::value;
+                            const long long o = (2LL * r * NBN) * os;
+                            p[o] = v[i][r].x;
+                            q[-o] = v[i][r].y;
+                        });
+                    }
+                }
+            });
+        });
+        run_stages<R, RL, 0, L, TPL, false, false, SY, M0, ML>(u, tw, lds_at, first, last);
     } else if constexpr (IO == FK_IO_R2C || IO == FK_IO_R2C_XR) {
         /* real line of 2L samples viewed as L complex z_j = x_2j + i x_2j+1;
            after the L-point DFT Z, X[k] = E[k] + W_2L^k O[k] with
@@ -704,349 +813,429 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         auto zld = [&](auto j) -> cx<R> { return lds_at(j); };
         run_stages<R, RL, 0, L, TPL, true, false, SY>(u, tw, lds_at, zld, gst);
     } else if constexpr (IO == FK_IO_R2C_RR) {
-        /* real line of 2L samples viewed as L complex z_j = x_2j + i x_2j+1;
-           after the L-point DFT Z, X[k] = E[k] + W_2L^k O[k] with
-           E = (Z[k] + conj Z[L-k])/2, O = (Z[k] - conj Z[L-k])/(2i),
-           k = 0..L (the role of rdft/ct-hc2c.c:197-210's HC2C_VIA_DFT). */
+        /* the real-to-real kinds that end in real outputs of an r2c of a line
+           of N2 = 2L samples: R2HC, DHT, REDFT10 / RODFT10 (the line read in
+           Makhoul's order) and REDFT00 / RODFT00 (the line read as its even /
+           odd extension).  These passes have several 4- or 8-byte accesses
+           and twiddles per element, so what bounds them is the latency and
+           the number of their memory instructions: the choice of the kind is
+           one branch around all loads and one around all stores, every
+           element's address is a thread base plus a uniform offset, and the
+           post-pass tables are read before the stages. */
         const R *inr = reinterpret_cast<const R *>(a.in) + bin;
-        cx<R> *out = reinterpret_cast<cx<R> *>(a.out);
         R *outr = reinterpret_cast<R *>(a.out) + bout;
         const cx<R> *wk = reinterpret_cast<const cx<R> *>(a.aux);
-        const cx<R> *rt = reinterpret_cast<const cx<R> *>(a.rtw);
-        /* fused real-to-real kind; a compile-time FK_RM_NONE in the plain
-           r2c / c2r instantiations */
-        const unsigned rm = (IO == FK_IO_R2C_RR || IO == FK_IO_C2R_RR) ? a.rmode : 0u;
+        const cx<R> *dt = reinterpret_cast<const cx<R> *>(a.rtw);
+        const unsigned rm = a.rmode;
+        const bool mak = rm == FK_RM_DCT2 || rm == FK_RM_DST2;
+        const bool ext = rm == FK_RM_E00 || rm == FK_RM_O00;
+        const long long is = a.is, os = a.os;
         constexpr long long N2 = 2LL * L;
-        /* REDFT10 / RODFT10 read the line reordered (Makhoul):
-           v_m = x_2m for m < L, x_{2(n-1-m)+1} above; the sine kind
-           negates the odd samples (RODFT10_k(x) = REDFT10_{n-1-k}((-1)^j x_j)) */
+        constexpr int R0 = RL::r[0], NB0 = L / R0;
+        constexpr bool M0 = MirOk<RL, TPL>::first;
+        using BF = Bfly<NB0, TPL, M0>;
+        constexpr int BPT = BF::BPT;
+        /* elements j = b + r*NB0 of butterfly b: f(i, r, b) for those in range */
+        auto each = [&](auto &&f) {
+            sfor<0, BPT>([&](auto ic) {
+                const int b = BF::template at<decltype(ic)::value>(u);
+                if ((NB0 % TPL == 0) || b < NB0) sfor<0, R0>([&](auto rc) { f(ic, rc, b); });
+            });
+        };
+        /* REDFT10 / RODFT10 read v_m = x_2m for m < L, x_{2(n-1-m)+1} above;
+           the sine kind negates the odd samples (RODFT10_k(x) =
+           REDFT10_{n-1-k}((-1)^j x_j)).  Samples 4j..4j+3 are elements j and
+           L-1-j: v_2j, v_{n-1-2j}, v_{2j+1}, v_{n-2-2j}. */
+        auto quads = [&](auto &v, auto &&quad) {
+            sfor<0, BPT>([&](auto ic) {
+                constexpr int i = decltype(ic)::value, im = BF::image(i);
+                const int b = BF::template at<i>(u);
+                sfor<0, R0 / 2>([&](auto rc) {
+                    constexpr int r = decltype(rc)::value;
+                    R q[4];
+                    quad(b, std::integral_constant<int, r * NB0>{}, q);
+                    v[i][r] = mk(q[0], q[2]);
+                    v[im][R0 - 1 - r] = mk(q[3], q[1]);
+                });
+            });
+        };
         auto vld = [&](int m) -> R {
             const long long q = m < L ? 2LL * m : 2 * (N2 - 1 - m) + 1;
-            const R v = inr[q * a.is];
-            return (rm == FK_RM_DST2 && m >= L) ? -v : v;
+            return inr[q * is];
         };
         /* REDFT00 / RODFT00 read the even extension x_0..x_{n-1},
            x_{n-2}..x_1 (n = L+1) or the odd one 0, x_0..x_{n-1}, 0,
            -x_{n-1}..-x_0 (n = L-1) of the line */
         auto eld = [&](long long m) -> R {
-            if (rm == FK_RM_E00) return inr[(m <= L ? m : N2 - m) * a.is];
+            if (rm == FK_RM_E00) return inr[(m <= L ? m : N2 - m) * is];
             if (m == 0 || m == L) return (R)0;
-            return m < L ? inr[(m - 1) * a.is] : -inr[(N2 - m - 1) * a.is];
+            return m < L ? inr[(m - 1) * is] : -inr[(N2 - m - 1) * is];
         };
-        auto gld = [&](int j) -> cx<R> {
-            if (!act) return mk((R)0, (R)0);
-            if constexpr (sizeof(R) == 4) {
-                /* v_2j, v_2j+1 are x_4j, x_4j+2 (first half) or x_{2n-4j-1},
-                   x_{2n-4j-3} (second half): one 16-byte quad each */
-                if ((rm == FK_RM_DCT2 || rm == FK_RM_DST2) && (fl & FK_REAL_QUAD)) {
-                    const float4 *q4 = reinterpret_cast<const float4 *>(inr);
-                    if (2 * j + 1 < L) {
-                        const float4 q = q4[j];
-                        return mk(q.x, q.z);
+        auto first = whole([&](auto &v) {
+            if (mak) {
+                asm volatile("");
+                if constexpr (M0) {
+                    if (fl & FK_REAL_QUAD) {
+                        asm volatile("");
+                        /* as pairs past L1 in FP32 (see FK_IO_R2C) */
+                        struct alignas(16) Q { R x[16 / sizeof(R)]; };
+                        auto fetch = [&](auto acc, auto *base) {
+                            typedef typename std::decay<decltype(*base)>::type T;
+                            constexpr int NT4 = 4 * sizeof(R) / sizeof(T), E = 4 / NT4;
+                            quads(v, [&](int b, auto oc, R *q) {
+                                const T *p = base + (b + decltype(oc)::value) * NT4;
+                                sfor<0, NT4>([&](auto hc) {
+                                    constexpr int h = decltype(hc)::value;
+                                    const T x = ldg(acc, p + h);
+                                    __builtin_memcpy(q + h * E, &x, sizeof(T));
+                                });
+                            });
+                        };
+                        if (nti) {
+                            asm volatile("");
+                            fetch(Acc<C_NT>{}, reinterpret_cast<const Q *>(inr));
+                        } else if constexpr (sizeof(R) == 4) {
+                            fetch(Acc<C_ONCE>{}, reinterpret_cast<const cx<R> *>(inr));
+                        } else {
+                            fetch(Acc<C_KEEP>{}, reinterpret_cast<const Q *>(inr));
+                        }
+                    } else {
+                        quads(v, [&](int b, auto oc, R *q) {
+                            const R *p = inr + 4 * b * is + (4LL * decltype(oc)::value) * is;
+                            q[0] = p[0];
+                            q[1] = p[is];
+                            q[2] = p[2 * is];
+                            q[3] = p[3 * is];
+                        });
                     }
-                    if (2 * j >= L) {
-                        const float4 q = q4[L - 1 - j];
-                        return rm == FK_RM_DST2 ? mk(-q.w, -q.y) : mk(q.w, q.y);
-                    }
+                } else {
+                    each([&](auto ic, auto rc, int b) {
+                        const int j = b + decltype(rc)::value * NB0;
+                        v[decltype(ic)::value][decltype(rc)::value] = mk(vld(2 * j), vld(2 * j + 1));
+                    });
                 }
+                if (rm == FK_RM_DST2) {
+                    asm volatile("");
+                    each([&](auto ic, auto rc, int b) {
+                        constexpr int r = decltype(rc)::value;
+                        cx<R> &x = v[decltype(ic)::value][r];
+                        const int j = b + r * NB0;
+                        if (R0 % 2 ? 2 * j >= L : 2 * r >= R0) x.x = -x.x;
+                        if (R0 % 2 ? 2 * j + 1 >= L : 2 * r >= R0) x.y = -x.y;
+                    });
+                }
+            } else if (ext) {
+                asm volatile("");
+                each([&](auto ic, auto rc, int b) {
+                    constexpr int r = decltype(rc)::value;
+                    cx<R> &x = v[decltype(ic)::value][r];
+                    const int j = b + r * NB0;
+                    if constexpr (R0 % 2 == 0 && r != 0 && 2 * r != R0) {
+                        /* inside one half of the extension */
+                        const long long sg = 2 * r < R0 ? is : -is;
+                        const R *p = 2 * r < R0 ? inr + 2 * j * is - (rm == FK_RM_E00 ? 0 : is)
+                                                : inr + (N2 - 2 * j) * is - (rm == FK_RM_E00 ? 0 : is);
+                        x = mk(p[0], p[sg]);
+                        if (2 * r > R0 && rm == FK_RM_O00) x = mk(-x.x, -x.y);
+                    } else {
+                        x = mk(eld(2 * j), eld(2 * j + 1));
+                    }
+                });
+            } else if (fl & FK_REAL_UNIT) {
+                each([&](auto ic, auto rc, int b) {
+                    constexpr int r = decltype(rc)::value;
+                    v[decltype(ic)::value][r] =
+                        ldg(Acc<C_ONCE>{}, reinterpret_cast<const cx<R> *>(inr) + b + r * NB0);
+                });
+            } else {
+                asm volatile("");
+                each([&](auto ic, auto rc, int b) {
+                    constexpr int r = decltype(rc)::value;
+                    const R *p = inr + 2 * b * is + (2LL * r * NB0) * is;
+                    v[decltype(ic)::value][r] = mk(p[0], p[is]);
+                });
             }
-            if (rm == FK_RM_DCT2 || rm == FK_RM_DST2) return mk(vld(2 * j), vld(2 * j + 1));
-            if (rm == FK_RM_E00 || rm == FK_RM_O00) return mk(eld(2 * j), eld(2 * j + 1));
-            if (fl & FK_REAL_UNIT) return reinterpret_cast<const cx<R> *>(inr)[j];
-            return mk(inr[(2 * j) * a.is], inr[(2 * j + 1) * a.is]);
-        };
+        });
         auto lst = [&](auto k, cx<R> v) { lds_at(k) = v; };
-        /* bin k <= L/2 gives bins k and L-k from the same Z[k], Z[L-k] and
-           one twiddle (W_2L^(L-k) = -conj W_2L^k); bins k = u + i*TPL in
-           groups of 8 (compile-time count): the group's twiddle loads are
-           in flight together */
+        /* bins k = u + i*TPL <= L/2, with L-k: one table entry each, two for
+           REDFT10 / RODFT10 (dt: exp(-i pi k / 2n) and that times W_n^k) */
         constexpr int HK = L / 2;
         constexpr int NK2 = (HK + 1 + TPL - 1) / TPL;
-        constexpr int GK = 8;
-        constexpr bool XR = IO == FK_IO_R2C_XR;
-        /* few bins per thread: their twiddles are loaded before the stages,
-           so the load latency hides behind the FFT instead of following it */
-        constexpr bool PRE = NK2 <= 20;
-        cx<R> wpre[PRE ? NK2 : 1];
-        if constexpr (PRE) {
-            sfor<0, NK2>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                const int k = u + i * TPL;
-                wpre[i] = wk[k <= HK ? k : HK];
-            });
-        }
-        /* cross-row form: twiddles of the first column stage, W_n0^(n1*p)
-           (n1 = the tile's line-group index, uniform over the workgroup) */
-        cx<R> wp[XR ? NL : 1];
-        if constexpr (XR) {
-            const long long n1 = line_ix(a, tile * NL).i1;
-            sfor<0, NL>([&](auto pc) {
-                constexpr int pp = decltype(pc)::value;
-                wp[pp] = pp == 0 ? mk((R)1, (R)0) : tw2<R>(a, n1 * pp);
-            });
-        }
-        run_stages<R, RL, 0, L, TPL, false, true, SY>(u, tw, lds_at, gld, lst);
-        /* cross-row form: the bins stay in registers until every bin of the
-           line has been formed, then replace Z in the line's LDS row */
-        cx<R> xs[XR ? 2 * NK2 : 1];
-        constexpr long long NONE = -0x7fffffffffffffffLL - 1; /* INT64_MIN */
-        if constexpr (XR) {
-            if (u == 0 && real) lbase[lt] = act ? bout : NONE;
-        }
-        /* bin k's outputs: the complex bin, or the real outputs of the
-           fused real-to-real kind */
-        auto emit = [&](int k, cx<R> X) {
-            if (act && rm == FK_RM_NONE) {
-                out[bout + (long long)k * a.os] = X;
-            } else if (act && rm == FK_RM_E00) {
-                outr[(long long)k * a.os] = X.x;             /* DCT-I: Re X_k */
-            } else if (act && rm == FK_RM_O00) {
-                if (k >= 1 && k < L) outr[(long long)(k - 1) * a.os] = -X.y; /* DST-I */
-            } else if (act) {
-                /* bin k gives two real outputs, k and n-k:
-                   R2HC r_k / i_k; DHT Re -+ Im; REDFT10
-                   c = exp(-i pi k / 2n) X: 2 Re c, -2 Im c */
-                R lo, hi;
-                if (rm == FK_RM_HC) {
-                    lo = X.x;
-                    hi = X.y;
-                } else if (rm == FK_RM_DHT) {
-                    lo = X.x - X.y;
-                    hi = X.x + X.y;
-                } else {
-                    const cx<R> c = mul(X, rt[2 * k]);
-                    lo = (R)2 * c.x;
-                    hi = (R)-2 * c.y;
-                }
-                long long ka = k, kb = N2 - k;
-                if (rm == FK_RM_DST2) {
-                    ka = N2 - 1 - k;
-                    kb = k - 1;
-                }
-                outr[ka * a.os] = lo;
-                if (k != 0 && k != L) outr[kb * a.os] = hi;
+        constexpr bool PRE = NK2 * sizeof(R) <= 48;
+        constexpr int GK = PRE ? NK2 : 4;
+        struct alignas(2 * sizeof(cx<R>)) W2 { cx<R> a, b; };
+        W2 w[GK];
+        auto tables = [&](auto gc) {
+            if (mak) {
+                asm volatile("");
+                sfor<0, GK>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (decltype(gc)::value * GK + i) * TPL;
+                    w[i] = reinterpret_cast<const W2 *>(dt)[k <= HK ? k : HK];
+                });
+            } else {
+                sfor<0, GK>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (decltype(gc)::value * GK + i) * TPL;
+                    w[i].a = wk[k <= HK ? k : HK];
+                });
             }
         };
-        sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
-            constexpr int g = decltype(gc)::value;
-            constexpr int cnt = (NK2 - g * GK) < GK ? (NK2 - g * GK) : GK;
-            cx<R> w[cnt];
-            sfor<0, cnt>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                const int k = u + (g * GK + i) * TPL;
-                if constexpr (PRE) w[i] = wpre[g * GK + i];
-                else if (k <= HK) w[i] = wk[k];
-            });
-            sfor<0, cnt>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                const int k = u + (g * GK + i) * TPL;
-                if (k <= HK) {
-                    const cx<R> zk = lds_at(k);
-                    const cx<R> zc = lds_at(k == 0 ? 0 : L - k);
-                    const R er = (R)0.5 * (zk.x + zc.x), ei = (R)0.5 * (zk.y - zc.y);
-                    /* O = (Z[k] - conj Z[L-k]) / (2i) */
-                    const R orr = (R)0.5 * (zk.y + zc.y), oi = (R)-0.5 * (zk.x - zc.x);
-                    const R wx = w[i].x, wy = w[i].y;
-                    /* X[k] = E + W O; X[L-k] = conj(E - W O), written as the
-                       form of bin L-k on its own (E' = conj E, O' = conj O,
-                       W' = -conj W) so that both round as that form does */
-                    const cx<R> X = mk(er + orr * wx - oi * wy, ei + orr * wy + oi * wx);
-                    const cx<R> Y = mk(er + orr * (-wx) - (-oi) * wy, (-ei) + orr * wy + (-oi) * (-wx));
-                    if constexpr (XR) {
-                        xs[2 * (g * GK + i)] = X;
-                        xs[2 * (g * GK + i) + 1] = Y;
-                    } else {
-                        emit(k, X);
-                        if (2 * k != L) emit(L - k, Y);
-                    }
-                }
-            });
-        });
-        if constexpr (XR) {
-            /* every thread of the line has read Z: the bins replace it */
-            SY::sync();
-            sfor<0, NK2>([&](auto ic) {
-                constexpr int i = decltype(ic)::value;
+        if constexpr (PRE) tables(std::integral_constant<int, 0>{});
+        run_stages<R, RL, 0, L, TPL, false, true, SY, M0>(u, tw, lds_at, first, lst);
+        /* f(d, k, Z[k], Z[L-k], tables) with d = k - u a compile-time constant */
+        auto bins = [&](auto gc, auto &&f) {
+            sfor<0, GK>([&](auto ic) {
+                constexpr int i = decltype(gc)::value * GK + decltype(ic)::value;
                 const int k = u + i * TPL;
-                if (k <= HK) {
-                    lds_at(k) = xs[2 * i];
-                    if (2 * k != L) lds_at(L - k) = xs[2 * i + 1];
-                }
+                if (act && i < NK2 && k <= HK)
+                    f(std::integral_constant<int, i * TPL>{}, k, (cx<R>)lds_at(k),
+                      (cx<R>)lds_at(k == 0 ? 0 : L - k), w[decltype(ic)::value]);
             });
-            __syncthreads();
-            /* first stage of the column DFT over the tile's NL rows
-               n = n1 + m*n2 (n2 = the line's batch index i0, n1 = i1; the
-               planner sets nb[0] = NL, so a tile is one n1): for every bin k
-               y_p = W_n0^(n1*p) sum_n2 X_n2[k] W_NL^(n2*p), n0 = a.tN,
-               stored to the tile's output line p */
-            for (int k = tid; k <= L; k += NT) {
-                cx<R> v[NL];
-                sfor<0, NL>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    v[q] = lds[G::idx(q, k)];
+        };
+        /* X[k] = E + W O and X[L-k] = conj(E - W O), both rounding as the
+           form of a bin on its own */
+        auto XY = [&](cx<R> zk, cx<R> zc, cx<R> wv, cx<R> &X, cx<R> &Y) {
+            const R er = (R)0.5 * (zk.x + zc.x), ei = (R)0.5 * (zk.y - zc.y);
+            const R orr = (R)0.5 * (zk.y + zc.y), oi = (R)-0.5 * (zk.x - zc.x);
+            X = mk(er + orr * wv.x - oi * wv.y, ei + orr * wv.y + oi * wv.x);
+            Y = mk(er + orr * (-wv.x) - (-oi) * wv.y, (-ei) + orr * wv.y + (-oi) * (-wv.x));
+        };
+        /* outputs k, n-k, L-k, L+k (one lower for the sine kinds' mirror) */
+        R *pk = outr + u * os, *pn = outr + (N2 - u) * os;
+        R *pm = outr + (L - u) * os, *pp = outr + (L + u) * os;
+        sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
+            if constexpr (!PRE) tables(gc);
+            if (mak) {
+                /* c_k = exp(-i pi k / 2n) X_k: with t that factor, A = 2 t E
+                   and B = 2 t W O, 2 c_k = A + B and, as exp(-i pi (L-k) / 2n)
+                   = exp(-i pi / 4) conj t, 2 c_{L-k} = exp(-i pi / 4)
+                   conj(A - B).  REDFT10: y_k = 2 Re c_k, y_{n-k} = -2 Im c_k;
+                   RODFT10: the same reversed. */
+                asm volatile("");
+                const bool sn = rm == FK_RM_DST2;
+                const long long st = sn ? -os : os;
+                R *qk = sn ? outr + (N2 - 1 - u) * os : pk, *qn = sn ? pk - os : pn;
+                R *qm = sn ? pp - os : pm, *qp = sn ? pm - os : pp;
+                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, W2 t) {
+                    constexpr R h = (R)0.70710678118654752440084436210484903928;
+                    const long long d = (long long)decltype(dc)::value * st;
+                    const cx<R> A = mul(t.a, mk(zk.x + zc.x, zk.y - zc.y));
+                    const cx<R> B = mul(t.b, mk(zk.y + zc.y, zc.x - zk.x));
+                    const cx<R> D = sub(A, B);
+                    qk[d] = A.x + B.x;
+                    if (k != 0) qn[-d] = -(A.y + B.y);
+                    if (2 * k != L) {
+                        qm[-d] = (D.x - D.y) * h;
+                        if (k != 0) qp[d] = (D.x + D.y) * h;
+                    }
                 });
-                Dft<R, NL, 1>::run(v);
-                sfor<0, NL>([&](auto pc) {
-                    constexpr int pp = decltype(pc)::value;
-                    const long long ob = lbase[pp];
-                    if (ob != NONE) out[ob + (long long)k * a.os] = pp == 0 ? v[0] : mul(v[pp], wp[pp]);
+            } else if (ext) {
+                /* DCT-I: Re X_k; DST-I: -Im X_k, one place lower */
+                asm volatile("");
+                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, W2 t) {
+                    const long long d = (long long)decltype(dc)::value * os;
+                    cx<R> X, Y;
+                    XY(zk, zc, t.a, X, Y);
+                    if (rm == FK_RM_E00) {
+                        pk[d] = X.x;
+                        if (2 * k != L) pm[-d] = Y.x;
+                    } else if (k != 0) {
+                        pk[d - os] = -X.y;
+                        if (2 * k != L) pm[-d - os] = -Y.y;
+                    }
+                });
+            } else {
+                /* R2HC: r_k, i_k; DHT: Re - Im, Re + Im, at k and n-k */
+                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, W2 t) {
+                    const long long d = (long long)decltype(dc)::value * os;
+                    cx<R> X, Y;
+                    XY(zk, zc, t.a, X, Y);
+                    if (rm == FK_RM_DHT) {
+                        X = mk(X.x - X.y, X.x + X.y);
+                        Y = mk(Y.x - Y.y, Y.x + Y.y);
+                    }
+                    pk[d] = X.x;
+                    if (k != 0) pn[-d] = X.y;
+                    if (2 * k != L) {
+                        pm[-d] = Y.x;
+                        if (k != 0) pp[d] = Y.y;
+                    }
                 });
             }
-        }
+        });
     } else if constexpr (IO == FK_IO_C2R_RR) {
-        /* half-length inverse: Z[k] = E[k] + i O[k],
-           E[k] = X[k] + conj X[L-k], O[k] = (X[k] - conj X[L-k]) W_2L^-k,
-           z = DFT^-1_L(Z) (unnormalized), y_2m = Re z_m, y_2m+1 = Im z_m.
-           Im X[0] and Im X[L] are ignored, as the r2cb codelets do. */
-        const cx<R> *in = reinterpret_cast<const cx<R> *>(a.in) + bin;
+        /* the real-to-real kinds that begin with real inputs of a c2r: HC2R
+           (bins r_k, i_k from the halfcomplex line), REDFT01 / RODFT01 (bins
+           V_k = exp(+i pi k / 2n)(x_k - i x_{n-k}), the sine kind on the
+           reversed line; outputs y_2i = v_i, y_2i+1 = v_{n-1-i}, the sine
+           kind's odd ones negated).  Bounded as the kinds above. */
         const R *inr = reinterpret_cast<const R *>(a.in) + bin;
         R *outr = reinterpret_cast<R *>(a.out) + bout;
         const cx<R> *wk = reinterpret_cast<const cx<R> *>(a.aux);
-        const cx<R> *rt = reinterpret_cast<const cx<R> *>(a.rtw);
-        /* fused real-to-real kind; a compile-time FK_RM_NONE in the plain
-           r2c / c2r instantiations */
-        const unsigned rm = (IO == FK_IO_R2C_RR || IO == FK_IO_C2R_RR) ? a.rmode : 0u;
+        const cx<R> *dt = reinterpret_cast<const cx<R> *>(a.rtw);
+        const bool hc = a.rmode == FK_RM_HC2R, sn = a.rmode == FK_RM_DST3;
+        const long long is = a.is, os = a.os;
         constexpr long long N2 = 2LL * L;
-        /* bin k of the fused real-to-real kinds: HC2R reads (r_k, i_k) from
-           the halfcomplex line; REDFT01 forms exp(+i pi k / 2n)(x_k - i x_{n-k})
-           (x_n = 0), RODFT01 the same on the reversed line */
-        auto rbin = [&](int k) -> cx<R> {
-            if (rm == FK_RM_HC2R)
-                return mk(inr[(long long)k * a.is],
-                          (k == 0 || k == L) ? (R)0 : inr[(N2 - k) * a.is]);
-            const bool s = rm == FK_RM_DST3;
-            const long long q0 = s ? N2 - 1 - k : k, q1 = s ? k - 1 : N2 - k;
-            const R xk = inr[q0 * a.is];
-            const R xn = k == 0 ? (R)0 : inr[q1 * a.is];
-            const cx<R> w = rt[2 * k];
-            return mk(w.x * xk - w.y * xn, -(w.x * xn + w.y * xk));
-        };
-        /* bins X[k], X[L-k] (k <= L/2) are read together and give Z[k] and
-           Z[L-k] with one twiddle (W_2L^(L-k) = -conj W_2L^k); they are
-           written to LDS before the stages, which read Z as it is */
         constexpr int HK = L / 2;
         constexpr int NK2 = (HK + 1 + TPL - 1) / TPL;
-        constexpr int GK = 8;
-        /* swapped Z (the backward DFT runs as the forward one on swapped
-           data): e = X[k] + conj X[L-k], d = X[k] - conj X[L-k],
-           o = d conj(W_2L^k); Z[k] = e + i o and, by the symmetry above,
-           Z[L-k] = conj e + i conj o */
-        auto zpair = [&](cx<R> xk, cx<R> xc, cx<R> w, cx<R> &z0, cx<R> &z1) {
-            const cx<R> e = mk(xk.x + xc.x, xk.y - xc.y);
-            const cx<R> d = mk(xk.x - xc.x, xk.y + xc.y);
-            const cx<R> o = mk(d.x * w.x + d.y * w.y, d.y * w.x - d.x * w.y);
-            z0 = mk(e.y + o.x, e.x - o.y);
-            z1 = mk(o.x - e.y, e.x + o.y);
-        };
-        if constexpr (IO == FK_IO_C2R_XR) {
-            /* last stage of the inverse column DFT over the tile's NL input
-               rows (row p = the line's batch index i0, n1 = i1; the planner
-               sets nb[0] = NL, so a tile is one n1): for every bin k
-               u_n2 = sum_p W_NL^(-n2*p) W_n0^(-n1*p) Y_p[k], n0 = a.tN,
-               which is line n2's half spectrum (its own output row) */
-            constexpr long long NONE = -0x7fffffffffffffffLL - 1; /* INT64_MIN */
-            if (u == 0 && real) lbase[lt] = act ? bin : NONE;
-            const long long n1 = line_ix(a, tile * NL).i1;
-            cx<R> wp[NL];
-            sfor<0, NL>([&](auto pc) {
-                constexpr int pp = decltype(pc)::value;
-                const cx<R> t = pp == 0 ? mk((R)1, (R)0) : tw2<R>(a, n1 * pp);
-                wp[pp] = mk(t.x, -t.y);
-            });
-            __syncthreads();
-            const cx<R> *inb = reinterpret_cast<const cx<R> *>(a.in);
-            /* bin k of every row of the tile: inverse DFT through the
-               forward one on swapped data */
-            auto coldft = [&](int k, cx<R> *v) {
-                sfor<0, NL>([&](auto pc) {
-                    constexpr int pp = decltype(pc)::value;
-                    const long long ib = lbase[pp];
-                    const cx<R> y = ib != NONE ? inb[ib + (long long)k * a.is] : mk((R)0, (R)0);
-                    v[pp] = swp(pp == 0 ? y : mul(y, wp[pp]));
-                });
-                Dft<R, NL, 1>::run(v);
-            };
-            for (int k = tid; k <= HK; k += NT) {
-                const cx<R> w = wk[k];
-                cx<R> v[NL], vm[NL];
-                coldft(k, v);
-                if (2 * k != L) coldft(L - k, vm);
-                sfor<0, NL>([&](auto qc) {
-                    constexpr int q = decltype(qc)::value;
-                    cx<R> xk = swp(v[q]);
-                    cx<R> xc = 2 * k == L ? xk : swp(vm[q]);
-                    if (k == 0) {
-                        xk.y = 0;
-                        xc.y = 0;
-                    }
-                    cx<R> z0, z1;
-                    zpair(xk, xc, w, z0, z1);
-                    lds[G::idx(q, k)] = z0;
-                    if (k != 0 && 2 * k != L) lds[G::idx(q, L - k)] = z1;
-                });
-            }
-            __syncthreads();
-        } else {
-            /* loads in groups of 8 (compile-time count) so that each group
-               is in flight at once, then its LDS stores */
-            sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
-                constexpr int g = decltype(gc)::value;
-                constexpr int cnt = (NK2 - g * GK) < GK ? (NK2 - g * GK) : GK;
-                cx<R> xa[cnt], xb[cnt], w[cnt];
-                sfor<0, cnt>([&](auto ic) {
-                    constexpr int i = decltype(ic)::value;
-                    const int k = u + (g * GK + i) * TPL;
-                    if (k <= HK) {
-                        xa[i] = !act ? mk((R)0, (R)0)
-                                : rm == FK_RM_NONE ? in[(long long)k * a.is] : rbin(k);
-                        xb[i] = !act ? mk((R)0, (R)0)
-                                : rm == FK_RM_NONE ? in[(long long)(L - k) * a.is] : rbin(L - k);
-                        w[i] = wk[k];
-                    }
-                });
-                sfor<0, cnt>([&](auto ic) {
-                    constexpr int i = decltype(ic)::value;
-                    const int k = u + (g * GK + i) * TPL;
-                    if (k <= HK) {
-                        cx<R> xk = xa[i], xc = xb[i];
-                        if (k == 0) {
-                            xk.y = 0;
-                            xc.y = 0;
-                        }
-                        cx<R> z0, z1;
-                        zpair(xk, xc, w[i], z0, z1);
-                        lds_at(k) = z0;
-                        if (k != 0 && 2 * k != L) lds_at(L - k) = z1;
-                    }
-                });
-            });
-            SY::sync();
-        }
-        auto gst = [&](int k, cx<R> v) {
-            /* v = swap(z_k) */
-            if (!act) return;
-            if (rm == FK_RM_DCT3 || rm == FK_RM_DST3) {
-                /* y_2i = v_i (i < L), y_{2i+1} = v_{n-1-i}: v_m goes to 2m
-                   below L, to 2(n-1-m)+1 above; RODFT01 negates odd outputs */
-                const long long m0 = 2LL * k, m1 = 2LL * k + 1;
-                const long long d0 = m0 < L ? 2 * m0 : 2 * (N2 - 1 - m0) + 1;
-                const long long d1 = m1 < L ? 2 * m1 : 2 * (N2 - 1 - m1) + 1;
-                R y0 = v.y, y1 = v.x;
-                if (rm == FK_RM_DST3) {
-                    if (d0 & 1) y0 = -y0;
-                    if (d1 & 1) y1 = -y1;
+        constexpr int GK = sizeof(R) == 4 ? 6 : 4;
+        struct alignas(2 * sizeof(cx<R>)) W2 { cx<R> a, b; };
+        /* samples k, n-k, L-k, L+k of the line (reversed for RODFT01) */
+        const long long st = sn ? -is : is, o = sn ? N2 - 1 : 0;
+        const R *pk = inr + o * is + u * st, *pn = inr + o * is + (N2 - u) * st;
+        const R *pm = inr + o * is + (L - u) * st, *pp = inr + o * is + (L + u) * st;
+        sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
+            constexpr int g = decltype(gc)::value;
+            constexpr int cnt = (NK2 - g * GK) < GK ? (NK2 - g * GK) : GK;
+            R xk[cnt], xn[cnt], xm[cnt], xp[cnt];
+            W2 w[cnt];
+            sfor<0, cnt>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int k = u + (g * GK + i) * TPL;
+                const long long d = (long long)((g * GK + i) * TPL) * st;
+                if (k <= HK) {
+                    xk[i] = pk[d];
+                    xn[i] = k == 0 ? (R)0 : pn[-d];
+                    xm[i] = pm[-d];
+                    xp[i] = pp[d];
                 }
-                outr[d0 * a.os] = y0;
-                outr[d1 * a.os] = y1;
-            } else if (fl & FK_REAL_UNIT) {
-                reinterpret_cast<cx<R> *>(outr)[k] = mk(v.y, v.x);
+            });
+            if (hc) {
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    w[i].a = wk[k <= HK ? k : HK];
+                });
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    if (k <= HK) {
+                        /* X[k] = (x_k, x_{n-k}), X[L-k] = (x_{L-k}, x_{L+k});
+                           Im X[0] = Im X[L] = 0.  As in FK_IO_C2R, swapped:
+                           e = X[k] + conj X[L-k], o = (X[k] - conj X[L-k])
+                           conj(W_n^k), Z[k] = e + i o, Z[L-k] = conj e + i conj o */
+                        const R ck = xn[i], cm = k == 0 ? (R)0 : xp[i];
+                        const cx<R> e = mk(xk[i] + xm[i], ck - cm);
+                        const cx<R> dd = mk(xk[i] - xm[i], ck + cm), t = w[i].a;
+                        const cx<R> oo = mk(dd.x * t.x + dd.y * t.y, dd.y * t.x - dd.x * t.y);
+                        lds_at(k) = mk(e.y + oo.x, e.x - oo.y);
+                        if (k != 0 && 2 * k != L) lds_at(L - k) = mk(oo.x - e.y, e.x + oo.y);
+                    }
+                });
             } else {
-                outr[(2 * k) * a.os] = v.y;
-                outr[(2 * k + 1) * a.os] = v.x;
+                asm volatile("");
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int k = u + (g * GK + i) * TPL;
+                    w[i] = reinterpret_cast<const W2 *>(dt)[k <= HK ? k : HK];
+                });
+                sfor<0, cnt>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    constexpr R h = (R)0.70710678118654752440084436210484903928;
+                    const int k = u + (g * GK + i) * TPL;
+                    if (k <= HK) {
+                        /* with t = exp(-i pi k / 2n): V_k = conj(t) p,
+                           p = x_k - i x_{n-k}, and conj V_{L-k} = conj(t) q,
+                           q = exp(-i pi / 4)(x_{L-k} + i x_{L+k}); so
+                           e = conj(t)(p + q), o = conj(t W_n^k)(p - q) */
+                        const cx<R> q = mk((xm[i] + xp[i]) * h, (xp[i] - xm[i]) * h);
+                        const cx<R> s_ = mk(xk[i] + q.x, q.y - xn[i]);
+                        const cx<R> f = mk(xk[i] - q.x, -xn[i] - q.y);
+                        const cx<R> t = w[i].a, t2 = w[i].b;
+                        const cx<R> e = mk(s_.x * t.x + s_.y * t.y, s_.y * t.x - s_.x * t.y);
+                        const cx<R> oo = mk(f.x * t2.x + f.y * t2.y, f.y * t2.x - f.x * t2.y);
+                        lds_at(k) = mk(e.y + oo.x, e.x - oo.y);
+                        if (k != 0 && 2 * k != L) lds_at(L - k) = mk(oo.x - e.y, e.x + oo.y);
+                    }
+                });
             }
-        };
+        });
+        SY::sync();
+        constexpr int RN = RL::r[RL::n - 1], NBN = L / RN;
+        constexpr bool ML = MirOk<RL, TPL>::last;
+        using BF = Bfly<NBN, TPL, ML>;
+        constexpr int BPT = BF::BPT;
+        /* v = swap(z_k): (v_2k+1, v_2k) */
+        auto last = whole([&](auto &v) {
+            auto each = [&](auto &&f) {
+                sfor<0, BPT>([&](auto ic) {
+                    const int b = BF::template at<decltype(ic)::value>(u);
+                    if (act && ((NBN % TPL == 0) || b < NBN))
+                        sfor<0, RN>([&](auto rc) {
+                            constexpr int r = decltype(rc)::value;
+                            f(b, std::integral_constant<int, r * NBN>{}, v[decltype(ic)::value][r]);
+                        });
+                });
+            };
+            if (!hc) {
+                asm volatile("");
+                if constexpr (ML) {
+                    /* elements k and L-1-k are outputs 4k..4k+3 */
+                    auto quads = [&](auto &&quad) {
+                        if (act)
+                            sfor<0, BPT>([&](auto ic) {
+                                constexpr int i = decltype(ic)::value, im = BF::image(i);
+                                const int b = BF::template at<i>(u);
+                                sfor<0, RN / 2>([&](auto rc) {
+                                    constexpr int r = decltype(rc)::value;
+                                    const cx<R> x = v[i][r], y = v[im][RN - 1 - r];
+                                    const R y1 = sn ? -y.x : y.x, y3 = sn ? -y.y : y.y;
+                                    const R q[4] = {x.y, y1, x.x, y3};
+                                    quad(b, std::integral_constant<int, r * NBN>{}, q);
+                                });
+                            });
+                    };
+                    if (fl & FK_REAL_QUAD) {
+                        asm volatile("");
+                        struct alignas(16) Q { R x[16 / sizeof(R)]; };
+                        constexpr int NQ = sizeof(R) / 4;
+                        Q *q4 = reinterpret_cast<Q *>(outr);
+                        quads([&](int b, auto oc, const R *q) {
+                            Q *p = q4 + (b + decltype(oc)::value) * NQ;
+                            sfor<0, NQ>([&](auto hc_) {
+                                constexpr int hh = decltype(hc_)::value;
+                                Q x;
+                                sfor<0, 4 / NQ>([&](auto ec) {
+                                    constexpr int e = decltype(ec)::value;
+                                    x.x[e] = q[hh * (4 / NQ) + e];
+                                });
+                                p[hh] = x;
+                            });
+                        });
+                    } else {
+                        quads([&](int b, auto oc, const R *q) {
+                            R *p = outr + 4 * b * os + (4LL * decltype(oc)::value) * os;
+                            p[0] = q[0];
+                            p[os] = q[1];
+                            p[2 * os] = q[2];
+                            p[3 * os] = q[3];
+                        });
+                    }
+                } else {
+                    each([&](int b, auto oc, cx<R> x) {
+                        const long long m0 = 2LL * (b + decltype(oc)::value), m1 = m0 + 1;
+                        const long long d0 = m0 < L ? 2 * m0 : 2 * (N2 - 1 - m0) + 1;
+                        const long long d1 = m1 < L ? 2 * m1 : 2 * (N2 - 1 - m1) + 1;
+                        outr[d0 * os] = (sn && (d0 & 1)) ? -x.y : x.y;
+                        outr[d1 * os] = (sn && (d1 & 1)) ? -x.x : x.x;
+                    });
+                }
+            } else if (fl & FK_REAL_UNIT) {
+                each([&](int b, auto oc, cx<R> x) {
+                    reinterpret_cast<cx<R> *>(outr)[b + decltype(oc)::value] = mk(x.y, x.x);
+                });
+            } else {
+                asm volatile("");
+                each([&](int b, auto oc, cx<R> x) {
+                    R *p = outr + 2 * b * os + (2LL * decltype(oc)::value) * os;
+                    p[0] = x.y;
+                    p[os] = x.x;
+                });
+            }
+        });
         auto zld = [&](auto j) -> cx<R> { return lds_at(j); };
-        run_stages<R, RL, 0, L, TPL, true, false, SY>(u, tw, lds_at, zld, gst);
+        run_stages<R, RL, 0, L, TPL, true, false, SY, false, ML>(u, tw, lds_at, zld, last);
     } else if constexpr (IO == FK_IO_BLUE) {
         /* Bluestein (dft/bluestein.c:82-128 conventions): a_j = x_j c_j,
            c_j = exp(-i pi j^2/n); conv = IDFT_L(DFT_L(a) * B),
@@ -1086,13 +1275,6 @@ stockham(fk_args a)
     stockham_body<R, NL, MODE, IO, PAD, RL, TPL, TPL * NL, SY>(a, remap_tile(a.xcd_remap),
                                                                smem_raw);
 }
-
-template <class T>
-struct AtOff;
-template <int OFF, int ALIGN>
-struct AtOff<At<OFF, ALIGN>> {
-    static constexpr int v = OFF;
-};
 
 /*
  * Row-mapped plain pass with one stage-0 butterfly per thread (L / R0 =

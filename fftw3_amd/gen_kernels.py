@@ -66,12 +66,36 @@ def choose_radices(n):
     return fs[0]
 
 
-def geometry(prec, L, rads, mode, io, tpl_div=1, nl_mul=1.0):
+def mirrored_radices(L, points=16):
+    """Radices and threads per line of the fused real-to-real kernels: each
+    thread holds `points` elements, and the first and last radix are even and
+    divide points / 2, so that both stages can run mirrored (a thread then has
+    elements j and L-1-j, whose samples are neighbours).  None if L has no
+    such factorization."""
+    if L % points:
+        return None
+    ends = [r for r in RADICES if r % 2 == 0 and (points // 2) % r == 0]
+    best = None
+    for r0 in ends:
+        for rn in ends:
+            if L % (r0 * rn):
+                continue
+            for mid in factorizations(L // (r0 * rn)):
+                c = [r0] + mid + [rn]
+                # fewest stages, then the largest end radices, then balance
+                key = (len(c), -min(r0, rn), -max(r0, rn), max(mid, default=1))
+                if best is None or key < best[0]:
+                    best = (key, c)
+    return (best[1], L // points) if best else None
+
+
+def geometry(prec, L, rads, mode, io, tpl_div=1, nl_mul=1.0, tpl=None):
     """Default geometry: one butterfly of the largest radix per thread and
     stage (tpl = L / Rmax); tpl_div > 1 gives each thread tpl_div of them;
     nl_mul scales the lines per workgroup of the default choice."""
     rmax = max(rads)
-    tpl = max(1, L // rmax // tpl_div)
+    if tpl is None:
+        tpl = max(1, L // rmax // tpl_div)
     pad = rads[0]
     lp = L + L // pad + 2
     csz = CSZ[prec]
@@ -93,6 +117,13 @@ def geometry(prec, L, rads, mode, io, tpl_div=1, nl_mul=1.0):
         # reals for the real-to-real kernels, which load one real per line)
         nl = 256 // (csz // 2 if io in ("R2C", "C2R", "DCT4") else csz)
         while nl > 1 and (nl * per_line > LDS_MAX - 1024 or nl * tpl > 1024):
+            nl //= 2
+        # real kernels: 128 B runs are enough when that lets two workgroups
+        # share a CU (FP64 512^2 x 64 REDFT10 120 -> 111 us, FP32 512^2 x 64
+        # REDFT01 60 -> 57); 64 B runs are not (FP32 2048^2 x 16 REDFT01 249
+        # -> 301, FP64 1024^2 x 32 257 -> 273)
+        rs = csz // 2
+        while io in ("R2C", "C2R", "DCT4") and nl * per_line > LDS_MAX // 2 - 1024 and nl * rs >= 256:
             nl //= 2
         # small transforms: more lines per workgroup for occupancy
         while nl * tpl < 256 and (nl * 2) * per_line <= LDS_TARGET and nl < 64:
@@ -219,15 +250,17 @@ def catalog():
                         # (runtime rmode; kept out of the plain r2c / c2r
                         # code), row and column mappings: the column one
                         # serves r2r dims whose lines are strided
-                        entries.append((prec, L, rads, "ROW", io + "_RR", g))
-                        gc = geometry(prec, L, rads, "COL", io)
+                        rr, tr = mirrored_radices(L) or (rads, None)
+                        entries.append((prec, L, rr, "ROW", io + "_RR",
+                                        geometry(prec, L, rr, "ROW", io, tpl=tr)))
+                        gc = geometry(prec, L, rr, "COL", io, tpl=tr)
                         # not for FP64 c2r at one line per workgroup
                         # (L = 5120, 6144, 8192): an execute through the
                         # 8192-point one aborted on the device, cause not
                         # established; strided lines of those lengths take
                         # the row-mapped kernel
                         if gc and not (prec == "double" and io == "C2R" and gc["nl"] == 1):
-                            entries.append((prec, L, rads, "COL", io + "_RR", gc))
+                            entries.append((prec, L, rr, "COL", io + "_RR", gc))
             # half-length r2c / c2r fused with one radix-8 stage of the next
             # dimension's DFT across the 8 rows of a tile (2-D and higher
             # real transforms): the remaining column pass is 8x shorter, so
@@ -252,9 +285,10 @@ def catalog():
             if (fam or L <= 64) and L <= 8192:
                 # DCT-IV / DST-IV of 2L reals through the L-point DFT
                 for mode in ("ROW", "COL"):
-                    g = geometry(prec, L, rads, mode, "DCT4")
+                    rr, tr = mirrored_radices(L) or (rads, None)
+                    g = geometry(prec, L, rr, mode, "DCT4", tpl=tr)
                     if g:
-                        entries.append((prec, L, rads, mode, "DCT4", g))
+                        entries.append((prec, L, rr, mode, "DCT4", g))
             # fused Bluestein on power-of-two convolution lengths; below 64
             # every length n with 2n - 1 <= L is 13-smooth and never takes
             # Bluestein
