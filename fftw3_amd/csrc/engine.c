@@ -105,7 +105,7 @@ void fk_free(void *p)
 /* ------------------------------------------------------------------ */
 /* cached device tables (freed by fk_cleanup)                          */
 
-enum { T_STAGE, T_TW2, T_LINE, T_CHIRP, T_BLUEB, T_DCT, T_DCT4 };
+enum { T_STAGE, T_TW2, T_LINE, T_CHIRP, T_BLUEB, T_DCT4 };
 
 typedef struct tbl {
     int type, prec, nrad;
@@ -203,21 +203,6 @@ static const void *line_table(int prec, long long n, long long count, hipStream_
     return t->dev;
 }
 
-/* twiddles of the fused REDFT10 / REDFT01 kernels (and their sine kinds) of
-   length n: for k <= n/4 the pair exp(-i pi k / 2n), exp(-i pi 5k / 2n) =
-   exp(-i pi k / 2n) W_n^k, next to each other */
-static const void *dct_table(int prec, long long n, hipStream_t st)
-{
-    const long long cnt = n / 4 + 1;
-    tbl *t = tbl_find(T_DCT, prec, n, 0, 0, 0);
-    if (t) return t->dev;
-    t = tbl_new(T_DCT, prec, n, 0, 0, 0, 2 * csz(prec) * (size_t)cnt);
-    if (!t) return 0;
-    if (fkm_gen_affine_tw(t->dev, prec, 0, 2, 4 * n, 1, 0, cnt, st)) return 0;
-    if (fkm_gen_affine_tw(t->dev, prec, 1, 2, 4 * n, 5, 0, cnt, st)) return 0;
-    return t->dev;
-}
-
 /* twiddles of the fused REDFT11 / RODFT11 kernels of length n = 2L: L input
    twiddles exp(-i pi (4m+1) / 4n), then L output twiddles exp(-i pi p / n) */
 static const void *dct4_table(int prec, long long n, hipStream_t st)
@@ -227,8 +212,8 @@ static const void *dct4_table(int prec, long long n, hipStream_t st)
     if (t) return t->dev;
     t = tbl_new(T_DCT4, prec, n, 0, 0, 0, 2 * csz(prec) * (size_t)L);
     if (!t) return 0;
-    if (fkm_gen_affine_tw(t->dev, prec, 0, 1, 8 * n, 4, 1, L, st)) return 0;
-    if (fkm_gen_affine_tw(t->dev, prec, L, 1, 2 * n, 1, 0, L, st)) return 0;
+    if (fkm_gen_affine_tw(t->dev, prec, 0, 8 * n, 4, 1, L, st)) return 0;
+    if (fkm_gen_affine_tw(t->dev, prec, L, 2 * n, 1, 0, L, st)) return 0;
     return t->dev;
 }
 
@@ -1853,7 +1838,7 @@ static int plan_r2r_1d(ctx *c, int kind, long long n, long long is, long long os
             const int dct3 = rm == FK_RM_DCT3 || rm == FK_RM_DST3;
             const int twid = dct2 || dct3 || rm == FK_RM_DCT4 || rm == FK_RM_DST4;
             if (rm == FK_RM_DCT4 || rm == FK_RM_DST4) wt = dct4_table(prec, n, c->st);
-            else if (twid) wt = dct_table(prec, n, c->st);
+            else if (twid) wt = line_table(prec, 4 * n, L + 1, c->st);
             if (!wk || (twid && !wt)) {
                 c->err = 1;
                 set_err("twiddle table allocation failed");
@@ -2207,10 +2192,24 @@ static void fill_magic(fk_args *a)
      its output, which the next pass reads, from 1 GiB on, four times the
      memory-side cache (512x512 x 256 775 -> 760; x 64 182 -> 208 the other
      way).
+   Only where every access of a wave covers whole 64-byte sectors (unit
+   strides, threads per line and butterflies of the end stages in fours): a
+   sector that several accesses share is fetched by each of them (32-point
+   lines 36.4 -> 31.9, but 24-point ones 34.5 -> 65, 16-point 42 -> 164).
    FP32 rows and column passes measured the same or slower.
    The quad loads of REDFT10 / RODFT10 rows, first pass and from 64 MiB on:
    FP32 2048^2 x 16 288 -> 239, FP32 2048 x 32768 138 -> 118, FP64 512^2 x 64
    126 -> 120; not FP64 alone (1024 x 32768 107 -> 116). */
+static int whole_sectors(const fk_pass *p)
+{
+    const fk_kernel *k = p->k;
+    const int nb0 = k->L / k->rad[0], nbn = k->L / k->rad[k->nrad - 1];
+    int i;
+    if (p->a.is != 1 || p->a.os != 1 || k->tpl % 4 || nb0 % 4 || nbn % 4) return 0;
+    for (i = 0; i < 3; ++i)
+        if (p->a.nb[i] > 1 && (p->a.ids[i] % 4 || p->a.ods[i] % 4)) return 0;
+    return 1;
+}
 static void mark_streams(fk_plan *P)
 {
     const long long MB = 1LL << 20;
@@ -2225,7 +2224,7 @@ static void mark_streams(fk_plan *P)
                 p->a.flags |= FK_NT_IN;
             continue;
         }
-        if (p->k->io != FK_IO_PLAIN || p->k->prec != 0) continue;
+        if (p->k->io != FK_IO_PLAIN || p->k->prec != 0 || !whole_sectors(p)) continue;
         if (P->npass == 1) {
             if (n >= 16 * MB && (!p->k->loop || n <= 512 * MB))
                 p->a.flags |= FK_NT_IN | FK_NT_OUT;

@@ -212,8 +212,8 @@ void fk_server_destroy(fk_server *s);
 int fkm_gen_stage_tw(void *out, int prec, int nrad, const int *rad, int total, hipStream_t st);
 int fkm_gen_tw2(double *lo, double *hi, long long N, long long b, hipStream_t st);
 int fkm_gen_line_tw(void *out, int prec, long long n, long long count, hipStream_t st);
-int fkm_gen_affine_tw(void *out, int prec, long long first, long long step, long long n, long long a,
-                      long long b, long long count, hipStream_t st);
+int fkm_gen_affine_tw(void *out, int prec, long long first, long long n, long long a, long long b,
+                      long long count, hipStream_t st);
 int fkm_gen_chirp(void *out, int prec, long long n, hipStream_t st);
 int fkm_gen_blue_b(void *out, long long n, long long M, hipStream_t st);
 int fkm_stream_copy(void *dst, const void *src, long long bytes, int mode, int ctas, hipStream_t st);

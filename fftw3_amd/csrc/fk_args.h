@@ -81,8 +81,8 @@ typedef struct {
     unsigned xcd_remap;       /* nonzero: spread tiles XCD-contiguously */
     unsigned rmode;           /* FK_RM_*: fused real-to-real kind */
     unsigned pad_;
-    const void *rtw;          /* FK_RM_DCT2/3, FK_RM_DST2/3: pairs exp(-i pi k / 2n),
-                                 exp(-i pi 5k / 2n), k <= n/4; FK_RM_DCT4, FK_RM_DST4:
+    const void *rtw;          /* FK_RM_DCT2/3, FK_RM_DST2/3: exp(-i pi k / 2n), k <= n/2;
+                                 FK_RM_DCT4, FK_RM_DST4:
                                  exp(-i pi (4m+1) / 4n), m < n/2, then exp(-i pi p / n) */
     /* division by multiplication, q / d = (2 q * qm >> 32) >> qs for q < 2^31:
        0 and 1 divide by nb[0] and nb[1] (qm[0] = 0: nlines >= 2^31, 64-bit

@@ -67,16 +67,16 @@ __global__ void k_gen_line_tw(cx<R> *out, long long n, long long count)
     out[t] = mk((R)c, (R)s);
 }
 
-/* out[step*t] = W_n^(a*t + b) */
+/* out[t] = W_n^(a*t + b) */
 template <typename R>
-__global__ void k_gen_affine_tw(cx<R> *out, long long step, long long n, long long a, long long b,
+__global__ void k_gen_affine_tw(cx<R> *out, long long n, long long a, long long b,
                                 long long count)
 {
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= count) return;
     double c, s;
     cexp_fp64(a * t + b, n, c, s);
-    out[step * t] = mk((R)c, (R)s);
+    out[t] = mk((R)c, (R)s);
 }
 
 /* c_m = exp(-i pi m^2 / n) = W_2n^(m^2 mod 2n) */
@@ -502,15 +502,15 @@ int fkm_gen_line_tw(void *out, int prec, long long n, long long count, hipStream
     return (int)hipGetLastError();
 }
 
-int fkm_gen_affine_tw(void *out, int prec, long long first, long long step, long long n, long long a,
-                      long long b, long long count, hipStream_t st)
+int fkm_gen_affine_tw(void *out, int prec, long long first, long long n, long long a, long long b,
+                      long long count, hipStream_t st)
 {
     if (prec == 0)
         hipLaunchKernelGGL(k_gen_affine_tw<double>, dim3(nblocks(count, 256)), dim3(256), 0, st,
-                           (cx<double> *)out + first, step, n, a, b, count);
+                           (cx<double> *)out + first, n, a, b, count);
     else
         hipLaunchKernelGGL(k_gen_affine_tw<float>, dim3(nblocks(count, 256)), dim3(256), 0, st,
-                           (cx<float> *)out + first, step, n, a, b, count);
+                           (cx<float> *)out + first, n, a, b, count);
     return (int)hipGetLastError();
 }
 

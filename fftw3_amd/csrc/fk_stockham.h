@@ -304,6 +304,8 @@ __device__ __forceinline__ void run_stages(int u, const cx<R> *tw, LdsF &&lds,
 template <class RL, int TPL>
 struct MirOk {
     static constexpr int L = RL::L(), R0 = RL::r[0], RN = RL::r[RL::n - 1];
+    /* one thread holds the whole line: every element's image is its own */
+    static constexpr bool self = RL::n == 1 && TPL == 1 && R0 % 2 == 0;
     static constexpr bool first = RL::n > 1 && R0 % 2 == 0 && (L / R0) % (2 * TPL) == 0;
     static constexpr bool last = RL::n > 1 && RN % 2 == 0 && (L / RN) % (2 * TPL) == 0;
 };
@@ -459,34 +461,51 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         constexpr long long N2 = 2LL * L;
         constexpr int R0 = RL::r[0], NB0 = L / R0, RN = RL::r[RL::n - 1], NBN = L / RN;
         constexpr bool M0 = MirOk<RL, TPL>::first, ML = MirOk<RL, TPL>::last;
+        constexpr bool SELF = MirOk<RL, TPL>::self;
         using BF0 = Bfly<NB0, TPL, M0>;
         using BFN = Bfly<NBN, TPL, ML>;
-        struct alignas(2 * sizeof(R)) P2 { R x, y; };
         auto first = whole([&](auto &v) {
-            sfor<0, BF0::BPT>([&](auto ic) {
-                constexpr int i = decltype(ic)::value, im = M0 ? BF0::image(i) : i;
-                const int b = BF0::template at<i>(u);
-                if ((NB0 % TPL == 0) || b < NB0) {
-                    if (M0 && (fl & FK_REAL_UNIT)) {
-                        asm volatile("");
-                        const P2 *p = reinterpret_cast<const P2 *>(inr) + b;
+            if ((M0 || SELF) && (fl & FK_REAL_UNIT)) {
+                asm volatile("");
+                if constexpr (SELF) {
+                    const cx<R> *p = reinterpret_cast<const cx<R> *>(inr);
+                    cx<R> x[R0];
+                    sfor<0, R0>([&](auto rc) { x[decltype(rc)::value] = p[decltype(rc)::value]; });
+                    sfor<0, R0>([&](auto rc) {
+                        constexpr int r = decltype(rc)::value;
+                        v[0][r] = mk(x[r].x, x[R0 - 1 - r].y);
+                    });
+                } else if constexpr (M0)
+                    sfor<0, BF0::BPT / 2>([&](auto ic) {
+                        constexpr int i = decltype(ic)::value, im = BF0::image(i);
+                        const cx<R> *p = reinterpret_cast<const cx<R> *>(inr);
+                        const cx<R> *pi = p + BF0::template at<i>(u), *pm = p + BF0::template at<im>(u);
+                        cx<R> x[R0], y[R0];
                         sfor<0, R0>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
-                            const P2 x = ldg(Acc<C_ONCE>{}, p + r * NB0);
-                            v[i][r].x = x.x;
-                            v[im][R0 - 1 - r].y = x.y;
+                            x[r] = ldg(Acc<C_ONCE>{}, pi + r * NB0);
+                            y[r] = ldg(Acc<C_ONCE>{}, pm + r * NB0);
                         });
-                    } else {
+                        sfor<0, R0>([&](auto rc) {
+                            constexpr int r = decltype(rc)::value;
+                            v[i][r] = mk(x[r].x, y[R0 - 1 - r].y);
+                            v[im][r] = mk(y[r].x, x[R0 - 1 - r].y);
+                        });
+                    });
+            } else {
+                sfor<0, BF0::BPT>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    const int b = BF0::template at<i>(u);
+                    if ((NB0 % TPL == 0) || b < NB0) {
                         const R *p = inr + 2 * b * is, *q = inr + (N2 - 1 - 2 * b) * is;
                         sfor<0, R0>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
                             const long long o = (2LL * r * NB0) * is;
-                            v[i][r].x = p[o];
-                            v[i][r].y = q[-o];
+                            v[i][r] = mk(p[o], q[-o]);
                         });
                     }
-                }
-            });
+                });
+            }
             sfor<0, BF0::BPT>([&](auto ic) {
                 constexpr int i = decltype(ic)::value;
                 const int b = BF0::template at<i>(u);
@@ -515,12 +534,12 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                 constexpr int i = decltype(ic)::value, im = ML ? BFN::image(i) : i;
                 const int b = BFN::template at<i>(u);
                 if (act && ((NBN % TPL == 0) || b < NBN)) {
-                    if (ML && (fl & FK_REAL_UNIT)) {
+                    if ((ML || SELF) && (fl & FK_REAL_UNIT)) {
                         asm volatile("");
-                        P2 *p = reinterpret_cast<P2 *>(outr) + b;
+                        cx<R> *p = reinterpret_cast<cx<R> *>(outr) + b;
                         sfor<0, RN>([&](auto rc) {
                             constexpr int r = decltype(rc)::value;
-                            p[r * NBN] = P2{v[i][r].x, v[im][RN - 1 - r].y};
+                            p[r * NBN] = mk(v[i][r].x, v[im][RN - 1 - r].y);
                         });
                     } else {
                         R *p = outr + 2 * b * os, *q = outr + (N2 - 1 - 2 * b) * os;
@@ -832,7 +851,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         const long long is = a.is, os = a.os;
         constexpr long long N2 = 2LL * L;
         constexpr int R0 = RL::r[0], NB0 = L / R0;
-        constexpr bool M0 = MirOk<RL, TPL>::first;
+        constexpr bool M0 = MirOk<RL, TPL>::first, SELF = MirOk<RL, TPL>::self;
         using BF = Bfly<NB0, TPL, M0>;
         constexpr int BPT = BF::BPT;
         /* elements j = b + r*NB0 of butterfly b: f(i, r, b) for those in range */
@@ -848,7 +867,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
            L-1-j: v_2j, v_{n-1-2j}, v_{2j+1}, v_{n-2-2j}. */
         auto quads = [&](auto &v, auto &&quad) {
             sfor<0, BPT>([&](auto ic) {
-                constexpr int i = decltype(ic)::value, im = BF::image(i);
+                constexpr int i = decltype(ic)::value, im = SELF ? i : BF::image(i);
                 const int b = BF::template at<i>(u);
                 sfor<0, R0 / 2>([&](auto rc) {
                     constexpr int r = decltype(rc)::value;
@@ -874,7 +893,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         auto first = whole([&](auto &v) {
             if (mak) {
                 asm volatile("");
-                if constexpr (M0) {
+                if constexpr (M0 || SELF) {
                     if (fl & FK_REAL_QUAD) {
                         asm volatile("");
                         /* as pairs past L1 in FP32 (see FK_IO_R2C) */
@@ -957,27 +976,27 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             }
         });
         auto lst = [&](auto k, cx<R> v) { lds_at(k) = v; };
-        /* bins k = u + i*TPL <= L/2, with L-k: one table entry each, two for
-           REDFT10 / RODFT10 (dt: exp(-i pi k / 2n) and that times W_n^k) */
+        /* bins k = u + i*TPL <= L/2, with L-k: one table entry W_n^k each, for
+           REDFT10 / RODFT10 also t_k and t_{L-k}, t_k = exp(-i pi k / 2n) */
         constexpr int HK = L / 2;
         constexpr int NK2 = (HK + 1 + TPL - 1) / TPL;
-        constexpr bool PRE = NK2 * sizeof(R) <= 48;
+        constexpr bool PRE = NK2 * sizeof(R) <= 40 && NR <= 512;
         constexpr int GK = PRE ? NK2 : 4;
-        struct alignas(2 * sizeof(cx<R>)) W2 { cx<R> a, b; };
-        W2 w[GK];
+        struct W3 { cx<R> w, t, s; };
+        W3 w[GK];
         auto tables = [&](auto gc) {
+            sfor<0, GK>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int k = u + (decltype(gc)::value * GK + i) * TPL;
+                w[i].w = wk[k <= HK ? k : HK];
+            });
             if (mak) {
                 asm volatile("");
                 sfor<0, GK>([&](auto ic) {
                     constexpr int i = decltype(ic)::value;
                     const int k = u + (decltype(gc)::value * GK + i) * TPL;
-                    w[i] = reinterpret_cast<const W2 *>(dt)[k <= HK ? k : HK];
-                });
-            } else {
-                sfor<0, GK>([&](auto ic) {
-                    constexpr int i = decltype(ic)::value;
-                    const int k = u + (decltype(gc)::value * GK + i) * TPL;
-                    w[i].a = wk[k <= HK ? k : HK];
+                    w[i].t = dt[k <= HK ? k : HK];
+                    w[i].s = dt[L - (k <= HK ? k : HK)];
                 });
             }
         };
@@ -1007,36 +1026,32 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
             if constexpr (!PRE) tables(gc);
             if (mak) {
-                /* c_k = exp(-i pi k / 2n) X_k: with t that factor, A = 2 t E
-                   and B = 2 t W O, 2 c_k = A + B and, as exp(-i pi (L-k) / 2n)
-                   = exp(-i pi / 4) conj t, 2 c_{L-k} = exp(-i pi / 4)
-                   conj(A - B).  REDFT10: y_k = 2 Re c_k, y_{n-k} = -2 Im c_k;
-                   RODFT10: the same reversed. */
+                /* c_k = t_k X_k; REDFT10: y_k = 2 Re c_k, y_{n-k} = -2 Im c_k;
+                   RODFT10: the same reversed */
                 asm volatile("");
                 const bool sn = rm == FK_RM_DST2;
                 const long long st = sn ? -os : os;
                 R *qk = sn ? outr + (N2 - 1 - u) * os : pk, *qn = sn ? pk - os : pn;
                 R *qm = sn ? pp - os : pm, *qp = sn ? pm - os : pp;
-                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, W2 t) {
-                    constexpr R h = (R)0.70710678118654752440084436210484903928;
+                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, const W3 &t) {
                     const long long d = (long long)decltype(dc)::value * st;
-                    const cx<R> A = mul(t.a, mk(zk.x + zc.x, zk.y - zc.y));
-                    const cx<R> B = mul(t.b, mk(zk.y + zc.y, zc.x - zk.x));
-                    const cx<R> D = sub(A, B);
-                    qk[d] = A.x + B.x;
-                    if (k != 0) qn[-d] = -(A.y + B.y);
+                    cx<R> X, Y;
+                    XY(zk, zc, t.w, X, Y);
+                    const cx<R> c = mul(X, t.t), e = mul(Y, t.s);
+                    qk[d] = (R)2 * c.x;
+                    if (k != 0) qn[-d] = (R)-2 * c.y;
                     if (2 * k != L) {
-                        qm[-d] = (D.x - D.y) * h;
-                        if (k != 0) qp[d] = (D.x + D.y) * h;
+                        qm[-d] = (R)2 * e.x;
+                        if (k != 0) qp[d] = (R)-2 * e.y;
                     }
                 });
             } else if (ext) {
                 /* DCT-I: Re X_k; DST-I: -Im X_k, one place lower */
                 asm volatile("");
-                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, W2 t) {
+                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, const W3 &t) {
                     const long long d = (long long)decltype(dc)::value * os;
                     cx<R> X, Y;
-                    XY(zk, zc, t.a, X, Y);
+                    XY(zk, zc, t.w, X, Y);
                     if (rm == FK_RM_E00) {
                         pk[d] = X.x;
                         if (2 * k != L) pm[-d] = Y.x;
@@ -1047,10 +1062,10 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                 });
             } else {
                 /* R2HC: r_k, i_k; DHT: Re - Im, Re + Im, at k and n-k */
-                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, W2 t) {
+                bins(gc, [&](auto dc, int k, cx<R> zk, cx<R> zc, const W3 &t) {
                     const long long d = (long long)decltype(dc)::value * os;
                     cx<R> X, Y;
-                    XY(zk, zc, t.a, X, Y);
+                    XY(zk, zc, t.w, X, Y);
                     if (rm == FK_RM_DHT) {
                         X = mk(X.x - X.y, X.x + X.y);
                         Y = mk(Y.x - Y.y, Y.x + Y.y);
@@ -1079,8 +1094,8 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         constexpr long long N2 = 2LL * L;
         constexpr int HK = L / 2;
         constexpr int NK2 = (HK + 1 + TPL - 1) / TPL;
-        constexpr int GK = sizeof(R) == 4 ? 6 : 4;
-        struct alignas(2 * sizeof(cx<R>)) W2 { cx<R> a, b; };
+        constexpr int GK = sizeof(R) == 4 ? 9 : 4;
+        struct W3 { cx<R> w, t, s; };
         /* samples k, n-k, L-k, L+k of the line (reversed for RODFT01) */
         const long long st = sn ? -is : is, o = sn ? N2 - 1 : 0;
         const R *pk = inr + o * is + u * st, *pn = inr + o * is + (N2 - u) * st;
@@ -1089,7 +1104,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             constexpr int g = decltype(gc)::value;
             constexpr int cnt = (NK2 - g * GK) < GK ? (NK2 - g * GK) : GK;
             R xk[cnt], xn[cnt], xm[cnt], xp[cnt];
-            W2 w[cnt];
+            W3 w[cnt];
             sfor<0, cnt>([&](auto ic) {
                 constexpr int i = decltype(ic)::value;
                 const int k = u + (g * GK + i) * TPL;
@@ -1101,59 +1116,57 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                     xp[i] = pp[d];
                 }
             });
+            sfor<0, cnt>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int k = u + (g * GK + i) * TPL;
+                w[i].w = wk[k <= HK ? k : HK];
+            });
+            cx<R> X[cnt], Y[cnt];
             if (hc) {
+                /* X[k] = (x_k, x_{n-k}), X[L-k] = (x_{L-k}, x_{L+k}),
+                   Im X[0] = Im X[L] = 0 */
                 sfor<0, cnt>([&](auto ic) {
                     constexpr int i = decltype(ic)::value;
                     const int k = u + (g * GK + i) * TPL;
-                    w[i].a = wk[k <= HK ? k : HK];
-                });
-                sfor<0, cnt>([&](auto ic) {
-                    constexpr int i = decltype(ic)::value;
-                    const int k = u + (g * GK + i) * TPL;
-                    if (k <= HK) {
-                        /* X[k] = (x_k, x_{n-k}), X[L-k] = (x_{L-k}, x_{L+k});
-                           Im X[0] = Im X[L] = 0.  As in FK_IO_C2R, swapped:
-                           e = X[k] + conj X[L-k], o = (X[k] - conj X[L-k])
-                           conj(W_n^k), Z[k] = e + i o, Z[L-k] = conj e + i conj o */
-                        const R ck = xn[i], cm = k == 0 ? (R)0 : xp[i];
-                        const cx<R> e = mk(xk[i] + xm[i], ck - cm);
-                        const cx<R> dd = mk(xk[i] - xm[i], ck + cm), t = w[i].a;
-                        const cx<R> oo = mk(dd.x * t.x + dd.y * t.y, dd.y * t.x - dd.x * t.y);
-                        lds_at(k) = mk(e.y + oo.x, e.x - oo.y);
-                        if (k != 0 && 2 * k != L) lds_at(L - k) = mk(oo.x - e.y, e.x + oo.y);
-                    }
+                    X[i] = mk(xk[i], xn[i]);
+                    Y[i] = mk(xm[i], k == 0 ? (R)0 : xp[i]);
                 });
             } else {
+                /* V_k = conj(t_k) (x_k - i x_{n-k}), t_k = exp(-i pi k / 2n) */
                 asm volatile("");
                 sfor<0, cnt>([&](auto ic) {
                     constexpr int i = decltype(ic)::value;
                     const int k = u + (g * GK + i) * TPL;
-                    w[i] = reinterpret_cast<const W2 *>(dt)[k <= HK ? k : HK];
+                    w[i].t = dt[k <= HK ? k : HK];
+                    w[i].s = dt[L - (k <= HK ? k : HK)];
                 });
                 sfor<0, cnt>([&](auto ic) {
                     constexpr int i = decltype(ic)::value;
-                    constexpr R h = (R)0.70710678118654752440084436210484903928;
                     const int k = u + (g * GK + i) * TPL;
-                    if (k <= HK) {
-                        /* with t = exp(-i pi k / 2n): V_k = conj(t) p,
-                           p = x_k - i x_{n-k}, and conj V_{L-k} = conj(t) q,
-                           q = exp(-i pi / 4)(x_{L-k} + i x_{L+k}); so
-                           e = conj(t)(p + q), o = conj(t W_n^k)(p - q) */
-                        const cx<R> q = mk((xm[i] + xp[i]) * h, (xp[i] - xm[i]) * h);
-                        const cx<R> s_ = mk(xk[i] + q.x, q.y - xn[i]);
-                        const cx<R> f = mk(xk[i] - q.x, -xn[i] - q.y);
-                        const cx<R> t = w[i].a, t2 = w[i].b;
-                        const cx<R> e = mk(s_.x * t.x + s_.y * t.y, s_.y * t.x - s_.x * t.y);
-                        const cx<R> oo = mk(f.x * t2.x + f.y * t2.y, f.y * t2.x - f.x * t2.y);
-                        lds_at(k) = mk(e.y + oo.x, e.x - oo.y);
-                        if (k != 0 && 2 * k != L) lds_at(L - k) = mk(oo.x - e.y, e.x + oo.y);
-                    }
+                    const cx<R> t = w[i].t, t2 = w[i].s;
+                    X[i] = mk(t.x * xk[i] - t.y * xn[i], -(t.x * xn[i] + t.y * xk[i]));
+                    Y[i] = mk(t2.x * xm[i] - t2.y * xp[i], -(t2.x * xp[i] + t2.y * xm[i]));
+                    /* Im V_0 = Im V_L = 0 */
+                    if (k == 0) X[i].y = Y[i].y = 0;
                 });
             }
+            /* as in FK_IO_C2R, swapped: e = X[k] + conj X[L-k], o = (X[k] -
+               conj X[L-k]) conj(W_n^k), Z[k] = e + i o, Z[L-k] = conj e + i conj o */
+            sfor<0, cnt>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int k = u + (g * GK + i) * TPL;
+                if (k <= HK) {
+                    const cx<R> e = mk(X[i].x + Y[i].x, X[i].y - Y[i].y);
+                    const cx<R> d = mk(X[i].x - Y[i].x, X[i].y + Y[i].y), t = w[i].w;
+                    const cx<R> o2 = mk(d.x * t.x + d.y * t.y, d.y * t.x - d.x * t.y);
+                    lds_at(k) = mk(e.y + o2.x, e.x - o2.y);
+                    if (k != 0 && 2 * k != L) lds_at(L - k) = mk(o2.x - e.y, e.x + o2.y);
+                }
+            });
         });
         SY::sync();
         constexpr int RN = RL::r[RL::n - 1], NBN = L / RN;
-        constexpr bool ML = MirOk<RL, TPL>::last;
+        constexpr bool ML = MirOk<RL, TPL>::last, SELF = MirOk<RL, TPL>::self;
         using BF = Bfly<NBN, TPL, ML>;
         constexpr int BPT = BF::BPT;
         /* v = swap(z_k): (v_2k+1, v_2k) */
@@ -1170,12 +1183,12 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             };
             if (!hc) {
                 asm volatile("");
-                if constexpr (ML) {
+                if constexpr (ML || SELF) {
                     /* elements k and L-1-k are outputs 4k..4k+3 */
                     auto quads = [&](auto &&quad) {
                         if (act)
                             sfor<0, BPT>([&](auto ic) {
-                                constexpr int i = decltype(ic)::value, im = BF::image(i);
+                                constexpr int i = decltype(ic)::value, im = SELF ? i : BF::image(i);
                                 const int b = BF::template at<i>(u);
                                 sfor<0, RN / 2>([&](auto rc) {
                                     constexpr int r = decltype(rc)::value;

@@ -138,19 +138,8 @@ static void stockham_ops(const fk_pass *ps, ops *o)
     if (k->variant >= 100) mfma_ops(k, &t);
     else stages_ops(k, &t);
     switch (k->io) {
-    case FK_IO_R2C_RR:
-        if (ps->a.rmode == FK_RM_DCT2 || ps->a.rmode == FK_RM_DST2) {
-            /* per pair of bins: 2 E and 2 O (4 add), two twiddle products,
-               their sum and difference (4 add), the turn by exp(-i pi / 4)
-               (2 add, 2 mul) */
-            t.add += 5 * L;
-            t.mul += L;
-            ops_acc(&t, L, &CMUL);
-            outs = L + 1;
-            break;
-        }
-        /* fall through */
     case FK_IO_R2C:
+    case FK_IO_R2C_RR:
     case FK_IO_R2C_XR:
         /* L+1 bins: E and O (4 add, 4 mul by 1/2), X = E + W O (4 fma) */
         outs = L + 1;
@@ -167,20 +156,17 @@ static void stockham_ops(const fk_pass *ps, ops *o)
             t.fma += outs * df / k->nl;
             ops_acc(&t, outs * (k->nl - 1) / k->nl, &CMUL);
         }
-        if (k->io == FK_IO_R2C_RR && ps->a.rmode == FK_RM_DHT) t.add += 2 * outs;
-        break;
-    case FK_IO_C2R_RR:
-        if (ps->a.rmode == FK_RM_DCT3 || ps->a.rmode == FK_RM_DST3) {
-            /* per pair of bins: the turn by exp(-i pi / 4) (2 add, 2 mul), sum
-               and difference (4 add), two twiddle products, Z[k] and Z[L-k]
-               (4 add) */
-            t.add += 5 * L;
-            t.mul += L;
-            ops_acc(&t, L, &CMUL);
-            break;
+        if (k->io == FK_IO_R2C_RR) {
+            const unsigned rm = ps->a.rmode;
+            if (rm == FK_RM_DHT) t.add += 2 * outs;
+            if (rm == FK_RM_DCT2 || rm == FK_RM_DST2) {
+                ops_acc(&t, outs, &CMUL);
+                t.mul += 2 * outs;
+            }
         }
-        /* fall through */
+        break;
     case FK_IO_C2R:
+    case FK_IO_C2R_RR:
     case FK_IO_C2R_XR:
         /* pre-pass per complex input: E, D (4 add), conj-twiddle product
            (2 mul + 2 fma), Z = E + i O (2 add) */
@@ -195,6 +181,12 @@ static void stockham_ops(const fk_pass *ps, ops *o)
             t.mul += (L + 1) * dm / k->nl;
             t.fma += (L + 1) * df / k->nl;
             ops_acc(&t, (L + 1) * (k->nl - 1) / k->nl, &CMUL);
+        }
+        if (k->io == FK_IO_C2R_RR &&
+            (ps->a.rmode == FK_RM_DCT3 || ps->a.rmode == FK_RM_DST3)) {
+            /* exp(+i pi k / 2n)(x_k - i x_{n-k}) per bin */
+            t.mul += 2 * (L + 1);
+            t.fma += 2 * (L + 1);
         }
         break;
     case FK_IO_BLUE: {

@@ -66,15 +66,18 @@ def choose_radices(n):
     return fs[0]
 
 
-def mirrored_radices(L, points=16):
+def mirrored_radices(L):
     """Radices and threads per line of the fused real-to-real kernels: each
-    thread holds `points` elements, and the first and last radix are even and
+    thread holds 16 elements (8 below 128, where 16 would leave too few
+    threads to read a line), and the first and last radix are even and
     divide points / 2, so that both stages can run mirrored (a thread then has
     elements j and L-1-j, whose samples are neighbours).  None if L has no
     such factorization."""
-    if L % points:
+    points = 16 if L >= 128 else 8
+    if L % points or L // points < 2:
         return None
-    ends = [r for r in RADICES if r % 2 == 0 and (points // 2) % r == 0]
+    # (24 = 4*3*2 measured slower than 6*4: its two-point ends)
+    ends = [r for r in RADICES if r in (4, 8) and (points // 2) % r == 0]
     best = None
     for r0 in ends:
         for rn in ends:
