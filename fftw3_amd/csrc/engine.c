@@ -54,6 +54,29 @@ void fk_set_async(int on) { g_async = on; }
 int fk_get_async(void) { return g_async; }
 void fk_set_timelimit(double t) { g_timelimit = t; }
 
+/* catalog entries by length: g_head[L] is the first, g_next[i] the one after
+   entry i, -1 at the end (planning looks kernels up for every divisor of a
+   length; set up once by fk_init) */
+#define MAX_L 16384
+static int g_head[MAX_L + 1];
+static int *g_next = 0;
+
+static pthread_once_t g_index_once = PTHREAD_ONCE_INIT;
+
+static void index_catalog(void)
+{
+    int i, n;
+    const fk_kernel *reg = fk_registry(&n);
+    int *next = (int *)malloc(sizeof(int) * (size_t)(n > 0 ? n : 1));
+    if (!next) return;
+    for (i = 0; i <= MAX_L; ++i) g_head[i] = -1;
+    for (i = n - 1; i >= 0; --i) {
+        next[i] = g_head[reg[i].L];
+        g_head[reg[i].L] = i;
+    }
+    g_next = next;
+}
+
 int fk_init(void)
 {
     int i, ndev = 0;
@@ -63,6 +86,11 @@ int fk_init(void)
         return -1;
     }
     g_reg = fk_registry(&g_nreg);
+    pthread_once(&g_index_once, index_catalog);
+    if (!g_next) {
+        set_err("out of memory");
+        return -1;
+    }
     for (i = 0; i < g_nreg; ++i) {
         if (g_reg[i].lds > 65536) {
             if (hipFuncSetAttribute(g_reg[i].fn, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -277,28 +305,53 @@ fail:
 /* ------------------------------------------------------------------ */
 /* kernel catalog queries                                              */
 
+static int first_of(long long L) { return g_next && L >= 0 && L <= MAX_L ? g_head[L] : -1; }
+
 static const fk_kernel *find_kernel(int prec, long long L, int mode, int io)
 {
     int i;
-    if (L > (1 << 20)) return 0;
-    for (i = 0; i < g_nreg; ++i) {
+    for (i = first_of(L); i >= 0; i = g_next[i]) {
         const fk_kernel *k = g_reg + i;
-        if (k->prec == prec && k->L == L && k->mode == mode && k->io == io) return k;
+        if (k->prec == prec && k->mode == mode && k->io == io) return k;
     }
     return 0;
 }
 
-static int has_single(int prec, long long n) { return find_kernel(prec, n, FK_ROW, FK_IO_PLAIN) != 0; }
+/* Lengths a longer line is split into: up to 64, powers of two times 1, 3 or 5,
+   powers of 3, 5 and 7, and four round ones.  The catalog's other lengths serve
+   whole lines only: they have no transposed-store kernel and shorter runs in
+   their column passes, and a split into them measured slower (us, one pass more
+   or shorter runs: FP32 444528 x 29 167 -> 283, FP64 real 7350 x 179 there and
+   back 56 -> 60). */
+static int is_factor(long long n)
+{
+    long long m = n;
+    int i;
+    if (n <= 64 || n == 100 || n == 1000 || n == 1001 || n == 10000) return 1;
+    while (m % 2 == 0) m /= 2;
+    if (m == 1 || m == 3 || m == 5) return 1;
+    for (i = 3; i <= 7; i += 2) {
+        for (m = n; m % i == 0; m /= i)
+            ;
+        if (m == 1) return 1;
+    }
+    return 0;
+}
+
+static int has_single(int prec, long long n)
+{
+    return is_factor(n) && find_kernel(prec, n, FK_ROW, FK_IO_PLAIN) != 0;
+}
 
 /* the catalog variant of (prec, L, mode, io) whose stages are all radix 16
    (the matrix-core substitution needs them), or NULL */
 static const fk_kernel *find_kernel_r16(int prec, long long L, int mode, int io)
 {
     int i, j;
-    for (i = 0; i < g_nreg; ++i) {
+    for (i = first_of(L); i >= 0; i = g_next[i]) {
         const fk_kernel *k = g_reg + i;
         int all16 = k->nrad > 0;
-        if (k->prec != prec || k->L != L || k->mode != mode || k->io != io) continue;
+        if (k->prec != prec || k->mode != mode || k->io != io) continue;
         for (j = 0; j < k->nrad; ++j) all16 &= k->rad[j] == 16;
         if (all16) return k;
     }
@@ -318,7 +371,7 @@ static int smooth_plannable(int prec, long long n, int depth)
     if (n == 1 || has_single(prec, n)) return 1;
     if (depth >= 3) return 0;
     for (n1 = 2; n1 <= 16384 && n1 < n; ++n1) {
-        if (n % n1) continue;
+        if (n % n1 || !is_factor(n1)) continue;
         if (!find_kernel(prec, n1, FK_COL, FK_IO_PLAIN)) continue;
         if (smooth_plannable(prec, n / n1, depth + 1)) return 1;
     }
@@ -342,6 +395,7 @@ typedef struct {
     int nchoice;
     int ci;                     /* decisions taken so far */
     int r16;                    /* restrict to radix-16 passes (FK_MFMA) */
+    int part;                   /* planning a part of a split line */
     int bin, bout;              /* buffers of the r2c / c2r problem's arrays */
     int nalt[FK_MAX_DECIDE];    /* alternatives at each decision */
     int dkind[FK_MAX_DECIDE];
@@ -365,12 +419,11 @@ static int decide(ctx *c, int nalt, int kind)
 static int find_variants(int prec, long long L, int mode, int io, const fk_kernel **out, int max)
 {
     int i, n = 0, v;
-    if (L > (1 << 20)) return 0;
     for (v = 0; v < max; ++v) {
         const fk_kernel *hit = 0;
-        for (i = 0; i < g_nreg; ++i) {
+        for (i = first_of(L); i >= 0; i = g_next[i]) {
             const fk_kernel *k = g_reg + i;
-            if (k->prec == prec && k->L == L && k->mode == mode && k->io == io && k->variant == v) {
+            if (k->prec == prec && k->mode == mode && k->io == io && k->variant == v) {
                 hit = k;
                 break;
             }
@@ -779,7 +832,7 @@ static int split_candidates(int prec, long long n, long long *out, int max)
         long long n2;
         double score;
         const fk_kernel *kc, *kt;
-        if (n % n1) continue;
+        if (n % n1 || !is_factor(n1)) continue;
         n2 = n / n1;
         kc = find_kernel(prec, n1, FK_COL, FK_IO_PLAIN);
         if (!kc) continue;
@@ -853,6 +906,7 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
         return 0;
     }
     kr = find_kernel(prec, n, FK_ROW, FK_IO_PLAIN);
+    if (c->part && !is_factor(n)) kr = 0;
     if (c->r16 && n != 16 && n != 256 && n != 4096) kr = 0;
     if (kr) {
         /* candidate thread mappings, the heuristic's choice first:
@@ -956,8 +1010,11 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
             bb[i + 1].is = ab[i + 1].os;
             bb[i + 1].os = b[i].os;
         }
-        return plan_c2c_1d(c, n2, 1, n1 * os, nb + 1, bb, FK_BUF_S0 + slot, 0, ob, oo, 0, swo,
-                           slot + 1);
+        ++c->part;
+        i = plan_c2c_1d(c, n2, 1, n1 * os, nb + 1, bb, FK_BUF_S0 + slot, 0, ob, oo, 0, swo,
+                        slot + 1);
+        --c->part;
+        return i;
     }
 blue:
     return plan_bluestein(c, n, is, os, nb, b, ib, io, ob, oo, swi, swo, slot);

@@ -163,6 +163,15 @@ def size_list(prec):
             s.add(p)
             p *= base
     s.update([100, 1000, 1001, 2187, 81, 729])
+    # products of 2, 3, 5 and 7: all up to 512, those with a factor 4 or 10 up
+    # to 1024, with 16 or 40 up to 2048 (each kernel costs build time, and the
+    # rounder lengths are the ones in use).  As two passes such a line is read
+    # and written twice: us, 64 MiB arrays, FP32 240 x 34952 69.1 -> 31.4,
+    # 1080 x 7767 61.0 -> 33.9, columns 270 143 -> 31; r2c there and back 240
+    # 101 -> 39
+    s.update(n for n in range(65, 2049) if smooth(n, (2, 3, 5, 7)) and
+             (n <= 512 or n % 16 == 0 or n % 40 == 0 or
+              n <= 1024 and (n % 4 == 0 or n % 10 == 0)))
     if lmax >= 10000:
         s.add(10000)
     return sorted(x for x in s if x <= lmax)
@@ -243,12 +252,14 @@ def catalog():
                             entries.append((prec, L, r8, mode, io,
                                             dict(gx, xs=1, lds=lp * gx["nl"] * CSZ[prec] // 2)))
             # half-length kernels for even real transforms (n = 2L)
-            if (fam or L <= 64) and L <= 8192:
+            if (fam or L <= 64 or smooth(L, (2, 3, 5, 7))) and L <= 8192:
                 for io in ("R2C", "C2R"):
                     g = geometry(prec, L, rads, "ROW", io)
                     if g:
                         entries.append((prec, L, rads, "ROW", io, g))
                         entries += variants(prec, L, rads, "ROW", io, g)
+                        if not fam and L > 64:
+                            continue
                         # the same kernel with a fused real-to-real kind
                         # (runtime rmode; kept out of the plain r2c / c2r
                         # code), row and column mappings: the column one
@@ -280,7 +291,8 @@ def catalog():
                         entries.append((prec, L, rads, "ROW", "R2C_XR", gx))
                         entries.append((prec, L, rads, "ROW", "C2R_XR", gx))
             # full-length real kernels for odd lengths (no half-length form)
-            if L % 2 == 1 and L <= 8192:
+            if L % 2 == 1 and L <= 8192 and (L <= 64 or L == 1001 or
+                                            any(smooth(L, (p,)) for p in (3, 5, 7))):
                 for io in ("R2C_FULL", "C2R_FULL"):
                     g = geometry(prec, L, rads, "ROW", "PLAIN")
                     if g:
