@@ -85,8 +85,8 @@ typedef struct {
                                  FK_RM_DCT4, FK_RM_DST4:
                                  exp(-i pi (4m+1) / 4n), m < n/2, then exp(-i pi p / n) */
     /* division by multiplication, q / d = (2 q * qm >> 32) >> qs for q < 2^31:
-       0 and 1 divide by nb[0] and nb[1] (qm[0] = 0: nlines >= 2^31, 64-bit
-       division), 2 by tb (qm[2] = 0: tN >= 2^31) */
+       0 and 1 divide by nb[0] and nb[1] (qm[0] = 0: nlines >= 2^31, divided
+       as 64-bit numbers), 2 by tb (qm[2] = 0: tN >= 2^31) */
     unsigned qm[3], qs[3];
 } fk_args;
 

@@ -331,6 +331,15 @@ __device__ __forceinline__ void cexp_fp64(long long m, long long n, double &c,
     s = -sn;
 }
 
+/* q / d for 0 <= q < 2^53, d > 0, through FP64: q is exact there and the
+   quotient off by at most one (a 64-bit integer division would be several
+   hundred instructions in every kernel, for the few passes that need it) */
+__device__ __forceinline__ long long div_large(long long q, long long d)
+{
+    const long long t = (long long)((double)q / (double)d), r = q - t * d;
+    return r < 0 ? t - 1 : r >= d ? t + 1 : t;
+}
+
 /* W_N^e in FP64 from the two-level table (see tw2) */
 __device__ __forceinline__ cx<double> tw2d(const fk_args &a, long long e);
 
@@ -354,7 +363,7 @@ __device__ __forceinline__ cx<double> tw2d(const fk_args &a, long long e)
         const double2 hi = reinterpret_cast<const double2 *>(a.thi)[q];
         return mk(lo.x * hi.x - lo.y * hi.y, lo.x * hi.y + lo.y * hi.x);
     }
-    const long long ih = e / b, il = e - ih * b;
+    const long long ih = div_large(e, b), il = e - ih * b;
     const double *lo = a.tlo + 2 * il, *hi = a.thi + 2 * ih;
     return mk(lo[0] * hi[0] - lo[1] * hi[1], lo[0] * hi[1] + lo[1] * hi[0]);
 }
@@ -374,10 +383,10 @@ __device__ __forceinline__ LineIx line_ix(const fk_args &a, long long q)
         r.i1 = q1 - q2 * (unsigned)a.nb[1];
         r.i2 = q2;
     } else {
-        r.i0 = q % a.nb[0];
-        q /= a.nb[0];
-        r.i1 = q % a.nb[1];
-        r.i2 = q / a.nb[1];
+        const long long q1 = div_large(q, a.nb[0]);
+        r.i0 = q - q1 * a.nb[0];
+        r.i2 = div_large(q1, a.nb[1]);
+        r.i1 = q1 - r.i2 * a.nb[1];
     }
     return r;
 }

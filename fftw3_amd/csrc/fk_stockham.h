@@ -138,7 +138,7 @@ struct SyncWave {
 /* What happens to a butterfly's registers after its loads (first stage) or
    before its stores (last stage). */
 struct NoOp {
-    template <int N, typename R>
+    template <int N, int I, typename R>
     __device__ __forceinline__ void run(int, cx<R> *) const
     {
     }
@@ -160,7 +160,7 @@ __device__ __forceinline__ void swap_if(bool sw, cx<R> *v)
 }
 struct SwapOp {
     bool sw;
-    template <int N, typename R>
+    template <int N, int I, typename R>
     __device__ __forceinline__ void run(int, cx<R> *v) const
     {
         swap_if<N>(sw, v);
@@ -170,32 +170,61 @@ struct SwapOp {
 /* Output post-op of the plain passes: four-step twiddle, then the swap.
    The twiddle of output k = b + r*Ns (last stage, r = 0..N-1) of a line with
    batch index i0 is W_N^(k*i0): looked up in the FP64 table every ANCH
-   outputs and stepped by W_N^(Ns*i0) in FP64 in between, so a thread gathers
-   2 table entries per ANCH outputs instead of 2 per output.  FP64 data
-   re-anchors every 4 (at most 3 products from a table value); FP32 data once
-   per butterfly (at most 15 FP64 products, ~1e-15, far below FP32 rounding). */
-template <int NS>
+   outputs of a butterfly and multiplied by powers of W_N^(Ns*i0) in FP64 in
+   between (binary splitting, so that the products do not wait for each
+   other).  FP64 data re-anchors every 4 (at most 2 products from a table
+   value); FP32 data once per butterfly (at most 4 products, the last power
+   itself 3 squarings, ~2e-15, far below FP32 rounding).  The lookups are made
+   before the stages, so that they do not add their latency to the end of the
+   pass, while they fit a few registers. */
+template <typename R, class RL, int TPL>
 struct PlainOut {
+    static constexpr int N = RL::r[RL::n - 1], NS = RL::ns(RL::n - 1);
+    static constexpr int BPT = (NS + TPL - 1) / TPL;
+    static constexpr int ANCH = sizeof(R) == 8 ? 4 : 16, NA = (N + ANCH - 1) / ANCH;
+    static constexpr bool EARLY = sizeof(R) == 4 && BPT * NA <= 4;
     const fk_args &a;
     bool tw, sw;
     long long i0;
-    cx<double> step;
-    __device__ __forceinline__ PlainOut(const fk_args &a_, unsigned fl, long long i0_)
+    cx<double> step, anchor[EARLY ? BPT * NA : 1];
+    __device__ __forceinline__ PlainOut(const fk_args &a_, unsigned fl, long long i0_, int u)
         : a(a_), tw(fl & FK_TW_OUT), sw(fl & FK_SWAP_OUT), i0(i0_), step(mk(1.0, 0.0))
     {
-        if (tw) step = tw2d(a, (long long)NS * i0);
+        if (tw) {
+            step = tw2d(a, (long long)NS * i0);
+            if constexpr (EARLY)
+                sfor<0, BPT * NA>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value / NA, g = decltype(ic)::value % NA;
+                    /* threads past the last butterfly look up the last one's */
+                    const int b = u + i * TPL < NS ? u + i * TPL : NS - 1;
+                    anchor[i * NA + g] = tw2d(a, (long long)(b + g * ANCH * NS) * i0);
+                });
+        }
     }
-    template <int N, typename R>
+    template <int N_, int I>
     __device__ __forceinline__ void run(int b, cx<R> *v) const
     {
         if (tw) {
-            constexpr int ANCH = sizeof(R) == 8 ? 4 : 16;
-            cx<double> cur = mk(1.0, 0.0);
-            sfor<0, N>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
-                if constexpr (r % ANCH == 0) cur = tw2d(a, (long long)(b + r * NS) * i0);
-                else cur = mul(cur, step);
-                v[r] = mul(v[r], mk((R)cur.x, (R)cur.y));
+            const cx<double> s2 = mul(step, step);
+            cx<double> s4 = s2, s8 = s2;
+            if constexpr (ANCH > 4 && N > 4) s4 = mul(s2, s2);
+            if constexpr (ANCH > 8 && N > 8) s8 = mul(s4, s4);
+            sfor<0, NA>([&](auto gc) {
+                constexpr int g = decltype(gc)::value;
+                cx<double> w[ANCH];
+                if constexpr (EARLY) w[0] = anchor[I * NA + g];
+                else w[0] = tw2d(a, (long long)(b + g * ANCH * NS) * i0);
+                sfor<1, ANCH>([&](auto rc) {
+                    constexpr int r = decltype(rc)::value;
+                    constexpr int h = r >= 8 ? 8 : r >= 4 ? 4 : r >= 2 ? 2 : 1;
+                    if constexpr (g * ANCH + r < N)
+                        w[r] = mul(w[r - h], h == 8 ? s8 : h == 4 ? s4 : h == 2 ? s2 : step);
+                });
+                sfor<0, ANCH>([&](auto rc) {
+                    constexpr int r = decltype(rc)::value;
+                    if constexpr (g * ANCH + r < N)
+                        v[g * ANCH + r] = mul(v[g * ANCH + r], mk((R)w[r].x, (R)w[r].y));
+                });
             });
         }
         swap_if<N>(sw, v);
@@ -251,10 +280,10 @@ __device__ __forceinline__ void stage(int u, const cx<R> *__restrict__ tw,
                     v[i][r] = mul(v[i][r], w[r - 1]);
                 });
             }
-            pre.template run<Rs>(b, v[i]);
+            pre.template run<Rs, i>(b, v[i]);
             Dft<R, Rs, 1>::run(v[i]);
             const int base = (b - k) * Rs + k;
-            fin.template run<Rs>(base, v[i]);
+            fin.template run<Rs, i>(base, v[i]);
             /* stage 0 (Ns = 1) writes Rs consecutive outputs from b*Rs */
             auto store = [&](auto &&put) {
                 sfor<0, Rs>([&](auto rc) {
@@ -389,7 +418,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                     });
                 });
             });
-            const PlainOut<RL::ns(RL::n - 1)> fin(a, fl, i0);
+            const PlainOut<R, RL, TPL> fin(a, fl, i0, u);
             run_stages<R, RL, 0, L, TPL, false, false, SY>(u, tw, lds_at, gld, gst, SwapOp{swi},
                                                            fin);
         } else {
@@ -1420,7 +1449,7 @@ __device__ __forceinline__ void run_xs(int u, const cx<R> *__restrict__ tw, R *b
                 });
             }
             Dft<R, Rs, 1>::run(v[i]);
-            if constexpr (S == RL::n - 1) fin.template run<Rs>(b, v[i]);
+            if constexpr (S == RL::n - 1) fin.template run<Rs, i>(b, v[i]);
         }
     });
     auto each_out = [&](auto &&f) {
@@ -1491,7 +1520,7 @@ stockham_xs(fk_args a)
     const bool swi = fl & FK_SWAP_IN;
     R *buf = reinterpret_cast<R *>(smem_raw) + (MODE == FK_ROW ? lt * LP : lt);
     auto idx = [](int j) { return MODE == FK_ROW ? j + j / PAD : j * NL; };
-    const PlainOut<RL::ns(RL::n - 1)> fin(a, fl, lx.i0);
+    const PlainOut<R, RL, TPL> fin(a, fl, lx.i0, u);
     auto gst = [&](int k, cx<R> v) {
         if (act) out[bout + k * a.os] = v;
     };
