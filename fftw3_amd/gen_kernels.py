@@ -470,7 +470,8 @@ def main():
         vcount[key] = v + 1
         numbered.append(e + (v,))
     entries = numbered
-    nparts = 8
+    # (many small units: one unit per core compiles a fifth slower)
+    nparts = 32
     parts = [[] for _ in range(nparts)]
     # round-robin by estimated cost so parts compile in similar time
     for i, e in enumerate(sorted(entries, key=lambda e: -e[1])):
