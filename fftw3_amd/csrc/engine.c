@@ -36,6 +36,7 @@ static int g_nreg = 0;
 static int g_inited = 0;
 static hipStream_t g_stream = 0;
 static int g_async = 0;
+static int g_ncu = 256;             /* compute units of the device */
 static double g_timelimit = -1.0;
 static __thread char g_err[512];
 
@@ -86,6 +87,11 @@ int fk_init(void)
         return -1;
     }
     g_reg = fk_registry(&g_nreg);
+    if (hipGetDevice(&i) == hipSuccess &&
+        hipDeviceGetAttribute(&ndev, hipDeviceAttributeMultiprocessorCount, i) == hipSuccess) {
+        if (ndev > 0) g_ncu = ndev;
+    } else
+        (void)hipGetLastError();
     pthread_once(&g_index_once, index_catalog);
     if (!g_next) {
         set_err("out of memory");
@@ -319,10 +325,10 @@ static const fk_kernel *find_kernel(int prec, long long L, int mode, int io)
 
 /* Lengths a longer line is split into: up to 64, powers of two times 1, 3 or 5,
    powers of 3, 5 and 7, and four round ones.  The catalog's other lengths serve
-   whole lines only: they have no transposed-store kernel and shorter runs in
-   their column passes, and a split into them measured slower (us, one pass more
-   or shorter runs: FP32 444528 x 29 167 -> 283, FP64 real 7350 x 179 there and
-   back 56 -> 60). */
+   whole lines only: without transposed-store kernels they end a split with
+   scattered stores, or (as split_candidates scores that) make it one pass
+   longer (us: FP32 444528 x 29 167 -> 283, FP64 real 7350 x 179 there and back
+   56 -> 60). */
 static int is_factor(long long n)
 {
     long long m = n;
@@ -446,11 +452,37 @@ static int forced(int prec, long long L, int mode, int io)
     return f && f->prec == prec && f->L == L && f->mode == mode && f->io == io;
 }
 
-static const fk_kernel *pick_variant(ctx *c, int prec, long long L, int mode, int io)
+static long long batch_count(int nb, const fk_dim *b);
+
+/* lines: how many the pass has (0: not known here) */
+static const fk_kernel *pick_variant(ctx *c, int prec, long long L, int mode, int io,
+                                     long long lines)
 {
     const fk_kernel *vs[16];
     int n = find_variants(prec, L, mode, io, vs, 16), v;
     if (!n) return 0;
+    if (!vs[0]->loop && lines > 0 && 2 * ((lines + vs[0]->nl - 1) / vs[0]->nl) <= g_ncu &&
+        ((mode == FK_ROW && io != FK_IO_TOUT) || vs[0]->nl * (int)csz(prec) >= 128)) {
+        /* the default geometry would leave half the CUs without a workgroup:
+           the same kernel with half the lines per workgroup comes first, where
+           there is one (same results; us, one transform: FP32 2^20 24.5 ->
+           20.0, 1024^2 16.7 -> 14.8, 256^2 10.4 -> 8.9, 1024 x 64 5.0 -> 4.6,
+           FP64 256 x 256 4.5 -> 4.1).  Not where two of them would share a CU
+           (FP32 2^20 x 63 column pass 265 -> 288), nor in column tiles and
+           transposed stores whose runs would fall below 64 bytes (FP32
+           4096 x 56 x 18, both, 33 -> 41) */
+        for (v = 1; v < n; ++v) {
+            const fk_kernel *h = vs[v];
+            int j, same = !h->loop && h->tpl == vs[0]->tpl && 2 * h->nl == vs[0]->nl &&
+                          h->nrad == vs[0]->nrad;
+            for (j = 0; same && j < h->nrad; ++j) same = h->rad[j] == vs[0]->rad[j];
+            if (same) {
+                vs[v] = vs[0];
+                vs[0] = h;
+                break;
+            }
+        }
+    }
     v = n > 1 ? decide(c, n, DEC_VARIANT) : 0;
     return forced(prec, L, mode, io) ? g_force : vs[v];
 }
@@ -940,9 +972,9 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
             memmove(b + 1, b, sizeof(fk_dim) * d);
             b[0] = t;
         }
-        if (m == 1) k = pick_variant(c, prec, n, FK_ROW, FK_IO_TOUT);
-        else if (m == 2) k = pick_variant(c, prec, n, FK_COL, FK_IO_PLAIN);
-        else k = pick_variant(c, prec, n, FK_ROW, FK_IO_PLAIN);
+        if (m == 1) k = pick_variant(c, prec, n, FK_ROW, FK_IO_TOUT, batch_count(nb, b));
+        else if (m == 2) k = pick_variant(c, prec, n, FK_COL, FK_IO_PLAIN, batch_count(nb, b));
+        else k = pick_variant(c, prec, n, FK_ROW, FK_IO_PLAIN, batch_count(nb, b));
         if (c->r16) {
             /* matrix-core plans: the all-radix-16 variant of the mapping */
             const fk_kernel *k16 = find_kernel_r16(prec, n, k->mode, k->io);
@@ -970,8 +1002,8 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
         if (!ncand) goto blue;
         n1 = cands[ncand > 1 ? decide(c, ncand, DEC_SPLIT) : 0];
         n2 = n / n1;
-        kA = pick_variant(c, prec, n1, FK_COL, FK_IO_PLAIN);
         H = batch_count(nb, b);
+        kA = pick_variant(c, prec, n1, FK_COL, FK_IO_PLAIN, n2 * H);
         need_scratch(c, slot, cs * (size_t)n * (size_t)H);
         /* pass A: lines n2_idx (tile dim), elements n1_idx at stride is*n2 */
         ab[0].n = n2;
@@ -1305,7 +1337,7 @@ static const fk_kernel *xr_kernel(ctx *c, const fk_problem *pb, int io, fk_dim *
     /* rows per tile: 8 by default, 4 (half the LDS, a 2x longer column
        pass) as the tuner's alternative */
     if (!find_kernel(c->P->prec, nl / 2, FK_ROW, io)) return 0;
-    k = pick_variant(c, c->P->prec, nl / 2, FK_ROW, io);
+    k = pick_variant(c, c->P->prec, nl / 2, FK_ROW, io, 0);
     if (!k) return 0;
     n0 = pb->dims[r - 2].n;
     if (n0 % k->nl || n0 / k->nl < 2) return 0;
@@ -1470,7 +1502,7 @@ static int plan_r2c(ctx *c, const fk_problem *pb)
         const fk_kernel *kx = xr_kernel(c, pb, FK_IO_R2C_XR, xe, &nxe);
         if (kx && decide(c, 2, DEC_VARIANT) == 0) return plan_r2c_xr(c, pb, kx, xe, nxe);
     }
-    if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_R2C);
+    if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_R2C, batch_count(nb, b));
     if (k) {
         size_t before = (size_t)P->npass;
         unsigned fl = 0;
@@ -1488,7 +1520,7 @@ static int plan_r2c(ctx *c, const fk_problem *pb)
         }
         if (unit) need_align(c, c->bin, (unsigned)(2 * rs));
         desc_add(P, "(r2c-fused L=%lld)", L);
-    } else if ((k = pick_variant(c, prec, nl, FK_ROW, FK_IO_R2C_FULL)) != 0) {
+    } else if ((k = pick_variant(c, prec, nl, FK_ROW, FK_IO_R2C_FULL, 0)) != 0) {
         /* one pass: full-length DFT of the real line, half the bins stored */
         size_t before = (size_t)P->npass;
         emit_stockham(c, k, pb->dims[r - 1].is, pb->dims[r - 1].os, nb, b, c->bin, 0, c->bout, 0,
@@ -1629,7 +1661,7 @@ static int plan_c2r(ctx *c, const fk_problem *pb)
     for (i = 0; i < pb->vrank; ++i) b[nb++] = pb->vdims[i];
     nb = squeeze(nb, b);
     sort_by_is(nb, b);
-    if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_C2R);
+    if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_C2R, batch_count(nb, b));
     if (k) {
         size_t before = (size_t)P->npass;
         unsigned fl = 0;
@@ -1647,7 +1679,7 @@ static int plan_c2r(ctx *c, const fk_problem *pb)
         }
         if (unit) need_align(c, c->bout, (unsigned)(2 * rs));
         desc_add(P, "(c2r-fused L=%lld)", L);
-    } else if ((k = pick_variant(c, prec, nl, FK_ROW, FK_IO_C2R_FULL)) != 0) {
+    } else if ((k = pick_variant(c, prec, nl, FK_ROW, FK_IO_C2R_FULL, 0)) != 0) {
         /* one pass: Hermitian expansion on load, real part on store */
         size_t before = (size_t)P->npass;
         emit_stockham(c, k, pb->dims[r - 1].is, pb->dims[r - 1].os, nb, b, c->bin, 0, c->bout, 0,
@@ -1875,14 +1907,14 @@ static int plan_r2r_1d(ctx *c, int kind, long long n, long long is, long long os
                 }
             }
             if (best > 4) dC = -1;
-            if (dC >= 0) k = pick_variant(c, prec, L, FK_COL, io);
+            if (dC >= 0) k = pick_variant(c, prec, L, FK_COL, io, 0);
             if (k) {
                 fk_dim t = b[dC];
                 memmove(b + 1, b, sizeof(fk_dim) * dC);
                 b[0] = t;
             }
         }
-        if (ok && !k) k = pick_variant(c, prec, L, FK_ROW, io);
+        if (ok && !k) k = pick_variant(c, prec, L, FK_ROW, io, 0);
         if (k) {
             size_t before = (size_t)P->npass;
             unsigned fl = 0;
@@ -2235,8 +2267,9 @@ static void fill_magic(fk_args *a)
     if (a->tb > 0 && a->tN < (1LL << 31)) fk_magic((unsigned long long)a->tb, &a->qm[2], &a->qs[2]);
 }
 
-/* Row passes that bypass the caches.  FP64 passes of plain lines read and write non-temporally where that
-   measured faster (us, arrays rotated; one pass unless noted):
+/* Row passes that bypass the caches.  FP64 passes of plain lines read and
+   write non-temporally where that measured faster (us, arrays rotated; one
+   pass unless noted):
      one pass, arrays of 16 MiB (together larger than the 32 MB of L2) and
      more: 512 x 2048 9.0 -> 7.0, 512 x 8192 28.2 -> 25.3, 512 x 65536 377 ->
      364, 4096 x 1024 28.6 -> 26.3, also where a second transform reads the
@@ -2244,8 +2277,10 @@ static void fill_magic(fk_args *a)
      16 MiB no difference;
      the pipelined kernels up to 512 MiB (4096 x 8192 206 -> 204; 4096 x 16384
      388 -> 404 the other way);
-     the first pass of several: its input from 64 MiB on (512x512 x 16 57.6 ->
-     53.7, x 64 203 -> 182, x 128 410 -> 391; x 4 19.4 -> 19.9 the other way),
+     the first pass of several: its input from 128 MiB on, where input and
+     output together exceed the memory-side cache (512x512 x 64 203 -> 182, x
+     128 410 -> 391; 2048x2048 x 1 56.0 -> 58.2 and x 4 of 512x512 19.4 -> 19.9
+     the other way),
      its output, which the next pass reads, from 1 GiB on, four times the
      memory-side cache (512x512 x 256 775 -> 760; x 64 182 -> 208 the other
      way).
@@ -2286,7 +2321,7 @@ static void mark_streams(fk_plan *P)
             if (n >= 16 * MB && (!p->k->loop || n <= 512 * MB))
                 p->a.flags |= FK_NT_IN | FK_NT_OUT;
         } else if (i == 0) {
-            if (n >= 64 * MB) p->a.flags |= FK_NT_IN;
+            if (n >= 128 * MB) p->a.flags |= FK_NT_IN;
             if (n >= 1024 * MB) p->a.flags |= FK_NT_OUT;
         }
     }

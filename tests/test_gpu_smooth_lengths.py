@@ -1,6 +1,6 @@
 """Products of 2, 3, 5 and 7 as lines: one pass where the catalog holds the
-length (rows, columns, half of an even real line), and longer lines that are
-split only into the lengths that have every kernel a split needs.  Relative L2
+length (rows, columns, half of an even real line), and longer lines, which are
+split into the lengths kept for that.  Relative L2
 within the suite's bars (1e-13 FP64, 2e-6 FP32)."""
 import re
 
