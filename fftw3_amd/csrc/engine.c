@@ -400,6 +400,7 @@ typedef struct {
     const int *choice;          /* decisions to replay (NULL: all defaults) */
     int nchoice;
     int ci;                     /* decisions taken so far */
+    int seen;                   /* most decisions taken so far (chunks replay them) */
     int r16;                    /* restrict to radix-16 passes (FK_MFMA) */
     int part;                   /* planning a part of a split line */
     int bin, bout;              /* buffers of the r2c / c2r problem's arrays */
@@ -407,10 +408,16 @@ typedef struct {
     int dkind[FK_MAX_DECIDE];
 } ctx;
 
-static int decide(ctx *c, int nalt, int kind)
+/* one of nalt alternatives: the replayed decision, else def.  The numbering of
+   the alternatives must depend on the problem and the catalog alone (wisdom
+   stores the numbers and may be used on another device); what the device or
+   a heuristic prefers goes into def. */
+static int decide(ctx *c, int nalt, int kind, int def)
 {
-    int i = c->ci++, v = 0;
+    int i = c->ci++, v = def;
     if (i < FK_MAX_DECIDE && c->choice && i < c->nchoice) v = c->choice[i];
+    else if (i < c->seen && i < FK_MAX_DECIDE) v = c->P->choice[i]; /* a later chunk */
+    if (c->seen <= i) c->seen = i + 1;
     if (v >= nalt) v = nalt - 1;
     if (v < 0) v = 0;
     if (i < FK_MAX_DECIDE) {
@@ -454,36 +461,38 @@ static int forced(int prec, long long L, int mode, int io)
 
 static long long batch_count(int nb, const fk_dim *b);
 
-/* lines: how many the pass has (0: not known here) */
+/* The kernel of vs[0..n), the catalog variants of one (prec, L, mode, io), that
+   a pass of `lines` lines (0: not known here) takes by default: vs[0], or,
+   where that geometry would leave half the CUs without a workgroup, the same
+   kernel with half the lines per workgroup, where there is one (same results;
+   us, one transform, FFTW_ESTIMATE: FP32 2^20
+   24.4 -> 19.3, 1024^2 18.4 -> 16.2, 512^2 10.3 -> 8.6, FP64 2^18 17.2 ->
+   12.3).  Not where two of them would share a CU (FP32 2^20 x 63 column pass
+   265 -> 288), nor in column tiles and transposed stores whose runs would fall
+   below 64 bytes (FP32 4096 x 56 x 18, both, 33 -> 41). */
+static int default_variant(int prec, int mode, int io, long long lines, const fk_kernel *const *vs,
+                           int n)
+{
+    int v, j;
+    if (vs[0]->loop || lines <= 0 || 2 * ((lines + vs[0]->nl - 1) / vs[0]->nl) > g_ncu) return 0;
+    if ((mode != FK_ROW || io == FK_IO_TOUT) && vs[0]->nl * (int)csz(prec) < 128) return 0;
+    for (v = 1; v < n; ++v) {
+        const fk_kernel *h = vs[v];
+        int same = !h->loop && h->tpl == vs[0]->tpl && 2 * h->nl == vs[0]->nl &&
+                   h->nrad == vs[0]->nrad;
+        for (j = 0; same && j < h->nrad; ++j) same = h->rad[j] == vs[0]->rad[j];
+        if (same) return v;
+    }
+    return 0;
+}
+
 static const fk_kernel *pick_variant(ctx *c, int prec, long long L, int mode, int io,
                                      long long lines)
 {
     const fk_kernel *vs[16];
     int n = find_variants(prec, L, mode, io, vs, 16), v;
     if (!n) return 0;
-    if (!vs[0]->loop && lines > 0 && 2 * ((lines + vs[0]->nl - 1) / vs[0]->nl) <= g_ncu &&
-        ((mode == FK_ROW && io != FK_IO_TOUT) || vs[0]->nl * (int)csz(prec) >= 128)) {
-        /* the default geometry would leave half the CUs without a workgroup:
-           the same kernel with half the lines per workgroup comes first, where
-           there is one (same results; us, one transform: FP32 2^20 24.5 ->
-           20.0, 1024^2 16.7 -> 14.8, 256^2 10.4 -> 8.9, 1024 x 64 5.0 -> 4.6,
-           FP64 256 x 256 4.5 -> 4.1).  Not where two of them would share a CU
-           (FP32 2^20 x 63 column pass 265 -> 288), nor in column tiles and
-           transposed stores whose runs would fall below 64 bytes (FP32
-           4096 x 56 x 18, both, 33 -> 41) */
-        for (v = 1; v < n; ++v) {
-            const fk_kernel *h = vs[v];
-            int j, same = !h->loop && h->tpl == vs[0]->tpl && 2 * h->nl == vs[0]->nl &&
-                          h->nrad == vs[0]->nrad;
-            for (j = 0; same && j < h->nrad; ++j) same = h->rad[j] == vs[0]->rad[j];
-            if (same) {
-                vs[v] = vs[0];
-                vs[0] = h;
-                break;
-            }
-        }
-    }
-    v = n > 1 ? decide(c, n, DEC_VARIANT) : 0;
+    v = n > 1 ? decide(c, n, DEC_VARIANT, default_variant(prec, mode, io, lines, vs, n)) : 0;
     return forced(prec, L, mode, io) ? g_force : vs[v];
 }
 
@@ -965,7 +974,7 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
             cand[ncand++] = 0;
             if (dT >= 0) cand[ncand++] = 1;
         }
-        m = cand[ncand > 1 ? decide(c, ncand, DEC_MODE) : 0];
+        m = cand[ncand > 1 ? decide(c, ncand, DEC_MODE, 0) : 0];
         if (m == 1 || m == 2) {
             int d = m == 1 ? dT : dC;
             fk_dim t = b[d];
@@ -1000,7 +1009,7 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
         const fk_kernel *kA;
         size_t before;
         if (!ncand) goto blue;
-        n1 = cands[ncand > 1 ? decide(c, ncand, DEC_SPLIT) : 0];
+        n1 = cands[ncand > 1 ? decide(c, ncand, DEC_SPLIT, 0) : 0];
         n2 = n / n1;
         H = batch_count(nb, b);
         kA = pick_variant(c, prec, n1, FK_COL, FK_IO_PLAIN, n2 * H);
@@ -1150,7 +1159,7 @@ static long long chunk_units(ctx *c, long long nunits, double unit_bytes)
         }
         return cand[1];
     }
-    return cand[decide(c, nc, DEC_CHUNK)];
+    return cand[decide(c, nc, DEC_CHUNK, 0)];
 }
 
 typedef int (*chunk_fn)(ctx *c, const fk_problem *q, int sw);
@@ -1500,7 +1509,7 @@ static int plan_r2c(ctx *c, const fk_problem *pb)
         fk_dim xe[1];
         int nxe = 0;
         const fk_kernel *kx = xr_kernel(c, pb, FK_IO_R2C_XR, xe, &nxe);
-        if (kx && decide(c, 2, DEC_VARIANT) == 0) return plan_r2c_xr(c, pb, kx, xe, nxe);
+        if (kx && decide(c, 2, DEC_VARIANT, 0) == 0) return plan_r2c_xr(c, pb, kx, xe, nxe);
     }
     if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_R2C, batch_count(nb, b));
     if (k) {
@@ -1636,7 +1645,7 @@ static int plan_c2r(ctx *c, const fk_problem *pb)
         fk_dim xe[1];
         int nxe = 0;
         const fk_kernel *kx = xr_kernel(c, pb, FK_IO_C2R_XR, xe, &nxe);
-        if (kx && decide(c, 2, DEC_VARIANT) == 0) return plan_c2r_xr(c, pb, kx, xe, nxe);
+        if (kx && decide(c, 2, DEC_VARIANT, 0) == 0) return plan_c2r_xr(c, pb, kx, xe, nxe);
     }
     /* leading dims first: backward c2c in place on the input (destroys it,
        api/plan-many-dft-c2r.c:41-42) */
@@ -2703,7 +2712,9 @@ static fk_plan *plan_internal(const fk_problem *pb, hipStream_t st)
             if (g_timelimit >= 0 && now_s() - t0 > g_timelimit) goto done;
             memcpy(trial, cur, sizeof(int) * ncur);
             trial[i] = a;
-            Q = build_plan(pb, st, trial, ncur, &cq);
+            /* what follows decision i takes its defaults (nothing after i has
+               been searched yet, and alternative a may lead to other ones) */
+            Q = build_plan(pb, st, trial, i + 1, &cq);
             if (!Q) continue;
             Q->rot = rot.buf;
             Q->nrot = rot.n;

@@ -1,0 +1,139 @@
+"""The planner's own rules on the CPU: a C program that includes the engine's
+source and runs its planning functions on the built catalog, without a device
+(no array, table or launch is made)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "fftw3_amd")
+ROCM = "/opt/rocm"
+
+HEAD = r"""
+#include "engine.c"
+static long long bad, seen;
+#define CHECK(c, ...) do { ++seen; if (!(c) && bad++ < 20) printf(__VA_ARGS__); } while (0)
+static void start(void) { g_reg = fk_registry(&g_nreg); index_catalog(); }
+static fk_plan *begin(ctx *c, int prec)
+{
+    fk_plan *P = (fk_plan *)calloc(1, sizeof(fk_plan));
+    P->prec = prec;
+    memset(c, 0, sizeof(*c));
+    c->P = P;
+    c->bin = FK_BUF_IN;
+    c->bout = FK_BUF_OUT;
+    return P;
+}
+"""
+
+
+def run(tmp_path, body):
+    if not os.path.exists(os.path.join(ROCM, "lib", "libamdhip64.so")):
+        pytest.skip("no HIP runtime to link against")
+    src = tmp_path / "t.c"
+    src.write_text(HEAD + body)
+    exe = str(tmp_path / "t")
+    subprocess.check_call(["gcc", "-std=gnu11", "-O1", "-w", "-D__HIP_PLATFORM_AMD__",
+                           "-I" + os.path.join(PKG, "csrc"), "-I" + os.path.join(ROCM, "include"),
+                           "-o", exe, str(src), "-L" + PKG, "-lfftw3_amd", "-L" + ROCM + "/lib",
+                           "-lamdhip64", "-lpthread", "-lm", "-Wl,-rpath," + PKG,
+                           "-Wl,-rpath," + ROCM + "/lib"])
+    out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout
+    *msgs, last = out.strip().split("\n")
+    bad, seen = map(int, last.split())
+    assert bad == 0, "\n".join(msgs)
+    assert seen > 0
+    return seen
+
+
+def test_stored_choice_is_the_same_kernel_on_any_device(tmp_path):
+    """A decision vector made on one device names the same kernels on another:
+    for every catalog key with alternatives, the default picked with 256, 64 and
+    8 compute units and every explicit choice resolve to the same entry wherever
+    they are replayed."""
+    run(tmp_path, r"""
+int main(void)
+{
+    static const int ncu[] = {256, 64, 8};
+    static const long long lines[] = {0, 1, 3, 16, 100, 700, 5000, 1LL << 33};
+    int i, a, b, l;
+    start();
+    for (i = 0; i < g_nreg; ++i) {
+        const fk_kernel *k = g_reg + i, *vs[16];
+        int n = find_variants(k->prec, k->L, k->mode, k->io, vs, 16), v;
+        if (k->variant || n < 2) continue;
+        for (l = 0; l < 8; ++l)
+            for (a = 0; a < 3; ++a)
+                for (v = -1; v < n; ++v) {
+                    const fk_kernel *first;
+                    ctx c;
+                    fk_plan *P = begin(&c, k->prec);
+                    int made = v;
+                    g_ncu = ncu[a];
+                    c.choice = v < 0 ? 0 : &made;
+                    c.nchoice = v >= 0;
+                    first = pick_variant(&c, k->prec, k->L, k->mode, k->io, lines[l]);
+                    made = P->choice[0];
+                    CHECK(v < 0 || first == vs[v], "L=%d choice %d\n", k->L, v);
+                    for (b = 0; b < 3; ++b) {
+                        ctx d;
+                        fk_plan *Q = begin(&d, k->prec);
+                        g_ncu = ncu[b];
+                        d.choice = &made;
+                        d.nchoice = 1;
+                        CHECK(pick_variant(&d, k->prec, k->L, k->mode, k->io, lines[l]) == first,
+                              "L=%d mode=%d io=%d lines=%lld made at %d CUs, replayed at %d\n", k->L,
+                              k->mode, k->io, lines[l], ncu[a], ncu[b]);
+                        free(Q);
+                    }
+                    free(P);
+                }
+    }
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
+
+
+def test_half_the_lines_where_the_grid_is_small(tmp_path):
+    """The default geometry of a pass: half the lines per workgroup exactly where
+    the catalog has such a variant, at most every other compute unit would have a
+    workgroup, and column runs (transposed stores) stay at 64 bytes; on either
+    side of the limit, with whole and ragged last tiles."""
+    run(tmp_path, r"""
+int main(void)
+{
+    int i, v, t, half = 0;
+    start();
+    g_ncu = 256;
+    for (i = 0; i < g_nreg; ++i) {
+        const fk_kernel *k = g_reg + i, *vs[16], *h = 0;
+        int n = find_variants(k->prec, k->L, k->mode, k->io, vs, 16);
+        static const long long tiles[] = {1, 2, 127, 128, 129, 256, 4000};
+        if (k->variant) continue;
+        for (v = 1; v < n && !h; ++v)
+            if (!vs[v]->loop && vs[v]->tpl == k->tpl && 2 * vs[v]->nl == k->nl &&
+                vs[v]->nrad == k->nrad && !memcmp(vs[v]->rad, k->rad, sizeof(int) * k->nrad))
+                h = vs[v];
+        for (t = 0; t < 7; ++t) {
+            long long end[2] = {tiles[t] * k->nl, tiles[t] * k->nl - k->nl + 1};
+            for (v = 0; v < 2; ++v) {
+                ctx c;
+                fk_plan *P = begin(&c, k->prec);
+                const int wide = k->mode == FK_ROW && k->io != FK_IO_TOUT;
+                const int run = k->nl * (k->prec ? 8 : 16);
+                const int take = h && !k->loop && tiles[t] <= 128 && (wide || run >= 128);
+                const fk_kernel *p = pick_variant(&c, k->prec, k->L, k->mode, k->io, end[v]);
+                CHECK(p == (take ? h : k), "prec=%d L=%d mode=%d io=%d lines=%lld: nl %d\n",
+                      k->prec, k->L, k->mode, k->io, end[v], p->nl);
+                half += take;
+                free(P);
+            }
+        }
+    }
+    CHECK(half > 100, "only %d cases take the half-lines kernel\n", half);
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
