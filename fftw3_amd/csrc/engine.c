@@ -1491,6 +1491,25 @@ static int plan_c2r_xr(ctx *c, const fk_problem *pb, const fk_kernel *kx, const 
     return c->err ? -1 : 0;
 }
 
+/* Whether the fused real kernels may run: out of place, on one line, or in
+   place on rows that each keep to their own place (real row 2 d apart, complex
+   row d apart, unit strides).  In any other in-place layout a line's outputs lie
+   on other lines' inputs, which another workgroup may not have read yet; the
+   staged forms read the whole input before they write. */
+static int real_lines_apart(const ctx *c, const fk_problem *pb)
+{
+    const fk_dim *l = pb->dims + pb->rank - 1;
+    int i, rows = l->is == 1 && l->os == 1, many = 0;
+    if (pb->in != pb->out || c->bin != FK_BUF_IN || c->bout != FK_BUF_OUT) return 1;
+    for (i = 0; i < pb->rank - 1 + pb->vrank; ++i) {
+        const fk_dim *d = i < pb->rank - 1 ? pb->dims + i : pb->vdims + i - (pb->rank - 1);
+        if (d->n == 1) continue;
+        many = 1;
+        rows &= pb->kind == FK_R2C ? d->is == 2 * d->os : d->os == 2 * d->is;
+    }
+    return rows || !many;
+}
+
 static int plan_r2c(ctx *c, const fk_problem *pb)
 {
     fk_plan *P = c->P;
@@ -1498,7 +1517,7 @@ static int plan_r2c(ctx *c, const fk_problem *pb)
     size_t cs = csz(prec), rs = rsz(prec);
     long long nl = pb->dims[r - 1].n, nh = nl / 2 + 1, L = nl / 2;
     fk_dim b[FK_MAXRANK * 2], lead[FK_MAXRANK];
-    int nb = 0;
+    int nb = 0, apart;
     const fk_kernel *k = 0;
     /* batch for the last-dim pass: leading dims + vdims */
     for (i = 0; i < r - 1; ++i) b[nb++] = pb->dims[i];
@@ -1511,7 +1530,9 @@ static int plan_r2c(ctx *c, const fk_problem *pb)
         const fk_kernel *kx = xr_kernel(c, pb, FK_IO_R2C_XR, xe, &nxe);
         if (kx && decide(c, 2, DEC_VARIANT, 0) == 0) return plan_r2c_xr(c, pb, kx, xe, nxe);
     }
-    if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_R2C, batch_count(nb, b));
+    apart = real_lines_apart(c, pb);
+    if (apart && nl % 2 == 0)
+        k = pick_variant(c, prec, L, FK_ROW, FK_IO_R2C, batch_count(nb, b));
     if (k) {
         size_t before = (size_t)P->npass;
         unsigned fl = 0;
@@ -1529,7 +1550,7 @@ static int plan_r2c(ctx *c, const fk_problem *pb)
         }
         if (unit) need_align(c, c->bin, (unsigned)(2 * rs));
         desc_add(P, "(r2c-fused L=%lld)", L);
-    } else if ((k = pick_variant(c, prec, nl, FK_ROW, FK_IO_R2C_FULL, 0)) != 0) {
+    } else if (apart && (k = pick_variant(c, prec, nl, FK_ROW, FK_IO_R2C_FULL, 0)) != 0) {
         /* one pass: full-length DFT of the real line, half the bins stored */
         size_t before = (size_t)P->npass;
         emit_stockham(c, k, pb->dims[r - 1].is, pb->dims[r - 1].os, nb, b, c->bin, 0, c->bout, 0,
@@ -1639,7 +1660,7 @@ static int plan_c2r(ctx *c, const fk_problem *pb)
     size_t cs = csz(prec), rs = rsz(prec);
     long long nl = pb->dims[r - 1].n, nh = nl / 2 + 1, L = nl / 2;
     fk_dim b[FK_MAXRANK * 2], lead[FK_MAXRANK];
-    int nb = 0;
+    int nb = 0, apart;
     const fk_kernel *k = 0;
     {
         fk_dim xe[1];
@@ -1670,7 +1691,9 @@ static int plan_c2r(ctx *c, const fk_problem *pb)
     for (i = 0; i < pb->vrank; ++i) b[nb++] = pb->vdims[i];
     nb = squeeze(nb, b);
     sort_by_is(nb, b);
-    if (nl % 2 == 0) k = pick_variant(c, prec, L, FK_ROW, FK_IO_C2R, batch_count(nb, b));
+    apart = real_lines_apart(c, pb);
+    if (apart && nl % 2 == 0)
+        k = pick_variant(c, prec, L, FK_ROW, FK_IO_C2R, batch_count(nb, b));
     if (k) {
         size_t before = (size_t)P->npass;
         unsigned fl = 0;
@@ -1688,7 +1711,7 @@ static int plan_c2r(ctx *c, const fk_problem *pb)
         }
         if (unit) need_align(c, c->bout, (unsigned)(2 * rs));
         desc_add(P, "(c2r-fused L=%lld)", L);
-    } else if ((k = pick_variant(c, prec, nl, FK_ROW, FK_IO_C2R_FULL, 0)) != 0) {
+    } else if (apart && (k = pick_variant(c, prec, nl, FK_ROW, FK_IO_C2R_FULL, 0)) != 0) {
         /* one pass: Hermitian expansion on load, real part on store */
         size_t before = (size_t)P->npass;
         emit_stockham(c, k, pb->dims[r - 1].is, pb->dims[r - 1].os, nb, b, c->bin, 0, c->bout, 0,
