@@ -642,6 +642,8 @@ static void emit_loops(ctx *c, const fk_pass *proto, int nb, const fk_dim *b0, s
     long long idx[FK_MAXRANK * 2] = {0};
     int nloop = nb > 3 ? nb - 3 : 0, i, j;
     fk_dim b[FK_MAXRANK * 2];
+    const int seq = c->P->nseq++;
+    const long long lines = batch_count(nb, b0);
     memcpy(b, b0, sizeof(fk_dim) * nb);
     /* beyond three batch dims, keep the two largest after b[0] (whose place
        the thread mapping may depend on) in the kernel and loop over the
@@ -668,6 +670,8 @@ static void emit_loops(ctx *c, const fk_pass *proto, int nb, const fk_dim *b0, s
         p->ooff = ooff;
         p->i2off = i2off;
         p->o2off = o2off;
+        p->seq = seq;
+        p->lines = lines;
         if (p->type == FK_PASS_STOCKHAM) {
             fill_batch3(p->a.nb, p->a.ids, p->a.ods, &p->a.nlines, nb < 3 ? nb : 3, b);
             p->grid = (unsigned)((p->a.nlines + p->k->nl - 1) / p->k->nl);
@@ -2342,17 +2346,18 @@ static void mark_streams(fk_plan *P)
         fk_pass *p = P->pass + i;
         long long n;
         if (p->type != FK_PASS_STOCKHAM || p->k->mode != FK_ROW) continue;
-        n = p->a.nlines * p->k->L * (long long)csz(p->k->prec);
+        /* bytes of the logical pass: its launches are alike */
+        n = p->lines * p->k->L * (long long)csz(p->k->prec);
         if (p->k->io == FK_IO_R2C_RR) {
-            if (i == 0 && n >= 64 * MB && (p->k->prec == 1 || P->npass > 1))
+            if (p->seq == 0 && n >= 64 * MB && (p->k->prec == 1 || P->nseq > 1))
                 p->a.flags |= FK_NT_IN;
             continue;
         }
         if (p->k->io != FK_IO_PLAIN || p->k->prec != 0 || !whole_sectors(p)) continue;
-        if (P->npass == 1) {
+        if (P->nseq == 1) {
             if (n >= 16 * MB && (!p->k->loop || n <= 512 * MB))
                 p->a.flags |= FK_NT_IN | FK_NT_OUT;
-        } else if (i == 0) {
+        } else if (p->seq == 0) {
             if (n >= 128 * MB) p->a.flags |= FK_NT_IN;
             if (n >= 1024 * MB) p->a.flags |= FK_NT_OUT;
         }

@@ -70,6 +70,9 @@ typedef struct {
     int i2buf, o2buf;           /* second input / output (split ops), -1 none */
     long long i2off, o2off;
     unsigned grid, block, lds;
+    int seq;                    /* logical pass of the plan: launches that share
+                                   a pass's batch dims have the same number */
+    long long lines;            /* lines of all launches of the logical pass */
     double bytes;               /* HBM bytes the pass moves (estimate) */
 } fk_pass;
 
@@ -84,6 +87,7 @@ typedef struct fk_plan {
     void *in2, *out2;           /* imaginary arrays at planning (FK_SPLIT_GENERAL) */
     int r2r[FK_MAXRANK];        /* FK_R2R: kind of each dim */
     int npass, cpass;
+    int nseq;                   /* logical passes */
     fk_pass *pass;
     int nscratch;
     size_t scratch_bytes[FK_MAX_SCRATCH];

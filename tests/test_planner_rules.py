@@ -137,3 +137,61 @@ int main(void)
     return 0;
 }
 """)
+
+
+EMIT = r"""
+/* one logical pass of kernel (prec, L, mode, io) over batch dims b, as the
+   planner emits it but without its tables */
+static void emit(ctx *c, int prec, int L, int io, int nb, const fk_dim *b, int ibuf, int obuf)
+{
+    fk_pass p;
+    memset(&p, 0, sizeof(p));
+    p.type = FK_PASS_STOCKHAM;
+    p.k = find_kernel(prec, L, FK_ROW, io);
+    p.ibuf = ibuf;
+    p.obuf = obuf;
+    p.a.is = p.a.os = 1;
+    emit_loops(c, &p, nb, b, prec ? 8 : 16, prec ? 8 : 16);
+}
+static unsigned nt(const fk_plan *P, int i) { return P->pass[i].a.flags & (FK_NT_IN | FK_NT_OUT); }
+"""
+
+
+def test_cache_rules_take_a_pass_with_its_loops(tmp_path):
+    """Batch dims beyond the three that a launch addresses become several launches
+    of one logical pass: all of them get the same cache flags, by the size of the
+    whole pass and by whether it is the plan's only or first one."""
+    run(tmp_path, EMIT + r"""
+int main(void)
+{
+    int m, one, i;
+    start();
+    for (one = 0; one < 2; ++one)
+        for (m = 1; m <= 1024; m *= 4) {
+            /* 512-point FP64 lines, five batch dims that do not merge: 6 * 5
+               launches of m * 64 lines */
+            fk_dim b[5] = {{8, 520, 520}, {8, 8320, 8320}, {m, 133120, 133120},
+                           {6, 133120LL * (m + 1), 133120LL * (m + 1)},
+                           {5, 133120LL * (m + 1) * 8, 133120LL * (m + 1) * 8}};
+            const long long bytes = 30LL * 64 * m * 512 * 16, MB = 1 << 20;
+            unsigned want0;
+            int n0;
+            ctx c;
+            fk_plan *P = begin(&c, 0);
+            emit(&c, 0, 512, FK_IO_PLAIN, 5, b, FK_BUF_IN, FK_BUF_OUT);
+            n0 = P->npass;
+            CHECK(n0 > 1, "one launch only\n");
+            if (!one) emit(&c, 0, 512, FK_IO_PLAIN, 5, b, FK_BUF_OUT, FK_BUF_OUT);
+            mark_streams(P);
+            if (one) want0 = bytes >= 16 * MB ? FK_NT_IN | FK_NT_OUT : 0;
+            else want0 = (bytes >= 128 * MB ? FK_NT_IN : 0) | (bytes >= 1024 * MB ? FK_NT_OUT : 0);
+            for (i = 0; i < P->npass; ++i)
+                CHECK(nt(P, i) == (i < n0 ? want0 : 0), "%s pass, %lld MiB, launch %d of %d: %u\n",
+                      one ? "only" : i < n0 ? "first" : "second", bytes / MB, i, P->npass, nt(P, i));
+            free(P->pass);
+            free(P);
+        }
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
