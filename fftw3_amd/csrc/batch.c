@@ -209,9 +209,7 @@ fk_batch *fk_batch_create(int prec, int ngroups, const int *n, const int *howman
             b->htab[p] = (fk_bpass *)realloc(b->htab[p], sizeof(fk_bpass) * (b->npass[p] + 1));
             e = b->htab[p] + b->npass[p]++;
             memset(e, 0, sizeof(*e));
-            e->a = ps->a;
-            e->a.in = (const char *)buf[ps->ibuf] + ps->ioff;
-            e->a.out = (char *)buf[ps->obuf] + ps->ooff;
+            fk_bind_pass(ps, buf, &e->a);
             e->kind = kind;
             e->tiles = (ps->a.nlines + menu[kind].nl - 1) / menu[kind].nl;
             e->first = b->total[p];

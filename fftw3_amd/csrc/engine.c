@@ -2814,18 +2814,38 @@ void fk_plan_set_stream(fk_plan *p, hipStream_t s)
 /* ------------------------------------------------------------------ */
 /* execution                                                           */
 
+/* Access forms that need more alignment than the plan asks of its arrays are
+   taken or not by the arrays of this call: the quads and pairs of the
+   real-to-real kernels, and the non-temporal accesses of short FP64 rows.  On
+   arrays off a 64-byte boundary every access of a row starts and ends inside a
+   sector that its neighbour fetches again; with 256 bytes and more per access
+   (16 threads a line) that costs less than the non-temporal form gains (us, 64
+   MiB arrays 16 bytes off, cached / non-temporal: 32 points, 4 threads, 33.5 /
+   72; 64, 8 threads, 26.1 / 33.1; 128, 8 threads, 34.6 / 53.3; 256, 16 threads,
+   29.2 / 28.1; 512, 64 threads, 28.4 / 26.1).  The quads of REDFT10 / RODFT10
+   rows gain at every length (FP32 2048 x 32768 141 / 109). */
+void fk_bind_pass(const fk_pass *ps, void *const *buf, fk_args *a)
+{
+    *a = ps->a;
+    a->in = (const char *)buf[ps->ibuf] + ps->ioff;
+    a->out = (char *)buf[ps->obuf] + ps->ooff;
+    if ((a->flags & FK_REAL_QUAD) &&
+        ((uintptr_t)(ps->k->io == FK_IO_R2C_RR ? a->in : (const void *)a->out) % 16))
+        a->flags &= ~FK_REAL_QUAD;
+    if (ps->k->io == FK_IO_DCT4 && (((uintptr_t)a->in | (uintptr_t)a->out) % (2 * rsz(ps->k->prec))))
+        a->flags &= ~FK_REAL_UNIT;
+    if (ps->k->io == FK_IO_PLAIN && ps->k->tpl < 16) {
+        if ((uintptr_t)a->in % 64) a->flags &= ~FK_NT_IN;
+        if ((uintptr_t)a->out % 64) a->flags &= ~FK_NT_OUT;
+    }
+}
+
 static int launch_pass(const fk_pass *ps, void *const *buf, hipStream_t st, int prec)
 {
     if (ps->type == FK_PASS_STOCKHAM) {
-        fk_args a = ps->a;
+        fk_args a;
         void *args[1];
-        a.in = (const char *)buf[ps->ibuf] + ps->ioff;
-        a.out = (char *)buf[ps->obuf] + ps->ooff;
-        if ((a.flags & FK_REAL_QUAD) &&
-            ((uintptr_t)(ps->k->io == FK_IO_R2C_RR ? a.in : (const void *)a.out) % 16))
-            a.flags &= ~FK_REAL_QUAD;
-        if (ps->k->io == FK_IO_DCT4 && (((uintptr_t)a.in | (uintptr_t)a.out) % (2 * rsz(prec))))
-            a.flags &= ~FK_REAL_UNIT;
+        fk_bind_pass(ps, buf, &a);
         args[0] = &a;
         return (int)hipLaunchKernel(ps->k->fn, (dim3){ps->grid, 1, 1}, (dim3){ps->block, 1, 1},
                                     args, ps->lds, st);

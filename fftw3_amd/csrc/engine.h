@@ -191,6 +191,9 @@ void fk_batch_destroy(fk_batch *b);
 int fk_plan_use_mfma(fk_plan *p);
 int fkm_mfma_probe(float *dev_out, hipStream_t st);
 int fk_enqueue(fk_plan *p, void *in, void *out, hipStream_t st);
+/* the arguments of a Stockham pass on the arrays buf[] (by FK_BUF_*): every
+   launch and work table takes them from here */
+void fk_bind_pass(const fk_pass *ps, void *const *buf, fk_args *a);
 int fk_enqueue_bound(fk_plan *p, void *in, void *out, void *const *scratch, hipStream_t st);
 int fkm_reset_counters(unsigned long long *c, int n, hipStream_t st);
 

@@ -300,9 +300,7 @@ static int launch_round(fk_server *s, sround *r)
             int kind = fk_menu_kind(s->menu[P->prec], s->nmenu[P->prec], ps->k);
             fk_bpass *e = r->htab[P->prec][j] + np[P->prec][j]++;
             memset(e, 0, sizeof(*e));
-            e->a = ps->a;
-            e->a.in = (const char *)buf[ps->ibuf] + ps->ioff;
-            e->a.out = (char *)buf[ps->obuf] + ps->ooff;
+            fk_bind_pass(ps, buf, &e->a);
             e->kind = kind;
             e->tiles = (ps->a.nlines + s->menu[P->prec][kind].nl - 1) / s->menu[P->prec][kind].nl;
             e->first = tot[P->prec][j];
