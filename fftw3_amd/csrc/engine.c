@@ -2316,7 +2316,10 @@ static void fill_magic(fk_args *a)
      the first pass of several: its input from 128 MiB on, where input and
      output together exceed the memory-side cache (512x512 x 64 203 -> 182, x
      128 410 -> 391; 2048x2048 x 1 56.0 -> 58.2 and x 4 of 512x512 19.4 -> 19.9
-     the other way),
+     the other way); in place, where there is one array, from 384 MiB on
+     (2048x2048 x 6 387 -> 343, 4096x4096 x 2 664 -> 658, 256x256 x 384 265 ->
+     255; 2048x2048 x 3 165 -> 187, 4096x4096 x 1 263 -> 304, 256x256 x 256 167
+     -> 180 the other way);
      its output, which the next pass reads, from 1 GiB on, four times the
      memory-side cache (512x512 x 256 775 -> 760; x 64 182 -> 208 the other
      way).
@@ -2358,7 +2361,8 @@ static void mark_streams(fk_plan *P)
             if (n >= 16 * MB && (!p->k->loop || n <= 512 * MB))
                 p->a.flags |= FK_NT_IN | FK_NT_OUT;
         } else if (p->seq == 0) {
-            if (n >= 128 * MB) p->a.flags |= FK_NT_IN;
+            const int one = P->inplace && p->ibuf == FK_BUF_IN && p->obuf == FK_BUF_OUT;
+            if (n >= (one ? 384 : 128) * MB) p->a.flags |= FK_NT_IN;
             if (n >= 1024 * MB) p->a.flags |= FK_NT_OUT;
         }
     }

@@ -241,3 +241,35 @@ int main(void)
     return 0;
 }
 """)
+
+
+def test_first_pass_reads_past_the_caches_by_its_footprint(tmp_path):
+    """The first of several FP64 row passes reads non-temporally when its arrays
+    exceed the memory-side cache: from 128 MiB each for two arrays, from 384 MiB
+    for one that is transformed in place; through staging counts as two."""
+    run(tmp_path, EMIT + r"""
+int main(void)
+{
+    const long long MB = 1 << 20;
+    int mb, how;
+    start();
+    for (how = 0; how < 3; ++how) /* out of place, in place, in place into staging */
+        for (mb = 64; mb <= 1024; mb += 64) {
+            fk_dim b[1] = {{mb * MB / (512 * 16), 512, 512}};
+            const int mid = how == 2 ? FK_BUF_S0 : FK_BUF_OUT;
+            const unsigned want = mb >= (how == 1 ? 384 : 128) ? FK_NT_IN : 0;
+            ctx c;
+            fk_plan *P = begin(&c, 0);
+            P->inplace = how > 0;
+            emit(&c, 0, 512, FK_IO_PLAIN, 1, b, FK_BUF_IN, mid);
+            emit(&c, 0, 512, FK_IO_PLAIN, 1, b, mid, FK_BUF_OUT);
+            mark_streams(P);
+            CHECK((nt(P, 0) & FK_NT_IN) == want && !nt(P, 1), "how=%d %d MiB: %u %u\n", how, mb,
+                  nt(P, 0), nt(P, 1));
+            free(P->pass);
+            free(P);
+        }
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
