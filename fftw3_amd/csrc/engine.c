@@ -2822,12 +2822,14 @@ void fk_plan_set_stream(fk_plan *p, hipStream_t s)
    taken or not by the arrays of this call: the quads and pairs of the
    real-to-real kernels, and the non-temporal accesses of short FP64 rows.  On
    arrays off a 64-byte boundary every access of a row starts and ends inside a
-   sector that its neighbour fetches again; with 256 bytes and more per access
-   (16 threads a line) that costs less than the non-temporal form gains (us, 64
-   MiB arrays 16 bytes off, cached / non-temporal: 32 points, 4 threads, 33.5 /
-   72; 64, 8 threads, 26.1 / 33.1; 128, 8 threads, 34.6 / 53.3; 256, 16 threads,
-   29.2 / 28.1; 512, 64 threads, 28.4 / 26.1).  The quads of REDFT10 / RODFT10
-   rows gain at every length (FP32 2048 x 32768 141 / 109). */
+   sector that its neighbour fetches again; where a wave's lanes cover lines in
+   pieces of 256 bytes and more (16, 32, 64 ... threads a line) that costs less
+   than the non-temporal form gains (us, 64 MiB arrays 16 bytes off, cached /
+   non-temporal: 32 points, 4 threads, 33.5 / 72; 64, 8 threads, 26.1 / 33.1;
+   128, 8 threads, 34.6 / 53.3; 320, 40 threads, 29.3 / 33.5; 256, 16 threads,
+   29.2 / 28.1; 512, 64 threads, 28.4 / 26.1; 1024, 64 threads, 16 MiB 9.7 /
+   9.0).  The quads of REDFT10 / RODFT10 rows gain at every length (FP32 2048 x
+   32768 141 / 109). */
 void fk_bind_pass(const fk_pass *ps, void *const *buf, fk_args *a)
 {
     *a = ps->a;
@@ -2838,7 +2840,7 @@ void fk_bind_pass(const fk_pass *ps, void *const *buf, fk_args *a)
         a->flags &= ~FK_REAL_QUAD;
     if (ps->k->io == FK_IO_DCT4 && (((uintptr_t)a->in | (uintptr_t)a->out) % (2 * rsz(ps->k->prec))))
         a->flags &= ~FK_REAL_UNIT;
-    if (ps->k->io == FK_IO_PLAIN && ps->k->tpl < 16) {
+    if (ps->k->io == FK_IO_PLAIN && (ps->k->tpl < 16 || (ps->k->tpl & (ps->k->tpl - 1)))) {
         if ((uintptr_t)a->in % 64) a->flags &= ~FK_NT_IN;
         if ((uintptr_t)a->out % 64) a->flags &= ~FK_NT_OUT;
     }
