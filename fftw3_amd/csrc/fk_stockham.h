@@ -591,7 +591,13 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
            What bounds it: the twiddle loads of its three stages and of the
            post-pass outnumber the data loads and live in the CU's L1, which
            the data streams through.  Data read past L1 (C_ONCE) leaves the
-           tables there: FP32 2048 x 65536 0.246 -> 0.205 ms. */
+           tables there: FP32 2048 x 65536 0.246 -> 0.205 ms.  Not where few
+           threads read a line: a sector that several loads share is then
+           fetched by each of them (64 MiB of FP32 input, us cached / C_ONCE:
+           14 samples, 1 thread, 58 / 69; 52, 2 threads, 47 / 60; 36, 3 threads,
+           46 / 50; 84, 6 threads, 45 / 39; with 4 threads only lines that start
+           at a sector: 64 samples 53 / 41, 56 samples 42 / 45). */
+        constexpr int ONCE = TPL >= 6 || (TPL == 4 && L % 8 == 0) ? C_ONCE : C_KEEP;
         const R *inr = reinterpret_cast<const R *>(a.in) + bin;
         cx<R> *out = reinterpret_cast<cx<R> *>(a.out);
         const cx<R> *wk = reinterpret_cast<const cx<R> *>(a.aux);
@@ -599,7 +605,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
         auto gld = hoisted([&](auto &&load) {
             if (fl & FK_REAL_UNIT) {
                 const cx<R> *inz = reinterpret_cast<const cx<R> *>(inr) + u;
-                load([&](int j) -> cx<R> { return ldg(Acc<C_ONCE>{}, inz + (j - u)); });
+                load([&](int j) -> cx<R> { return ldg(Acc<ONCE>{}, inz + (j - u)); });
             } else {
                 asm volatile("");
                 const R *inu = inr + 2 * u * is;
@@ -810,7 +816,10 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             __syncthreads();
         } else {
             /* loads in groups of 8 (compile-time count) so that each group
-               is in flight at once, then its LDS stores */
+               is in flight at once, then its LDS stores; through L1, since
+               the bins k and L-k of short lines share sectors (64 MiB of FP32
+               output, us with C_ONCE / this: 30 samples 49.6 / 39.6, 64 41.1 /
+               32.1, 128 33.4 / 28.2, 320 36.7 / 33.2; from 512 on the same) */
             const cx<R> *ink = in + bin + u * is, *inm = in + bin + (L - u) * is;
             sfor<0, (NK2 + GK - 1) / GK>([&](auto gc) {
                 constexpr int g = decltype(gc)::value;
@@ -821,8 +830,8 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                     const int k = u + (g * GK + i) * TPL;
                     const long long d = (long long)((g * GK + i) * TPL) * is;
                     if (k <= HK) {
-                        xa[i] = ldg(Acc<C_ONCE>{}, ink + d);
-                        xb[i] = ldg(Acc<C_ONCE>{}, inm - d);
+                        xa[i] = ink[d];
+                        xb[i] = inm[-d];
                         w[i] = wk[k];
                     }
                 });
@@ -990,10 +999,14 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                     }
                 });
             } else if (fl & FK_REAL_UNIT) {
+                /* past L1 where a line has 8 threads and more (see FK_IO_R2C;
+                   R2HC of 64 samples, 4 threads, is a tenth faster through L1,
+                   of 128 the same) */
                 each([&](auto ic, auto rc, int b) {
                     constexpr int r = decltype(rc)::value;
                     v[decltype(ic)::value][r] =
-                        ldg(Acc<C_ONCE>{}, reinterpret_cast<const cx<R> *>(inr) + b + r * NB0);
+                        ldg(Acc<(TPL >= 8 ? C_ONCE : C_KEEP)>{},
+                            reinterpret_cast<const cx<R> *>(inr) + b + r * NB0);
                 });
             } else {
                 asm volatile("");
