@@ -496,6 +496,19 @@ static const fk_kernel *pick_variant(ctx *c, int prec, long long L, int mode, in
     return forced(prec, L, mode, io) ? g_force : vs[v];
 }
 
+/* The row kernel of a fused real-to-real kind.  Where the catalog has two forms
+   (gen_kernels.py, rr_forms), the first, mirrored, is the default of the kinds
+   that read or write quads, the second of the others. */
+static const fk_kernel *pick_rr_row(ctx *c, int prec, long long L, int io, int rm)
+{
+    const fk_kernel *vs[16];
+    const int quads = rm == FK_RM_DCT2 || rm == FK_RM_DST2 || rm == FK_RM_DCT3 || rm == FK_RM_DST3;
+    int n = find_variants(prec, L, FK_ROW, io, vs, 16), v;
+    if (!n) return 0;
+    v = n > 1 ? decide(c, n, DEC_VARIANT, !quads) : 0;
+    return forced(prec, L, FK_ROW, io) ? g_force : vs[v];
+}
+
 int fk_catalog_size(void)
 {
     if (!g_reg) g_reg = fk_registry(&g_nreg);
@@ -1950,7 +1963,7 @@ static int plan_r2r_1d(ctx *c, int kind, long long n, long long is, long long os
                 b[0] = t;
             }
         }
-        if (ok && !k) k = pick_variant(c, prec, L, FK_ROW, io, 0);
+        if (ok && !k) k = pick_rr_row(c, prec, L, io, rm);
         if (k) {
             size_t before = (size_t)P->npass;
             unsigned fl = 0;

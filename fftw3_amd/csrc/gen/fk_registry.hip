@@ -43,7 +43,7 @@ extern "C" const fk_kernel *fk_registry(int *count)
     if (!all) {
         int n, off = 0;
         const fk_kernel *t;
-        fk_kernel *buf = (fk_kernel *)malloc(sizeof(fk_kernel) * 2571);
+        fk_kernel *buf = (fk_kernel *)malloc(sizeof(fk_kernel) * 2615);
         t = fk_registry_part0(&n); memcpy(buf + off, t, sizeof(fk_kernel) * n); off += n;
         t = fk_registry_part1(&n); memcpy(buf + off, t, sizeof(fk_kernel) * n); off += n;
         t = fk_registry_part2(&n); memcpy(buf + off, t, sizeof(fk_kernel) * n); off += n;

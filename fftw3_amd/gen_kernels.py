@@ -92,6 +92,41 @@ def mirrored_radices(L):
     return (best[1], L // points) if best else None
 
 
+def rr_forms(prec, L, rads, mode, io):
+    """(radices, threads per line) of the fused real-to-real kernels of a
+    length, the default first.  The mirrored form pays where a line's samples
+    are neighbours and the kind reads or writes them in quads or pairs
+    (REDFT10 / 01 / 11 rows, FP32 2048 x 32768 156 -> 111 us); elsewhere the
+    plain one has more threads per line or fewer stages.  us, 64 MiB arrays,
+    mirrored / plain:
+      columns of 3 * 2^k and 5 * 2^k points from 80 on: FP64 RODFT00 96 67 /
+      39, REDFT00 80 50 / 39, FP32 HC2R 320 46.7 / 38.9, 768 6 to 15% faster
+      plain; not powers of two (FP32 REDFT10 512 +14%, R2HC 4096 +11%);
+      REDFT11 columns: the same lengths below 2048, FP32 320 50.6 / 44.1 (from
+      2048 on plain is up to 20% slower, with two stages and a radix 16, 160
+      and 192 points, 3 to 10%), and FP64 512, 38.9 / 35.3;
+      rows of 3 * 2^k and 5 * 2^k points from 320 on and of 512: REDFT10 / 01
+      up to 50% faster mirrored (2048 samples FP32 32.3 / 37.6 through the
+      quads), the other kinds 5 to 30% faster plain (FP64 HC2R 320 36.0 /
+      31.4, FP32 REDFT00 6144 97 / 66): both forms, and the planner takes them
+      by kind;
+      c2r rows of 8192: plain 5% faster for every kind."""
+    mir, plain = mirrored_radices(L), (rads, None)
+    if not mir:
+        return [plain]
+    pow2 = L & (L - 1) == 0
+    if io == "DCT4":
+        if mode == "COL" and ((not pow2 and 80 <= L < 2048 and not (len(rads) == 2 and max(rads) == 16))
+                              or (prec == "double" and L == 512)):
+            return [plain]
+        return [mir]
+    if mode == "COL":
+        return [plain] if not pow2 and L >= 80 else [mir]
+    if io == "C2R" and L == 8192:
+        return [plain]
+    return [mir, plain] if (not pow2 and L >= 320) or L == 512 else [mir]
+
+
 def geometry(prec, L, rads, mode, io, tpl_div=1, nl_mul=1.0, tpl=None):
     """Default geometry: one butterfly of the largest radix per thread and
     stage (tpl = L / Rmax); tpl_div > 1 gives each thread tpl_div of them;
@@ -264,9 +299,10 @@ def catalog():
                         # (runtime rmode; kept out of the plain r2c / c2r
                         # code), row and column mappings: the column one
                         # serves r2r dims whose lines are strided
-                        rr, tr = mirrored_radices(L) or (rads, None)
-                        entries.append((prec, L, rr, "ROW", io + "_RR",
-                                        geometry(prec, L, rr, "ROW", io, tpl=tr)))
+                        for rr, tr in rr_forms(prec, L, rads, "ROW", io):
+                            entries.append((prec, L, rr, "ROW", io + "_RR",
+                                            geometry(prec, L, rr, "ROW", io, tpl=tr)))
+                        rr, tr = rr_forms(prec, L, rads, "COL", io)[0]
                         gc = geometry(prec, L, rr, "COL", io, tpl=tr)
                         # not for FP64 c2r at one line per workgroup
                         # (L = 5120, 6144, 8192): an execute through the
@@ -300,7 +336,7 @@ def catalog():
             if (fam or L <= 64) and L <= 8192:
                 # DCT-IV / DST-IV of 2L reals through the L-point DFT
                 for mode in ("ROW", "COL"):
-                    rr, tr = mirrored_radices(L) or (rads, None)
+                    rr, tr = rr_forms(prec, L, rads, mode, "DCT4")[0]
                     g = geometry(prec, L, rr, mode, "DCT4", tpl=tr)
                     if g:
                         entries.append((prec, L, rr, mode, "DCT4", g))

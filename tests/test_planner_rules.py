@@ -274,3 +274,40 @@ int main(void)
     return 0;
 }
 """)
+
+
+def test_rows_in_two_forms_are_taken_by_kind(tmp_path):
+    """Where the catalog has a real-to-real row kernel in two forms, the kinds
+    that read or write quads take the first (mirrored) by default, the others the
+    second; a stored choice is taken as it is."""
+    run(tmp_path, r"""
+int main(void)
+{
+    static const int r2c[] = {FK_RM_HC, FK_RM_DHT, FK_RM_E00, FK_RM_O00, FK_RM_DCT2, FK_RM_DST2};
+    static const int c2r[] = {FK_RM_HC2R, FK_RM_HC2R, FK_RM_HC2R, FK_RM_HC2R, FK_RM_DCT3, FK_RM_DST3};
+    int i, j, v, two = 0;
+    start();
+    for (i = 0; i < g_nreg; ++i) {
+        const fk_kernel *k = g_reg + i, *vs[16];
+        int n;
+        if (k->variant || k->mode != FK_ROW || (k->io != FK_IO_R2C_RR && k->io != FK_IO_C2R_RR)) continue;
+        n = find_variants(k->prec, k->L, k->mode, k->io, vs, 16);
+        CHECK(n <= 2, "L=%d: %d forms\n", k->L, n);
+        two += n == 2;
+        for (j = 0; j < 6; ++j)
+            for (v = -1; v < n; ++v) {
+                ctx c;
+                fk_plan *P = begin(&c, k->prec);
+                const int want = v >= 0 ? v : n == 2 && j < 4;
+                c.choice = v < 0 ? 0 : &v;
+                c.nchoice = v >= 0;
+                CHECK(pick_rr_row(&c, k->prec, k->L, k->io, (k->io == FK_IO_R2C_RR ? r2c : c2r)[j]) ==
+                          vs[want], "prec=%d L=%d io=%d kind %d choice %d\n", k->prec, k->L, k->io, j, v);
+                free(P);
+            }
+    }
+    CHECK(two > 0, "no kernel in two forms\n");
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
