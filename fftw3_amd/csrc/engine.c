@@ -403,6 +403,8 @@ typedef struct {
     int seen;                   /* most decisions taken so far (chunks replay them) */
     int r16;                    /* restrict to radix-16 passes (FK_MFMA) */
     int part;                   /* planning a part of a split line */
+    int lean;                   /* no scratch where one pass does (transposing_split) */
+    int trans;                  /* took a transposing_split */
     int bin, bout;              /* buffers of the r2c / c2r problem's arrays */
     int nalt[FK_MAX_DECIDE];    /* alternatives at each decision */
     int dkind[FK_MAX_DECIDE];
@@ -924,6 +926,43 @@ static int split_candidates(int prec, long long n, long long *out, int max)
 }
 
 /*
+ * Whether whole lines of n points, strided on one side and with a unit-stride
+ * batch on the other, run as two passes although the catalog has the length.
+ * Without a transposed-store kernel one pass scatters runs of its workgroup's
+ * lines; a split that ends in such a kernel reads and writes more but in long
+ * runs.  us, one pass / two:
+ *   strided stores, FP32 5 lines a workgroup and fewer (runs below 48 bytes),
+ *   FP64 3 and fewer: FP32 64 MiB 500 points 73 / 66, 864 97 / 57, 1728 148 /
+ *   59, FP64 864 71 / 58, 1728 79 / 61; with longer runs one pass is as fast
+ *   or faster (FP32 336 0.96 of the two, FP64 540 0.93);
+ *   strided loads, FP32 3 lines and fewer, FP64 one: FP32 700 105 / 72, 1728
+ *   116 / 84, FP64 1728 86 / 75; FP32 576, 4 lines, 72 / 73;
+ *   only from 64 MiB on, beyond which the caches no longer gather the runs, and
+ *   from 16 MiB with one line a workgroup in FP32 (16 MiB: FP32 1728 1.45 of
+ *   the two passes' time, 864 0.97, FP64 1728 0.74; 4 MiB and below: one pass
+ *   up to twice as fast).
+ */
+static int transposing_split(ctx *c, const fk_kernel *kr, long long n, long long is, long long os,
+                             int nb, const fk_dim *b)
+{
+    const int prec = c->P->prec;
+    const long long MB = 1LL << 20, bytes = n * batch_count(nb, b) * (long long)csz(prec);
+    long long n1[1];
+    int i, st = 0, ld = 0;
+    if (c->lean || c->part || is_factor(n)) return 0;
+    if (bytes < 64 * MB && !(prec == 1 && kr->nl == 1 && bytes >= 16 * MB)) return 0;
+    for (i = 0; i < nb; ++i) {
+        if (b[i].n < 2) continue;
+        if (llabs_(b[i].is) + llabs_(b[i].os) <= 4) return 0; /* the column mapping */
+        st |= llabs_(os) > 1 && llabs_(b[i].os) == 1;
+        ld |= llabs_(is) > 1 && llabs_(b[i].is) == 1;
+    }
+    if (!(st && kr->nl <= (prec ? 5 : 3)) && !(ld && kr->nl <= (prec ? 3 : 1))) return 0;
+    if (!smooth_plannable(prec, n, 0) || !split_candidates(prec, n, n1, 1)) return 0;
+    return find_kernel(prec, n / n1[0], FK_ROW, FK_IO_TOUT) != 0;
+}
+
+/*
  * Batched 1-D complex DFT of length n: element j of batch line h at
  * h-offset + j*is (input) / j*os (output).  Strides in complex elements.
  */
@@ -966,6 +1005,10 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
     kr = find_kernel(prec, n, FK_ROW, FK_IO_PLAIN);
     if (c->part && !is_factor(n)) kr = 0;
     if (c->r16 && n != 16 && n != 256 && n != 4096) kr = 0;
+    if (kr && transposing_split(c, kr, n, is, os, nb, b)) {
+        kr = 0;
+        c->trans = 1;
+    }
     if (kr) {
         /* candidate thread mappings, the heuristic's choice first:
            0 ROW, 1 ROW with transposed store, 2 COL */
@@ -2381,8 +2424,8 @@ static void mark_streams(fk_plan *P)
     }
 }
 
-static fk_plan *build_plan(const fk_problem *pb0, hipStream_t st, const int *choice, int nchoice,
-                           ctx *cout)
+static fk_plan *build_plan1(const fk_problem *pb0, hipStream_t st, const int *choice, int nchoice,
+                            ctx *cout, int lean, int *trans)
 {
     fk_problem pb = *pb0;
     fk_plan *P;
@@ -2416,6 +2459,7 @@ static fk_plan *build_plan(const fk_problem *pb0, hipStream_t st, const int *cho
     c.r16 = (pb.flags & FK_MFMA) && pb.prec == 1 && pb.kind == FK_C2C;
     c.bin = FK_BUF_IN;
     c.bout = FK_BUF_OUT;
+    c.lean = lean;
     P->split = pb.split;
     P->in2 = pb.in2;
     P->out2 = pb.out2;
@@ -2521,10 +2565,33 @@ done_ok:
     if (cout) *cout = c;
     ok = 1;
 fail:
+    *trans = c.trans;
     if (!ok) {
         fk_plan_destroy(P);
         return 0;
     }
+    return P;
+}
+
+static size_t scratch_total(const fk_plan *p)
+{
+    size_t n = 0;
+    int i;
+    for (i = 0; i < FK_MAX_SCRATCH; ++i) n += (p->scratch_bytes[i] + 255) & ~(size_t)255;
+    return n;
+}
+
+/* A transposing_split takes scratch for speed alone: where the device has no
+   room for it the plan is the one-pass one, and where the allocation-free
+   execute has none, that execute runs the one-pass one (P->lean). */
+static fk_plan *build_plan(const fk_problem *pb, hipStream_t st, const int *choice, int nchoice,
+                           ctx *cout)
+{
+    int trans = 0, t;
+    fk_plan *P = build_plan1(pb, st, choice, nchoice, cout, 0, &trans);
+    if (!P && trans) return build_plan1(pb, st, 0, 0, cout, 1, &t);
+    if (P && trans && scratch_total(P) > FK_STATIC_SCRATCH_BYTES)
+        P->lean = build_plan1(pb, st, 0, 0, 0, 1, &t);
     return P;
 }
 
@@ -2799,6 +2866,7 @@ void fk_plan_destroy(fk_plan *p)
 {
     int i;
     if (!p) return;
+    fk_plan_destroy(p->lean);
     for (i = 0; i < FK_MAX_SCRATCH; ++i) fk_free(p->scratch[i]);
     free(p->pass);
     free(p);
@@ -2906,7 +2974,11 @@ int fk_execute_noalloc(fk_plan *p, void *in, void *out)
                 p->align_need, p->align_in, p->align_out);
         return (int)hipErrorInvalidValue;
     }
-    for (i = 0; i < FK_MAX_SCRATCH; ++i) off += (p->scratch_bytes[i] + 255) & ~(size_t)255;
+    off = scratch_total(p);
+    if (off > FK_STATIC_SCRATCH_BYTES && p->lean) {
+        p->lean->stream = p->stream;
+        return fk_execute_noalloc(p->lean, in, out);
+    }
     if (off > FK_STATIC_SCRATCH_BYTES) {
         set_err("execute_noalloc: plan needs %zu bytes of scratch, the static scratch holds %zu",
                 off, (size_t)FK_STATIC_SCRATCH_BYTES);

@@ -88,6 +88,9 @@ typedef struct fk_plan {
     int r2r[FK_MAXRANK];        /* FK_R2R: kind of each dim */
     int npass, cpass;
     int nseq;                   /* logical passes */
+    struct fk_plan *lean;       /* the same transform without scratch, for
+                                   fk_execute_noalloc when this plan's scratch
+                                   does not fit (NULL: none) */
     fk_pass *pass;
     int nscratch;
     size_t scratch_bytes[FK_MAX_SCRATCH];

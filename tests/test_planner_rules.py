@@ -311,3 +311,48 @@ int main(void)
     return 0;
 }
 """)
+
+
+def test_transposing_lines_without_a_transposed_store(tmp_path):
+    """Whole lines strided on one side only: two passes where the length has no
+    transposed-store kernel, its split ends in one, the lines of a workgroup make
+    short runs and the array is large; one pass in the other cases, for rows,
+    columns and small batches, and always when scratch is to be avoided."""
+    run(tmp_path, r"""
+int main(void)
+{
+    int prec, L, w, taken = 0;
+    start();
+    for (prec = 0; prec < 2; ++prec)
+        for (L = 2; L <= 2048; ++L) {
+            const fk_kernel *k = find_kernel(prec, L, FK_ROW, FK_IO_PLAIN);
+            long long mb, n1[1];
+            int tout = 0;
+            if (!k) continue;
+            if (!is_factor(L) && split_candidates(prec, L, n1, 1))
+                tout = find_kernel(prec, L / n1[0], FK_ROW, FK_IO_TOUT) != 0;
+            for (mb = 1; mb <= 256; mb *= 2)
+                for (w = 0; w < 5; ++w) { /* store, load, rows, columns, store without scratch */
+                    const long long H = (mb << 20) / (L * (prec ? 8 : 16)) + 1;
+                    const fk_dim b = {H, w == 1 || w == 3 ? 1 : L, w == 1 || w == 2 ? L : 1};
+                    const int few = w == 1 ? (prec ? 3 : 1) : (prec ? 5 : 3);
+                    const int want = tout && w != 2 && w != 3 && w != 4 && k->nl <= few &&
+                                     (mb >= 64 || (prec && k->nl == 1 && mb >= 16));
+                    ctx c;
+                    fk_plan *P = begin(&c, prec);
+                    c.lean = w == 4;
+                    CHECK(transposing_split(&c, k, L, w == 1 || w == 3 ? H : 1,
+                                            w == 1 || w == 2 ? 1 : H, 1, &b) == want,
+                          "prec=%d L=%d nl=%d form %d %lld MiB\n", prec, L, k->nl, w, mb);
+                    taken += want;
+                    c.lean = 0;
+                    c.part = 1;
+                    CHECK(!transposing_split(&c, k, L, 1, H, 1, &b), "part of a split\n");
+                    free(P);
+                }
+        }
+    CHECK(taken > 100, "only %d\n", taken);
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
