@@ -323,31 +323,14 @@ static const fk_kernel *find_kernel(int prec, long long L, int mode, int io)
     return 0;
 }
 
-/* Lengths a longer line is split into: up to 64, powers of two times 1, 3 or 5,
-   powers of 3, 5 and 7, and four round ones.  The catalog's other lengths serve
-   whole lines only: without transposed-store kernels they end a split with
-   scattered stores, or (as split_candidates scores that) make it one pass
-   longer (us: FP32 444528 x 29 167 -> 283, FP64 real 7350 x 179 there and back
-   56 -> 60). */
-static int is_factor(long long n)
+/* whether longer lines may be split into n (gen_kernels.py, size_list) */
+static int is_factor(int prec, long long n)
 {
-    long long m = n;
-    int i;
-    if (n <= 64 || n == 100 || n == 1000 || n == 1001 || n == 10000) return 1;
-    while (m % 2 == 0) m /= 2;
-    if (m == 1 || m == 3 || m == 5) return 1;
-    for (i = 3; i <= 7; i += 2) {
-        for (m = n; m % i == 0; m /= i)
-            ;
-        if (m == 1) return 1;
-    }
-    return 0;
+    const fk_kernel *k = find_kernel(prec, n, FK_ROW, FK_IO_PLAIN);
+    return k && k->factor;
 }
 
-static int has_single(int prec, long long n)
-{
-    return is_factor(n) && find_kernel(prec, n, FK_ROW, FK_IO_PLAIN) != 0;
-}
+static int has_single(int prec, long long n) { return is_factor(prec, n); }
 
 /* the catalog variant of (prec, L, mode, io) whose stages are all radix 16
    (the matrix-core substitution needs them), or NULL */
@@ -377,7 +360,7 @@ static int smooth_plannable(int prec, long long n, int depth)
     if (n == 1 || has_single(prec, n)) return 1;
     if (depth >= 3) return 0;
     for (n1 = 2; n1 <= 16384 && n1 < n; ++n1) {
-        if (n % n1 || !is_factor(n1)) continue;
+        if (n % n1 || !is_factor(prec, n1)) continue;
         if (!find_kernel(prec, n1, FK_COL, FK_IO_PLAIN)) continue;
         if (smooth_plannable(prec, n / n1, depth + 1)) return 1;
     }
@@ -892,7 +875,7 @@ static int split_candidates(int prec, long long n, long long *out, int max)
         long long n2;
         double score;
         const fk_kernel *kc, *kt;
-        if (n % n1 || !is_factor(n1)) continue;
+        if (n % n1 || !is_factor(prec, n1)) continue;
         n2 = n / n1;
         kc = find_kernel(prec, n1, FK_COL, FK_IO_PLAIN);
         if (!kc) continue;
@@ -949,7 +932,7 @@ static int transposing_split(ctx *c, const fk_kernel *kr, long long n, long long
     const long long MB = 1LL << 20, bytes = n * batch_count(nb, b) * (long long)csz(prec);
     long long n1[1];
     int i, st = 0, ld = 0;
-    if (c->lean || c->part || is_factor(n)) return 0;
+    if (c->lean || c->part || kr->factor) return 0;
     if (bytes < 64 * MB && !(prec == 1 && kr->nl == 1 && bytes >= 16 * MB)) return 0;
     for (i = 0; i < nb; ++i) {
         if (b[i].n < 2) continue;
@@ -1003,7 +986,7 @@ static int plan_c2c_1d(ctx *c, long long n, long long is, long long os, int nb_,
         return 0;
     }
     kr = find_kernel(prec, n, FK_ROW, FK_IO_PLAIN);
-    if (c->part && !is_factor(n)) kr = 0;
+    if (kr && c->part && !kr->factor) kr = 0;
     if (c->r16 && n != 16 && n != 256 && n != 4096) kr = 0;
     if (kr && transposing_split(c, kr, n, is, os, nb, b)) {
         kr = 0;

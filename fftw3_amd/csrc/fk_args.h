@@ -116,6 +116,7 @@ typedef struct {
     int variant;       /* 0 = default geometry; >0 autotuner alternatives */
     int loop;          /* 1: each workgroup runs several tiles (grid sized to
                           the workgroups the device holds at once) */
+    int factor;        /* 1: longer lines may be split into this length */
 } fk_kernel;
 
 /* elementwise passes around the Stockham kernels (multi-pass paths) */

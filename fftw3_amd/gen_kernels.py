@@ -180,7 +180,11 @@ def smooth(n, primes):
     return n == 1
 
 
-def size_list(prec):
+def factor_list(prec):
+    """Lengths a longer line is split into, and whole lines of their own: small
+    ones, the families with transposed-store kernels (2^k times 1, 3 or 5),
+    powers of 3, 5 and 7, and a few that make lines of 1000, 1001, 2187, 10^k
+    and their products two passes."""
     lmax = 8192 if prec == "double" else 16384
     s = set()
     for n in range(2, 65):
@@ -197,19 +201,31 @@ def size_list(prec):
         while p <= lmax:
             s.add(p)
             p *= base
-    s.update([100, 1000, 1001, 2187, 81, 729])
-    # products of 2, 3, 5 and 7: all up to 512, those with a factor 4 or 10 up
-    # to 1024, with 16 or 40 up to 2048 (each kernel costs build time, and the
-    # rounder lengths are the ones in use).  As two passes such a line is read
-    # and written twice: us, 64 MiB arrays, FP32 240 x 34952 69.1 -> 31.4,
-    # 1080 x 7767 61.0 -> 33.9, columns 270 143 -> 31; r2c there and back 240
-    # 101 -> 39
+    s.update([100, 1000, 1001])
+    if lmax >= 10000:
+        s.add(10000)
+    return s
+
+
+def size_list(prec):
+    s = factor_list(prec)
+    # whole lines only: products of 2, 3, 5 and 7, all up to 512, those with a
+    # factor 4 or 10 up to 1024, with 16 or 40 up to 2048.  As two passes such a
+    # line is read and written twice: us, 64 MiB arrays, FP32 240 x 34952 69.1
+    # -> 31.4, 1080 x 7767 61.0 -> 33.9, columns 270 143 -> 31; r2c there and
+    # back 240 101 -> 39.  The ranges are bounded by build time alone (about 1.5
+    # s of compile time a kernel, 6 to 12 kernels a length): 8 lengths up to
+    # 1024 and 26 up to 2048 are left to two passes, 1260, 1500 and 1764 among
+    # them.
+    # Not factors of longer lines (fk_kernel.factor): they have no
+    # transposed-store kernels, so a split that ends in one scatters, and one
+    # that begins with one leaves a rest that takes a pass more (us, with them
+    # as factors / without: FP32 444528 x 29 283 / 167, FP64 real 7350 x 179
+    # there and back 60 / 56).
     s.update(n for n in range(65, 2049) if smooth(n, (2, 3, 5, 7)) and
              (n <= 512 or n % 16 == 0 or n % 40 == 0 or
               n <= 1024 and (n % 4 == 0 or n % 10 == 0)))
-    if lmax >= 10000:
-        s.add(10000)
-    return sorted(x for x in s if x <= lmax)
+    return sorted(s)
 
 
 def variants(prec, L, rads, mode, io, g0):
@@ -513,6 +529,7 @@ def main():
     for i, e in enumerate(sorted(entries, key=lambda e: -e[1])):
         parts[i % nparts].append(e)
     written = set()
+    factors = {prec: factor_list(prec) for prec in PREC}
     for p, es in enumerate(parts):
         lines = ['// generated by fftw3_amd/gen_kernels.py -- do not edit',
                  '#include "../fk_stockham.h"', '',
@@ -522,24 +539,27 @@ def main():
             prec, L, rads, mode, io, g, var = e
             targs, rl = cxx_entry(e[:6])
             radarr = ",".join(map(str, rads))
+            fac = int(L in factors[prec])
             if g.get("xs"):
                 xargs = "%s,%d,FK_%s,%d,%s,%d" % (prec, g["nl"], mode, g["pad"], rl, g["tpl"])
                 lines.append(
                     '        {%d, %d, %d, {%s}, %d, %d, FK_%s, FK_IO_%s, fk::stockham_xs_lds<%s>(), '
-                    '%s::twsize(), (const void *)&fk::stockham_xs<%s>, %d},'
-                    % (PREC[prec], L, len(rads), radarr, g["tpl"], g["nl"], mode, io, xargs, rl, xargs, var))
+                    '%s::twsize(), (const void *)&fk::stockham_xs<%s>, %d, 0, %d},'
+                    % (PREC[prec], L, len(rads), radarr, g["tpl"], g["nl"], mode, io, xargs, rl, xargs, var,
+                       fac))
                 continue
             if g.get("pipe"):
                 pargs = "%s,%d,%d,%s,%d" % (prec, g["nl"], g["pad"], rl, g["tpl"])
                 lines.append(
                     '        {%d, %d, %d, {%s}, %d, %d, FK_%s, FK_IO_%s, fk::stockham_lds<%s>(), '
-                    '%s::twsize(), (const void *)&fk::stockham_pipe<%s>, %d, 1},'
-                    % (PREC[prec], L, len(rads), radarr, g["tpl"], g["nl"], mode, io, targs, rl, pargs, var))
+                    '%s::twsize(), (const void *)&fk::stockham_pipe<%s>, %d, 1, %d},'
+                    % (PREC[prec], L, len(rads), radarr, g["tpl"], g["nl"], mode, io, targs, rl, pargs, var,
+                       fac))
                 continue
             lines.append(
                 '        {%d, %d, %d, {%s}, %d, %d, FK_%s, FK_IO_%s, fk::stockham_lds<%s>(), '
-                '%s::twsize(), (const void *)&fk::stockham<%s>, %d},'
-                % (PREC[prec], L, len(rads), radarr, g["tpl"], g["nl"], mode, io, targs, rl, targs, var))
+                '%s::twsize(), (const void *)&fk::stockham<%s>, %d, 0, %d},'
+                % (PREC[prec], L, len(rads), radarr, g["tpl"], g["nl"], mode, io, targs, rl, targs, var, fac))
         lines += ['    };', '    *n = (int)(sizeof(tab) / sizeof(tab[0]));', '    return tab;', '}', '']
         path = os.path.join(OUT, "fk_inst_%d.hip" % p)
         written.add(path)

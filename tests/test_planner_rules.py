@@ -329,7 +329,7 @@ int main(void)
             long long mb, n1[1];
             int tout = 0;
             if (!k) continue;
-            if (!is_factor(L) && split_candidates(prec, L, n1, 1))
+            if (!is_factor(prec, L) && split_candidates(prec, L, n1, 1))
                 tout = find_kernel(prec, L / n1[0], FK_ROW, FK_IO_TOUT) != 0;
             for (mb = 1; mb <= 256; mb *= 2)
                 for (w = 0; w < 5; ++w) { /* store, load, rows, columns, store without scratch */
@@ -352,6 +352,43 @@ int main(void)
                 }
         }
     CHECK(taken > 100, "only %d\n", taken);
+    printf("%lld %lld\n", bad, seen);
+    return 0;
+}
+""")
+
+
+def test_splits_use_the_lengths_kept_for_them(tmp_path):
+    """Every kernel of a length carries the same factor flag, the flagged lengths
+    are gen_kernels.factor_list, and the first length of every split candidate
+    (up to four per line) is flagged while its rest can be planned from flagged
+    lengths."""
+    import sys
+    sys.path.insert(0, PKG)
+    import gen_kernels as g
+    lists = "".join("static const int fac_%d[] = {%s, 0};\n" %
+                    (i, ",".join(map(str, sorted(g.factor_list(p) & set(g.size_list(p))))))
+                    for i, p in ((0, "double"), (1, "float")))
+    run(tmp_path, lists + r"""
+int main(void)
+{
+    int prec, i, j, n;
+    start();
+    for (i = 0; i < g_nreg; ++i) {
+        const int *f = g_reg[i].prec ? fac_1 : fac_0;
+        int in = 0;
+        for (j = 0; f[j]; ++j) in |= f[j] == g_reg[i].L;
+        CHECK(in == g_reg[i].factor, "L=%d prec=%d: flag %d\n", g_reg[i].L, g_reg[i].prec, g_reg[i].factor);
+    }
+    for (prec = 0; prec < 2; ++prec)
+        for (n = 2; n < 30000; ++n) {
+            long long c[4];
+            int nc = smooth_plannable(prec, n, 0) ? split_candidates(prec, n, c, 4) : 0;
+            for (j = 0; j < nc; ++j) {
+                const fk_kernel *k = find_kernel(prec, c[j], FK_COL, FK_IO_PLAIN);
+                CHECK(k && k->factor && smooth_plannable(prec, n / c[j], 1), "n=%d: %lld\n", n, c[j]);
+            }
+        }
     printf("%lld %lld\n", bad, seen);
     return 0;
 }
