@@ -101,6 +101,52 @@ static inline void fk_magic(unsigned long long d, unsigned *m, unsigned *s)
     *s = k;
 }
 
+/* The index arithmetic of the kernels, in host code too (the tests run it on
+   the CPU). */
+#ifdef __HIPCC__
+#define FK_BOTH static __host__ __device__ __forceinline__
+#else
+#define FK_BOTH static inline
+#endif
+
+/* q / d through fk_magic's multiplier and shift, q < 2^31 */
+FK_BOTH unsigned fk_div_small(unsigned q, unsigned m, unsigned s)
+{
+    return (unsigned)(((unsigned long long)(2 * q) * m) >> 32) >> s;
+}
+
+/* q / d for 0 <= q < 2^53, d > 0, through FP64: q is exact there and the
+   quotient off by at most one (a 64-bit integer division would be several
+   hundred instructions in every kernel, for the few passes that need it) */
+FK_BOTH long long fk_div_large(long long q, long long d)
+{
+    const long long t = (long long)((double)q / (double)d), r = q - t * d;
+    return r < 0 ? t - 1 : r >= d ? t + 1 : t;
+}
+
+/* batch indices of line q of a pass (0 <= q < nlines) */
+typedef struct {
+    long long i0, i1, i2;
+} fk_line;
+FK_BOTH fk_line fk_line_ix(const fk_args *a, long long q)
+{
+    fk_line r;
+    if (a->qm[0]) {
+        const unsigned u = (unsigned)q;
+        const unsigned q1 = fk_div_small(u, a->qm[0], a->qs[0]);
+        const unsigned q2 = fk_div_small(q1, a->qm[1], a->qs[1]);
+        r.i0 = u - q1 * (unsigned)a->nb[0];
+        r.i1 = q1 - q2 * (unsigned)a->nb[1];
+        r.i2 = q2;
+    } else {
+        const long long q1 = fk_div_large(q, a->nb[0]);
+        r.i0 = q - q1 * a->nb[0];
+        r.i2 = fk_div_large(q1, a->nb[1]);
+        r.i1 = q1 - r.i2 * a->nb[1];
+    }
+    return r;
+}
+
 typedef struct {
     int prec;          /* 0 = double, 1 = float */
     int L;             /* FFT length computed by the kernel */

@@ -331,15 +331,6 @@ __device__ __forceinline__ void cexp_fp64(long long m, long long n, double &c,
     s = -sn;
 }
 
-/* q / d for 0 <= q < 2^53, d > 0, through FP64: q is exact there and the
-   quotient off by at most one (a 64-bit integer division would be several
-   hundred instructions in every kernel, for the few passes that need it) */
-__device__ __forceinline__ long long div_large(long long q, long long d)
-{
-    const long long t = (long long)((double)q / (double)d), r = q - t * d;
-    return r < 0 ? t - 1 : r >= d ? t + 1 : t;
-}
-
 /* W_N^e in FP64 from the two-level table (see tw2) */
 __device__ __forceinline__ cx<double> tw2d(const fk_args &a, long long e);
 
@@ -357,39 +348,20 @@ __device__ __forceinline__ cx<double> tw2d(const fk_args &a, long long e)
        of line i0 < n2, n1 n2 = N), and n1*p of the cross-row kernels. */
     const long long b = a.tb;
     if (a.qm[2]) {                             /* N < 2^31: 32-bit split */
-        const unsigned ue = (unsigned)e, q = __umulhi(2 * ue, a.qm[2]) >> a.qs[2];
+        const unsigned ue = (unsigned)e, q = fk_div_small(ue, a.qm[2], a.qs[2]);
         const unsigned l = ue - q * (unsigned)b;
         const double2 lo = reinterpret_cast<const double2 *>(a.tlo)[l];
         const double2 hi = reinterpret_cast<const double2 *>(a.thi)[q];
         return mk(lo.x * hi.x - lo.y * hi.y, lo.x * hi.y + lo.y * hi.x);
     }
-    const long long ih = div_large(e, b), il = e - ih * b;
+    const long long ih = fk_div_large(e, b), il = e - ih * b;
     const double *lo = a.tlo + 2 * il, *hi = a.thi + 2 * ih;
     return mk(lo[0] * hi[0] - lo[1] * hi[1], lo[0] * hi[1] + lo[1] * hi[0]);
 }
 
 /* batch indices of line q of a pass (0 <= q < nlines) */
-struct LineIx {
-    long long i0, i1, i2;
-};
-__device__ __forceinline__ LineIx line_ix(const fk_args &a, long long q)
-{
-    LineIx r;
-    if (a.qm[0]) {
-        const unsigned u = (unsigned)q;
-        const unsigned q1 = __umulhi(2 * u, a.qm[0]) >> a.qs[0];
-        const unsigned q2 = __umulhi(2 * q1, a.qm[1]) >> a.qs[1];
-        r.i0 = u - q1 * (unsigned)a.nb[0];
-        r.i1 = q1 - q2 * (unsigned)a.nb[1];
-        r.i2 = q2;
-    } else {
-        const long long q1 = div_large(q, a.nb[0]);
-        r.i0 = q - q1 * a.nb[0];
-        r.i2 = div_large(q1, a.nb[1]);
-        r.i1 = q1 - r.i2 * a.nb[1];
-    }
-    return r;
-}
+typedef fk_line LineIx;
+__device__ __forceinline__ LineIx line_ix(const fk_args &a, long long q) { return fk_line_ix(&a, q); }
 
 /* input and output offset of a line, in elements of its array */
 __device__ __forceinline__ void line_off(const fk_args &a, const LineIx &x, long long &bin,
