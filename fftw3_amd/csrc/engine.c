@@ -211,8 +211,8 @@ static long long isqrt_ceil(long long n)
 /* FP64 two-level table of W_N^e: lo (b entries) then hi (N/b+1 entries) */
 static const double *tw2_table(long long N, long long *b_out, hipStream_t st)
 {
-    /* split b ~ sqrt(N), a power of two when N is one (the kernels then
-       index the two levels by mask and shift) */
+    /* split b ~ sqrt(N), a power of two when N is one (both levels are then
+       about the same size; the kernels split an exponent by fk_args.qm[2]) */
     long long b = isqrt_ceil(N);
     if ((N & (N - 1)) == 0) {
         b = 1;

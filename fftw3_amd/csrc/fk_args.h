@@ -104,7 +104,7 @@ static inline void fk_magic(unsigned long long d, unsigned *m, unsigned *s)
 /* The index arithmetic of the kernels, in host code too (the tests run it on
    the CPU). */
 #ifdef __HIPCC__
-#define FK_BOTH static __host__ __device__ __forceinline__
+#define FK_BOTH static __host__ __device__ inline __attribute__((always_inline))
 #else
 #define FK_BOTH static inline
 #endif
