@@ -390,7 +390,10 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
     const unsigned fl = a.flags;
     const bool swi = fl & FK_SWAP_IN, swo = fl & FK_SWAP_OUT;
     const bool nti = fl & FK_NT_IN, nto = fl & FK_NT_OUT;
-    constexpr bool NTP = sizeof(R) == 8 && MODE == FK_ROW && IO == FK_IO_PLAIN;
+    /* kernels that the non-temporal flags can reach (whole_sectors in engine.c) */
+    constexpr int NB_0 = L / RL::r[0], NB_N = L / RL::r[RL::n - 1];
+    constexpr bool NTP = sizeof(R) == 8 && MODE == FK_ROW && IO == FK_IO_PLAIN && TPL % 4 == 0 &&
+                         NB_0 % 4 == 0 && NB_N % 4 == 0;
     auto lds_at = [&](auto j) -> cx<R> & {
         if constexpr (NT == NR) return lds[G::idx(lt, j)];
         else return real ? lds[G::idx(lt, j)] : trash[tid & 63];
