@@ -639,20 +639,22 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
             });
         }
         /* cross-row form: twiddles of the first column stage, W_n0^(n1*p) (n1 =
-           the tile's line-group index, uniform over the workgroup), looked up
-           before the stages, whose loads hide the lookups: after them 1024 x
-           1024 r2c x 64 FP32 took 231 us instead of 208, x 32 FP64 199 instead
-           of 190 (at 2048 x 2048 219 / 216) */
+           the tile's line-group index, uniform over the workgroup).  Below 1024
+           points they are looked up before the stages, whose loads hide the
+           lookups (r2c of 1024 x 1024 x 64 FP32 231 us after them, 208 before,
+           x 32 FP64 199 / 190); at 1024, where they cost 12 registers, after
+           (2048 x 2048 x 64 FP32 890.6, before 892.8) */
         long long tin = 0, tout = 0;
         cx<R> wp[XR ? NL : 1];
-        if constexpr (XR) {
+        auto column_tw = [&]() {
             const LineIx tx = line_ix(a, tile * NL);
             line_off(a, tx, tin, tout);
             sfor<0, NL>([&](auto pc) {
                 constexpr int pp = decltype(pc)::value;
                 wp[pp] = pp == 0 ? mk((R)1, (R)0) : tw2<R>(a, tx.i1 * pp);
             });
-        }
+        };
+        if constexpr (XR && L < 1024) column_tw();
         run_stages<R, RL, 0, L, TPL, false, true, SY>(u, tw, lds_at, gld, lst);
         /* bins k = u + i*TPL <= L/2 and L-k of the line: f(i, k, X[k], X[L-k]) */
         auto bins = [&](auto &&f) {
@@ -698,6 +700,7 @@ __device__ __forceinline__ void stockham_body(const fk_args &a, long long tile,
                 }
             });
         } else {
+            if constexpr (L >= 1024) column_tw();
             /* the bins stay in registers until every bin of the line has
                been formed, then replace Z in the line's LDS row */
             cx<R> xs[2 * NK2];
