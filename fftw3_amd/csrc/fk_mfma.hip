@@ -72,7 +72,7 @@ __device__ __forceinline__ void split(float x, _Float16 &hi, _Float16 &lo)
  * LDS: a coalesced load of the whole tile (threads along the line for unit
  * element stride, across lines otherwise), S radix-16 stages on the matrix
  * cores with the tile in LDS, and a coalesced store of the tile with the
- * output post-op (four-step twiddle, scale, backward swap).  Each wave runs
+ * output post-op (four-step twiddle, backward swap).  Each wave runs
  * groups of 32 butterflies (one MFMA column each) of the tile's
  * NL * L/16 butterflies per stage.
  */
