@@ -913,34 +913,42 @@ static int split_candidates(int prec, long long n, long long *out, int max)
  * batch on the other, run as two passes although the catalog has the length.
  * Without a transposed-store kernel one pass scatters runs of its workgroup's
  * lines; a split that ends in such a kernel reads and writes more but in long
- * runs.  us, one pass / two:
- *   strided stores, FP32 5 lines a workgroup and fewer (runs below 48 bytes),
- *   FP64 3 and fewer: FP32 64 MiB 500 points 73 / 66, 864 97 / 57, 1728 148 /
- *   59, FP64 864 71 / 58, 1728 79 / 61; with longer runs one pass is as fast
- *   or faster (FP32 336 0.96 of the two, FP64 540 0.93);
- *   strided loads, FP32 3 lines and fewer, FP64 one: FP32 700 105 / 72, 1728
- *   116 / 84, FP64 1728 86 / 75; FP32 576, 4 lines, 72 / 73;
- *   only from 64 MiB on, beyond which the caches no longer gather the runs, and
- *   from 16 MiB with one line a workgroup in FP32 (16 MiB: FP32 1728 1.45 of
- *   the two passes' time, 864 0.97, FP64 1728 0.74; 4 MiB and below: one pass
- *   up to twice as fast).
+ * runs.  From which size (MiB) the two passes pay, by the lines a workgroup has
+ * (the runs' length); 0: never.  One pass as a part of the two passes' time, 400
+ * to 2016 points:
+ *   strided stores, FP32: 1 line 4 MiB 0.97-1.09, 8 MiB 1.12-1.35, 64 MiB 2.3;
+ *   2 lines 8 MiB 0.89-1.07, 12 MiB 0.97-1.15, 64 MiB 1.6-1.8; 3 lines 16 MiB
+ *   0.95-1.23, 24 MiB 1.35-1.64; 4 lines 16 MiB 0.73-0.92, 24 MiB 1.18-1.42; 5
+ *   lines 24 MiB 0.96-1.07, 32 MiB 0.97-1.12, 64 MiB 1.12-1.23; 6 and more, to
+ *   128 MiB, 0.57-1.05;
+ *   strided stores, FP64: 1 line 16 MiB 0.74-0.85, 24 MiB 1.01-1.22, 64 MiB 1.3;
+ *   2 and 3 lines 24 MiB 0.82-1.12, 32 MiB 0.79-1.38 (mean 1.08); 4 and 5 lines
+ *   64 MiB 0.87-1.08, 128 MiB 0.94-1.18 (1.07); 7 lines 128 MiB 0.89;
+ *   strided loads, FP32, 1 to 3 lines: 4 MiB 0.70-1.07, 8 MiB 0.97-1.27, 64 MiB
+ *   1.19-1.86; 4 lines 8 to 128 MiB 0.83-1.11 (0.97);
+ *   strided loads, FP64, 1 line: 4 MiB 0.74-0.98, 8 MiB 1.02-1.26, 64 MiB 1.16-
+ *   1.30; 2 lines 0.74-1.27 (0.96).
+ * Below those sizes the caches gather the runs.
  */
 static int transposing_split(ctx *c, const fk_kernel *kr, long long n, long long is, long long os,
                              int nb, const fk_dim *b)
 {
+    static const short from_st[2][6] = {{0, 20, 28, 28, 96, 96}, {0, 6, 10, 20, 20, 28}};
+    static const short from_ld[2][6] = {{0, 6, 0, 0, 0, 0}, {0, 6, 6, 6, 0, 0}};
     const int prec = c->P->prec;
-    const long long MB = 1LL << 20, bytes = n * batch_count(nb, b) * (long long)csz(prec);
+    const long long mb = n * batch_count(nb, b) * (long long)csz(prec) >> 20;
     long long n1[1];
     int i, st = 0, ld = 0;
-    if (c->lean || c->part || kr->factor) return 0;
-    if (bytes < 64 * MB && !(prec == 1 && kr->nl == 1 && bytes >= 16 * MB)) return 0;
+    if (c->lean || c->part || kr->factor || kr->nl > 5) return 0;
     for (i = 0; i < nb; ++i) {
         if (b[i].n < 2) continue;
         if (llabs_(b[i].is) + llabs_(b[i].os) <= 4) return 0; /* the column mapping */
         st |= llabs_(os) > 1 && llabs_(b[i].os) == 1;
         ld |= llabs_(is) > 1 && llabs_(b[i].is) == 1;
     }
-    if (!(st && kr->nl <= (prec ? 5 : 3)) && !(ld && kr->nl <= (prec ? 3 : 1))) return 0;
+    st = st ? from_st[prec][kr->nl] : 0;
+    ld = ld ? from_ld[prec][kr->nl] : 0;
+    if (!(st && mb >= st) && !(ld && mb >= ld)) return 0;
     if (!smooth_plannable(prec, n, 0) || !split_candidates(prec, n, n1, 1)) return 0;
     return find_kernel(prec, n / n1[0], FK_ROW, FK_IO_TOUT) != 0;
 }

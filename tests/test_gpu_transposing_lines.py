@@ -14,18 +14,21 @@ from gpu_util import TOL, cdt, inputs_c
 pytestmark = pytest.mark.gpu
 
 
-# (prec, n, MiB, passes): 900 FP32 has 2 lines a workgroup, 1728 one (FP64 1), 225 no
-# split that ends in a transposed store
-@pytest.mark.parametrize("prec,n,mib,passes", [
-    ("float", 900, 8, 1), ("float", 900, 66, 2), ("float", 1728, 17, 2), ("float", 225, 66, 1),
-    ("double", 1728, 17, 1), ("double", 1728, 66, 2), ("float", 1008, 130, 2)])
+# (prec, n, MiB, passes with strided stores, with strided loads): lines a workgroup
+# FP32 900 two, 1728 one, 648 three, 1008 four, 784 five; FP64 1728 one, 648 three;
+# 225 has no split that ends in a transposed store
+@pytest.mark.parametrize("prec,n,mib,st,ld", [
+    ("float", 900, 4, 1, 1), ("float", 900, 8, 1, 2), ("float", 900, 66, 2, 2),
+    ("float", 1728, 4, 1, 1), ("float", 1728, 17, 2, 2), ("float", 648, 16, 1, 2),
+    ("float", 648, 24, 2, 2), ("float", 784, 32, 2, 1), ("float", 225, 66, 1, 1),
+    ("float", 1008, 130, 2, 1), ("double", 1728, 4, 1, 1), ("double", 1728, 16, 1, 2),
+    ("double", 1728, 66, 2, 2), ("double", 648, 32, 2, 1)])
 @pytest.mark.parametrize("side", ["store", "load"])
 @pytest.mark.parametrize("sign", [-1, 1])
-def test_transposing(eng, prec, n, mib, passes, side, sign):
+def test_transposing(eng, prec, n, mib, st, ld, side, sign):
     size = np.dtype(cdt(prec)).itemsize
-    h = (mib << 20) // (n * size) + 1
-    if side == "load" and n == 1008:
-        passes = 1    # 4 lines a workgroup
+    h = (mib << 20) // (n * size)
+    passes = st if side == "store" else ld
     x = inputs_c(n * h, n, prec)
     a = fa.DeviceBuffer.from_array(x)
     b = fa.DeviceBuffer(x.nbytes)

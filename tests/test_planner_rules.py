@@ -316,8 +316,9 @@ int main(void)
 def test_transposing_lines_without_a_transposed_store(tmp_path):
     """Whole lines strided on one side only: two passes where the length has no
     transposed-store kernel, its split ends in one, the lines of a workgroup make
-    short runs and the array is large; one pass in the other cases, for rows,
-    columns and small batches, and always when scratch is to be avoided."""
+    short runs and the array is large, the larger the longer the runs are; one pass
+    in the other cases, for rows, columns and small batches, and always when scratch
+    is to be avoided.  Sizes just below a power of two count as that size."""
     run(tmp_path, r"""
 int main(void)
 {
@@ -331,13 +332,19 @@ int main(void)
             if (!k) continue;
             if (!is_factor(prec, L) && split_candidates(prec, L, n1, 1))
                 tout = find_kernel(prec, L / n1[0], FK_ROW, FK_IO_TOUT) != 0;
-            for (mb = 1; mb <= 256; mb *= 2)
+            for (mb = 1; mb <= 256; mb += mb < 32 ? 1 : 16)
                 for (w = 0; w < 5; ++w) { /* store, load, rows, columns, store without scratch */
-                    const long long H = (mb << 20) / (L * (prec ? 8 : 16)) + 1;
+                    const long long H = (mb << 20) / (L * (prec ? 8 : 16)); /* just below */
                     const fk_dim b = {H, w == 1 || w == 3 ? 1 : L, w == 1 || w == 2 ? L : 1};
-                    const int few = w == 1 ? (prec ? 3 : 1) : (prec ? 5 : 3);
-                    const int want = tout && w != 2 && w != 3 && w != 4 && k->nl <= few &&
-                                     (mb >= 64 || (prec && k->nl == 1 && mb >= 16));
+                    /* the largest size that still is one pass, by lines a workgroup */
+                    static const int one_st[2][6] = {{0, 16, 24, 24, 64, 64}, {0, 4, 8, 16, 16, 24}};
+                    static const int one_ld[2][6] = {{0, 4}, {0, 4, 4, 4}};
+                    static const int two_st[2][6] = {{0, 24, 32, 32, 128, 128}, {0, 8, 12, 24, 24, 32}};
+                    const int side = w == 1, q = k->nl > 5 ? 0 : k->nl;
+                    const int one = side ? one_ld[prec][q] : one_st[prec][q];
+                    const int two = side ? 8 : two_st[prec][q];
+                    const int want = tout && w < 2 && one && mb >= two;
+                    if (one && mb > one && mb < two) continue; /* either will do */
                     ctx c;
                     fk_plan *P = begin(&c, prec);
                     c.lean = w == 4;
